@@ -319,9 +319,10 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   p.words = a->words;
   p.R = a->R > 0 ? a->R : 1;
   p.C = a->C > 0 ? a->C : 1;
-  p.q_frame0 = a->q_frame0;
-  p.q_tok0 = a->q_tok0;
-  p.k_tok0 = a->k_tok0;
+  p.qo = (uint32_t)(a->q_tok0 % p.R);
+  p.ko = (uint32_t)(a->k_tok0 % p.C);
+  p.qf0 = (int)(a->q_tok0 / p.R - a->q_frame0);
+  p.kf0 = (int)(a->k_tok0 / p.C);
   p.total_work = (int)work;
   p.n_vwork = (int)vwork;
   p.n_twork = (int)twork;
@@ -356,6 +357,10 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   // and the rows past the end) and is planned "generic".
   const bool tail_cross = stream_tail_crosses_frame(a->n_q, a->n_k, a->k_tok0, p.C);
   const bool stream_src = src32 && str24 && !tail_cross;
+  // A plan holds generic blocks only where a tile touches more than two query
+  // frames or a key block more than two parts.
+  const bool generic = a->n_q > 0 && (p.R < a->block_q - 1 || p.C < kBN || tail_cross);
+  p.rel_lds = generic && p.words <= kRelWords;
   p.use_stream = (!fp32 && (a->D == 128 || a->D == 96 || a->D == 64) && a->block_q == kPPBM && !force_pp &&
                   stream_src && (a->n_q == 0 || (p.R >= 255 && p.C >= 64))) ? 1 : 0;
   // D = 192 and 256: the wide single-stream loop on the 4-wave kernel's

@@ -29,13 +29,14 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 template <int D>
-__global__ __launch_bounds__(kThreads, 1) void attn_fwd_f32_kernel(AttnParams p) {
+__global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void attn_fwd_f32_kernel(AttnParams p) {
   constexpr int PITCH = D + 4;   // floats per LDS row
   constexpr int NG = D / 8;      // float4 pairs of S's contraction
   constexpr int NT = D / 32;     // 32-wide d tiles of O
   constexpr int C4 = D / 4;      // float4 per K/V row
   __shared__ __attribute__((aligned(16))) float ks[kBN * PITCH];
   __shared__ __attribute__((aligned(16))) float vs[kBN * PITCH];
+  __shared__ uint32_t relw[kBM * kRelPitch];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -102,6 +103,8 @@ __global__ __launch_bounds__(kThreads, 1) void attn_fwd_f32_kernel(AttnParams p)
   const float cs = p.scale_log2;
   const int my_tile_row = 32 * wave + i32;
 
+  // published by the first block's barrier
+  if (p.rel_lds && !it.text) load_rel_rows<kBM>(p, relw, r0, nrows, tid, kThreads);
   for (int e = e0; e < e1; ++e) {
     const uint2 ent = p.entries[e];
     const uint32_t cx = ent.x, cy = ent.y;
@@ -137,11 +140,11 @@ __global__ __launch_bounds__(kThreads, 1) void attn_fwd_f32_kernel(AttnParams p)
     }
 
     if ((cy & 3u) != kKindNone) {
-      const uint32_t keep = block_keep_bits(p, cx, cy, my_tile_row, my_row, nrows, h);
+      const uint32_t keep = block_keep_bits(p, cx, cy, my_tile_row, my_row, nrows, h, relw);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s0[r] = ((keep >> r) & 1u) ? s0[r] : -INFINITY;
-        s1[r] = ((keep >> (r + 16)) & 1u) ? s1[r] : -INFINITY;
+        s0[r] = keep_or_ninf(s0[r], keep, r);
+        s1[r] = keep_or_ninf(s1[r], keep, r + 16);
       }
     }
 

@@ -61,8 +61,14 @@ struct AttnParams {
   const uint2* entries;
   int n_tiles, n_vt, n_tt;
   const uint32_t* rel;
-  int words, R, C, q_frame0;
-  int64_t q_tok0, k_tok0;
+  int words, R, C;
+  // Frames of the row sources, reduced to 32 bits: query row r is token
+  // qo + r of relation row qf0 on (qo < R), key row c token ko + c of key
+  // frame kf0 on (ko < C).  rel_lds: the plan may hold generic blocks and a
+  // tile's relation rows fit LDS (load_rel_rows).
+  uint32_t qo, ko;
+  int qf0, kf0;
+  int rel_lds;
   int total_work;
   // Work items: n_vwork video tiles (n_vt per head) and n_twork text items
   // (n_tt tiles per head, each split into text_chunks key ranges).  Unsplit
@@ -440,43 +446,89 @@ __device__ __forceinline__ void item_entries(const AttnParams& p, const WorkItem
   }
 }
 
+// Relation rows of a tile's query rows in LDS, for the masks of generic blocks:
+// row r of the tile at relw[r * pitch .. + words).  Kept there (up to
+// kRelWords words per row, 256 key frames) so that a generic block costs one
+// LDS read per key frame it touches instead of a dependent global read, which
+// would also wait for the K/V copies in flight.
+constexpr int kRelWords = 8;                      // key frames / 32 that fit
+constexpr int kRelPitch = kRelWords + 1;          // odd, so 32 rows hit distinct banks
+template <int BM>
+__device__ __forceinline__ void load_rel_rows(const AttnParams& p, uint32_t* relw, int64_t r0, int nrows, int tid,
+                                              int threads) {
+  for (int i = tid; i < BM * p.words; i += threads) {
+    const int r = i / p.words, w = i - r * p.words;
+    const int64_t row = r0 + r < nrows ? r0 + r : (int64_t)nrows - 1;
+    relw[r * kRelPitch + w] = p.rel[(int64_t)(p.qf0 + (int)((p.qo + (uint32_t)row) / (uint32_t)p.R)) * p.words + w];
+  }
+}
+
 // Mask of one key block for this lane's query row (row `tile_row` of its
 // tile, `my_row` of its source), for a block of kind two-part or generic:
 // bit r covers register r%16 of the S^T accumulator of key half r/16, which
 // holds key 8q + j + 4h of the block with q = r/4, j = r%4 (h = lane / 32).
+// key_prefix: the bits of the block's first c keys (0 <= c <= 64).
+__device__ __forceinline__ uint32_t key_prefix(int c, int h) {
+  const int in8 = (c & 7) - 4 * h;
+  const int n = 4 * (c >> 3) + (in8 < 0 ? 0 : (in8 > 4 ? 4 : in8));
+  return n >= 32 ? 0xFFFFFFFFu : ((1u << n) - 1u);
+}
+
 __device__ __forceinline__ uint32_t block_keep_bits(const AttnParams& p, uint32_t cx, uint32_t cy, int tile_row,
-                                                    int64_t my_row, int nrows, int h) {
+                                                    int64_t my_row, int nrows, int h, const uint32_t* relw) {
   if ((cy & 3u) == kKindTwoPart) {
     const int bits = (cy >> 2) & 0xF;
-    const int kb = (int)((cy >> 8) & 0xFF) - 4 * h;
+    const int kb = (int)((cy >> 8) & 0xFF);
     const int qs = (cy >> 16) & 0xFF;
     const bool rb = tile_row >= qs;
     const uint32_t lo_ok = (bits >> (rb ? 2 : 0)) & 1;
     const uint32_t hi_ok = (bits >> (rb ? 3 : 1)) & 1;
-    int n_lo = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int c = kb - 8 * q;
-      n_lo += c < 0 ? 0 : (c > 4 ? 4 : c);
-    }
-    const uint32_t lo_mask = n_lo >= 32 ? 0xFFFFFFFFu : ((1u << n_lo) - 1u);
+    const uint32_t lo_mask = key_prefix(kb > kBN ? kBN : kb, h);
     return (lo_ok ? lo_mask : 0u) | (hi_ok ? ~lo_mask : 0u);
   }
+  // Generic: the block's keys run through consecutive key frames, each a
+  // contiguous range [a, b) of the block; every lane looks its row's bit of
+  // the frame up once per range.  Issue bound: one 32-bit division per block
+  // and a few instructions per frame.  Deciding each key by itself (a 64-bit
+  // division and a dependent read per key) cost such a block several times
+  // its MFMAs: 24 frames of 130 tokens, 12 heads, D = 128, 37 text tokens
+  // took 268 us per call, 70 us with the ranges.
   const bool extra = (cx >> 31) != 0;
-  const int64_t k0 = (int64_t)(cx & 0x7fffffffu) * kBN;
-  const int64_t nsrc = extra ? p.n_x : p.n_k;
-  const int64_t qtok = p.q_tok0 + (my_row < nrows ? my_row : (int64_t)nrows - 1);
-  const int qf_row = (int)(qtok / p.R) - p.q_frame0;
-  const uint32_t* relrow = p.rel + (int64_t)qf_row * p.words;
-  uint32_t keep = 0;
-  for (int r = 0; r < 32; ++r) {
-    const int64_t key = k0 + 8 * (r >> 2) + 4 * h + (r & 3);
-    if (key < nsrc) {
-      const int64_t kf = (p.k_tok0 + key) / p.C;
-      if ((kf >> 5) < p.words && ((relrow[kf >> 5] >> (kf & 31)) & 1u)) keep |= 1u << r;
+  const uint32_t k0 = (cx & 0x7fffffffu) * kBN;
+  const uint32_t nsrc = (uint32_t)(extra ? p.n_x : p.n_k);
+  const uint32_t limit = nsrc - k0 < (uint32_t)kBN ? nsrc - k0 : (uint32_t)kBN;   // valid keys of the block
+  const uint32_t x0 = p.ko + k0, C = (uint32_t)p.C;
+  const uint32_t f0 = x0 / C;
+  uint32_t kf = (uint32_t)p.kf0 + f0;
+  uint32_t end = C - (x0 - f0 * C);                 // first key past frame kf
+  uint32_t keep = 0, below = 0;
+  for (;;) {
+    const uint32_t e = end < limit ? end : limit;
+    const uint32_t upto = key_prefix((int)e, h);
+    if ((kf >> 5) < (uint32_t)p.words) {
+      uint32_t word;
+      if (p.rel_lds) {
+        word = relw[tile_row * kRelPitch + (kf >> 5)];
+      } else {
+        const uint32_t row = (uint32_t)(my_row < nrows ? my_row : (int64_t)nrows - 1);
+        word = p.rel[(int64_t)(p.qf0 + (int)((p.qo + row) / (uint32_t)p.R)) * p.words + (kf >> 5)];
+      }
+      if ((word >> (kf & 31)) & 1u) keep |= upto & ~below;
     }
+    below = upto;
+    if (e >= limit) break;
+    end += C;
+    ++kf;
   }
   return keep;
+}
+
+// s of the keys a lane keeps, -inf of the others (bit r of `keep`: key
+// register r of s0, bit 16 + r of s1): a sign-extended bit and a bitwise
+// select per score.
+__device__ __forceinline__ float keep_or_ninf(float s, uint32_t keep, int r) {
+  const uint32_t m = (uint32_t)((int32_t)(keep << (31 - r)) >> 31);
+  return __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, s) & m) | (~m & 0xff800000u));
 }
 
 template <int D, typename E>
@@ -500,6 +552,7 @@ __global__ __launch_bounds__(kThreads, D >= 192 ? 1 : 2) void attn_fwd_kernel(At
   static_assert(NI % kWaves == 0, "tile must split evenly over waves");
 
   __shared__ __attribute__((aligned(1024))) char smem_raw[2 * STAGE];
+  __shared__ uint32_t relw[kBM * kRelPitch];
   lds_char* smem = (lds_char*)smem_raw;
 
   const int lane = threadIdx.x & 63;
@@ -702,11 +755,11 @@ __global__ __launch_bounds__(kThreads, D >= 192 ? 1 : 2) void attn_fwd_kernel(At
     // Masks (bit r of `keep`: register r%16 of key half r/16).
     const uint32_t kind = cy & 3u;
     if (kind != kKindNone) {
-      const uint32_t keep = block_keep_bits(p, cx, cy, my_tile_row, my_row, nrows, h);
+      const uint32_t keep = block_keep_bits(p, cx, cy, my_tile_row, my_row, nrows, h, relw);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s0[r] = ((keep >> r) & 1u) ? s0[r] : -INFINITY;
-        s1[r] = ((keep >> (r + 16)) & 1u) ? s1[r] : -INFINITY;
+        s0[r] = keep_or_ninf(s0[r], keep, r);
+        s1[r] = keep_or_ninf(s1[r], keep, r + 16);
       }
     }
 
@@ -811,6 +864,8 @@ __global__ __launch_bounds__(kThreads, D >= 192 ? 1 : 2) void attn_fwd_kernel(At
     }
   };
 
+  // before the first copies; the barrier of the first block publishes them
+  if (p.rel_lds && !text) load_rel_rows<kBM>(p, relw, r0, nrows, threadIdx.x, kThreads);
   if (e0 < e1) {
     nx = __builtin_amdgcn_readlane(ec_x, 0);
     ny = __builtin_amdgcn_readlane(ec_y, 0);
@@ -936,6 +991,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void attn_fwd_pp_kernel(AttnParams p
   static_assert(NI % 4 == 0, "tile must split evenly over the DMA waves");
 
   __shared__ __attribute__((aligned(1024))) char smem_raw[2 * kPPStages * TILE];
+  __shared__ uint32_t relw[kPPBM * kRelPitch];
   lds_char* smem = (lds_char*)smem_raw;
 
   const int lane = threadIdx.x & 63;
@@ -1187,11 +1243,11 @@ __global__ __launch_bounds__(kPPThreads, 1) void attn_fwd_pp_kernel(AttnParams p
     // Masks (bit r of `keep`: register r%16 of key half r/16).
     const uint32_t kind = cy & 3u;
     if (kind != kKindNone) {
-      const uint32_t keep = block_keep_bits(p, cx, cy, my_tile_row, my_row, nrows, h);
+      const uint32_t keep = block_keep_bits(p, cx, cy, my_tile_row, my_row, nrows, h, relw);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s0[r] = ((keep >> r) & 1u) ? s0[r] : -INFINITY;
-        s1[r] = ((keep >> (r + 16)) & 1u) ? s1[r] : -INFINITY;
+        s0[r] = keep_or_ninf(s0[r], keep, r);
+        s1[r] = keep_or_ninf(s1[r], keep, r + 16);
       }
     }
 
@@ -1319,6 +1375,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void attn_fwd_pp_kernel(AttnParams p
       *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(
           smem + (2 * kPPStages - 1) * TILE + (z * kPPThreads + (int)threadIdx.x) * 16) = u32x4{0, 0, 0, 0};
   }
+  if (p.rel_lds && !text) load_rel_rows<kPPBM>(p, relw, r0, nrows, threadIdx.x, kPPThreads);
   __syncthreads();
 
   // Block b of the plan, or a stand-in past the end: row 0 of a key source,

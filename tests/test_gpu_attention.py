@@ -141,6 +141,33 @@ def test_random_geometries(seed, gpu, monkeypatch):
     torch.testing.assert_close(lse.cpu(), rl, atol=2e-2, rtol=0, msg=what)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("cfg", [
+    # T, P, W, kfi, off, H, Hkv, D, n_txt: frames shorter than a key block or a tile
+    (300, 3, 2, 8, 5, 2, 1, 64, 0),      # 10 relation words: rows looked up in global memory
+    (256, 1, 1, 4, 3, 1, 1, 128, 5),     # 8 words: the most that LDS holds; one token per frame
+    (257, 2, 1, 4, 0, 1, 1, 128, 0),     # 9 words
+    (12, 63, 1, 4, 2, 2, 2, 128, 0),     # three frames in some blocks
+    (12, 64, 1, 4, 1, 2, 2, 64, 9),      # frames on the block grid
+    (7, 65, 2, 3, 1, 2, 2, 96, 0),       # block edges one token into a frame
+    (3, 254, 1, None, 0, 2, 2, 128, 3),  # the longest frames with generic blocks in 256-row tiles
+], ids=str)
+def test_generic_masks_short_frames(cfg, dt, gpu):
+    T, P, W, kfi, off, H, Hkv, D, n_txt = cfg
+    N = T * P
+    q, k, v, qt, kt, vt = _draw([(1, N, H, D), (1, N, Hkv, D), (1, N, Hkv, D), (1, n_txt, H, D),
+                                 (1, n_txt, Hkv, D), (1, n_txt, Hkv, D)], seed=P, dtype=dt)
+    m = _meta(T, P, W, 1, kfi, off)
+    args = dict(k_text=kt.to(gpu), v_text=vt.to(gpu)) if n_txt else {}
+    out, lse = lv.lvsa_attention(q.to(gpu), k.to(gpu), v.to(gpu), m, return_lse=True, **args)
+    rows = [set(r) for r in om.build_frame_mask(T, P, W, 1, kfi, offset=off).rows]
+    ro, rl = oa.per_frame_sdpa(q.float(), k.float(), v.float(), rows, P, k_extra=kt.float() if n_txt else None,
+                               v_extra=vt.float() if n_txt else None)
+    tol = dict(max_abs=FP32_MAX_ABS, mean_abs=FP32_MEAN_ABS) if dt == torch.float32 else {}
+    _close(out, ro, str(cfg), **tol)
+    torch.testing.assert_close(lse.cpu(), rl, atol=2e-5 if dt == torch.float32 else 2e-2, rtol=1e-6)
+
+
 def test_repeat_call_is_bitwise_identical(gpu):
     T, P, H, D = 12, 300, 4, 128
     m = _meta(T, P, 2, 1, 4, 1)
