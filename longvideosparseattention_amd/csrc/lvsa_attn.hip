@@ -20,13 +20,16 @@ namespace {
 constexpr int kTextChunkBlocks = 128;
 constexpr int kMaxTextChunks = 64;
 
-// Text chunks per text tile for the arguments (1 = no split).
-int text_chunks_of(const lvsa_attn_args* a) {
-  if (a->n_tq == 0 || a->dtype == LVSA_FP32) return 1;   // the fp32 kernel runs text tiles whole
+// Text chunks per text tile (1 = no split): of a 16-bit call with a workspace,
+// and of an fp32 call with room for its split operands.
+int text_chunks_any(const lvsa_attn_args* a) {
+  if (a->n_tq == 0) return 1;
   const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
   const int64_t c = ceil_div(blocks, kTextChunkBlocks);
   return (int)(c < 1 ? 1 : (c > kMaxTextChunks ? kMaxTextChunks : c));
 }
+
+int text_chunks_of(const lvsa_attn_args* a) { return a->dtype == LVSA_FP32 ? 1 : text_chunks_any(a); }
 
 int64_t text_ws_bytes(const lvsa_attn_args* a, int chunks) {
   if (a->n_tq == 0 || chunks <= 1) return 0;
@@ -50,6 +53,25 @@ int64_t queue_offset(const lvsa_attn_args* a, int chunks, int vsplit) {
 }
 int64_t ws_bytes(const lvsa_attn_args* a, int vsplit) {
   return queue_offset(a, text_chunks_of(a), vsplit) + kQueueBytes;
+}
+
+// fp32: the text-split partials, the counters (unused) and, from
+// f32_split_offset, K and V of every key block as fp16 pairs
+// (lvsa_attn_f32.hip).  0 blocks where that scratch would pass kMaxSplitBytes
+// (as much as K and V themselves: 2.3 GB for 121 frames of 1560 tokens, 12
+// heads, D = 128) or the grid's 2^31: such a call runs the fp32 kernel.
+constexpr int64_t kMaxSplitBytes = 16LL << 30;
+int64_t f32_split_slots(const lvsa_attn_args* a) {
+  if (a->dtype != LVSA_FP32) return 0;
+  const int64_t slots = 2LL * a->B * a->Hkv * (ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN));
+  return slots >= (int64_t)INT32_MAX || f32_split_bytes(slots, a->D) > kMaxSplitBytes ? 0 : slots;
+}
+int64_t f32_split_offset(const lvsa_attn_args* a) {
+  return align256(queue_offset(a, text_chunks_any(a), 0) + kQueueBytes);
+}
+int64_t f32_ws_bytes(const lvsa_attn_args* a) {
+  const int64_t slots = f32_split_slots(a);
+  return slots ? f32_split_offset(a) + f32_split_bytes(slots, a->D) : ws_bytes(a, 0);
 }
 
 // Zero the work-queue counters (a kernel, not a memset, so the call can be
@@ -134,7 +156,7 @@ __global__ __launch_bounds__(256) void attn_text_merge_kernel(const float* ws, i
     acc.w += w * o.w;
   }
   const float inv = L > 0.f ? 1.0f / L : 0.f;
-  E* op = reinterpret_cast<E*>(ot + 2 * (batch * s0 + row * s1 + head * s2)) + 4 * dq;
+  E* op = reinterpret_cast<E*>(ot + sizeof(E) * (batch * s0 + row * s1 + head * s2)) + 4 * dq;
   op[0] = (E)(acc.x * inv);
   op[1] = (E)(acc.y * inv);
   op[2] = (E)(acc.z * inv);
@@ -268,7 +290,11 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
                  "lvsa_attn_fwd: query rows map to relation rows [%lld, %lld], the relation has %d rows",
                  (long long)first, (long long)last, a->rel_rows);
   }
-  const int chunks = a->workspace ? text_chunks_of(a) : 1;
+  // fp32 with room for the split operands: K and V as fp16 pairs, text tiles
+  // in chunks; without it (a smaller workspace, or none) the fp32 MFMAs and
+  // whole text tiles.
+  const int64_t split_slots = fp32 && a->workspace && a->workspace_bytes >= f32_ws_bytes(a) ? f32_split_slots(a) : 0;
+  const int chunks = !a->workspace ? 1 : split_slots ? text_chunks_any(a) : text_chunks_of(a);
   const int64_t ws_need = a->workspace ? ws_bytes(a, 0) : 0;   // without the video split
   LVSA_REQUIRE(a->workspace_bytes >= ws_need, LVSA_ERR_CAPACITY,
                "lvsa_attn_fwd: workspace of %lld bytes < %lld needed (lvsa_attn_workspace_query)",
@@ -329,6 +355,13 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   p.text_chunks = chunks;
   p.text_first = chunks == 1 ? 1 : 0;
   p.ws = chunks > 1 ? (float*)a->workspace : nullptr;
+  p.split = nullptr;
+  p.split_exp = nullptr;
+  p.split_slots = (int)split_slots;
+  if (split_slots) {
+    p.split = (char*)a->workspace + f32_split_offset(a);
+    p.split_exp = (int32_t*)(p.split + split_slots * 4LL * kBN * a->D);
+  }
   p.vsplit = 0;
   p.vws = nullptr;
   // The single-stream kernel (D = 64, 96 and 128 here; 192 and 256 below)
@@ -417,7 +450,7 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   const int bq = a->block_q;
   const bool bf16 = a->dtype == LVSA_BF16;
   int rc;
-  if (fp32) rc = launch_f32(p, a->D, stream);
+  if (fp32) rc = launch_f32(p, a->D, cus, stream);
   else if (a->D == 256) rc = launch_d256(p, bq, bf16, stream);
   else if (a->D == 128) rc = launch_d128(p, bq, bf16, stream);
   else if (a->D == 96) rc = launch_d96(p, bq, bf16, stream);
@@ -435,7 +468,11 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   if (chunks == 1) return rc;
   const int64_t threads = (int64_t)a->B * a->H * a->n_tq * (a->D / 4);
   const dim3 grid((unsigned)ceil_div(threads, 256));
-  if (bf16) {
+  if (fp32) {
+    hipLaunchKernelGGL(attn_text_merge_kernel<float>, grid, dim3(256), 0, stream, (const float*)a->workspace,
+                       chunks, a->B, a->H, a->n_tq, a->D, (char*)a->ot, a->ot_str[0], a->ot_str[1], a->ot_str[2],
+                       a->lse_t);
+  } else if (bf16) {
     hipLaunchKernelGGL(attn_text_merge_kernel<__bf16>, grid, dim3(256), 0, stream, (const float*)a->workspace,
                        chunks, a->B, a->H, a->n_tq, a->D, (char*)a->ot, a->ot_str[0], a->ot_str[1], a->ot_str[2],
                        a->lse_t);
@@ -458,6 +495,6 @@ extern "C" int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes
                "lvsa_attn_workspace_query: bad sizes");
   LVSA_REQUIRE(a->D == 64 || a->D == 96 || a->D == 128 || a->D == 192 || a->D == 256, LVSA_ERR_UNSUPPORTED,
                "lvsa_attn_workspace_query: head_dim %d not supported", a->D);
-  *bytes = ws_bytes(a, vsplit_pref(a));
+  *bytes = a->dtype == LVSA_FP32 ? f32_ws_bytes(a) : ws_bytes(a, vsplit_pref(a));
   return LVSA_OK;
 }

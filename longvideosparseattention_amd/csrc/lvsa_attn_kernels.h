@@ -98,6 +98,11 @@ struct AttnParams {
   // at `queues`; null: one work-group per item, mapped by map_work.
   uint32_t* queues;
   int grid;
+  // fp32 inputs: K and V split into fp16 pairs (lvsa_attn_f32.hip), split_slots
+  // blocks at `split` with their exponents at split_exp; null: the fp32 kernel
+  char* split;
+  int32_t* split_exp;
+  int split_slots;
 };
 
 // Bytes of the work-queue counters at the end of the attention workspace.
@@ -119,8 +124,10 @@ int launch_d96(const AttnParams& prm, int block_q, bool bf16, hipStream_t stream
 int launch_d128(const AttnParams& prm, int block_q, bool bf16, hipStream_t stream);
 int launch_d192(const AttnParams& prm, int block_q, bool bf16, hipStream_t stream);
 int launch_d256(const AttnParams& prm, int block_q, bool bf16, hipStream_t stream);
-// fp32 inputs (lvsa_attn_f32.hip): 128-row tiles, every head size.
-int launch_f32(const AttnParams& prm, int D, hipStream_t stream);
+// fp32 inputs (lvsa_attn_f32.hip): 128-row tiles, every head size, `cus`
+// compute units; scratch of `slots` split key blocks (their exponents last).
+int launch_f32(const AttnParams& prm, int D, int cus, hipStream_t stream);
+int64_t f32_split_bytes(int64_t slots, int D);
 
 namespace {
 

@@ -7,12 +7,14 @@ one CPU generator, seed 0, fp32 randn drawn in order q, k, v, then text q,
 k, v, shapes [B, N, H, D], rounded to the compute dtype.
 """
 
+import ctypes as C
 import math
 
 import pytest
 import torch
 
 import longvideosparseattention_amd as lv
+from longvideosparseattention_amd import _capi as capi
 from longvideosparseattention_amd import hip_ops
 from oracle import attention as oa
 from oracle import lvsa_mask as om
@@ -408,6 +410,108 @@ def test_fp32_small_configs(cfg, gpu):
         o, lse = lv.lvsa_attention(g[0], g[1], g[2], m, return_lse=True)
     _close(o, ro, f"fp32 D={D}", max_abs=FP32_MAX_ABS, mean_abs=FP32_MEAN_ABS)
     torch.testing.assert_close(lse.cpu(), rl, atol=2e-5, rtol=1e-6)
+
+
+@pytest.mark.parametrize("D", [64, 96, 128, 192, 256])
+@pytest.mark.parametrize("P,H,n_txt", [
+    (70, 2, 9),       # few tiles: two key groups per work-group (D <= 128), odd key tails
+    (256, 12, 0),
+    (300, 60, 130),   # more tiles than compute units; text tiles in chunks at T = 40
+])
+def test_fp32_split_is_no_further_from_float64(P, H, n_txt, D, gpu):
+    """fp32 inputs on the split fp16 MFMAs: error against float64 attention at
+    most that of the fp32-MFMA kernel (``scratch=False``), video rows, text
+    rows and LSE."""
+    if H == 60 and D != 128:
+        H = 30
+    T = 40 if (P == 300 and D == 64) else 8
+    m = _meta(T, P, 1, 1, 4, 2)
+    N = T * P
+    q, k, v, qt, kt, vt = (x.to(gpu) for x in _draw(
+        [(1, N, H, D), (1, N, H // 2, D), (1, N, H // 2, D), (1, n_txt, H, D), (1, n_txt, H // 2, D),
+         (1, n_txt, H // 2, D)], seed=D + P, dtype=torch.float32))
+    plan = m.full_plan(gpu, N, N, n_txt, n_txt, D, torch.float32)
+    kw = dict(kx=kt, vx=vt, qt=qt) if n_txt else {}
+    split = hip_ops.attn_fwd(q, k, v, plan, return_lse=True, **kw)
+    plain = hip_ops.attn_fwd(q, k, v, plan, return_lse=True, scratch=False, **kw)
+    rows = [set(r) for r in om.build_frame_mask(T, P, 1, 1, 4, offset=2).rows]
+    heads = [0, H - 1]
+    for hd in heads:
+        kk, vv = k[0, :, hd // 2].double(), v[0, :, hd // 2].double()
+        if n_txt:
+            kk, vv = torch.cat([kk, kt[0, :, hd // 2].double()]), torch.cat([vv, vt[0, :, hd // 2].double()])
+        frame = torch.arange(N, device=gpu) // P
+        ok = torch.zeros(T, T, dtype=torch.bool)
+        for f, r in enumerate(rows):
+            ok[f, sorted(r)] = True
+        seen = ok.to(gpu)[frame][:, frame]
+        seen = torch.cat([seen, torch.ones(N, n_txt, dtype=torch.bool, device=gpu)], 1)
+        s = (q[0, :, hd].double() @ kk.T / D ** 0.5).masked_fill(~seen, float("-inf"))
+        want = [torch.softmax(s, -1) @ vv, torch.logsumexp(s, -1)]
+        if n_txt:
+            st = qt[0, :, hd].double() @ kk.T / D ** 0.5
+            want += [torch.softmax(st, -1) @ vv, torch.logsumexp(st, -1)]
+
+        def errors(res):
+            o, ot, lse, lse_t = res
+            got = [o[0, :, hd], lse[0, hd]] + ([ot[0, :, hd], lse_t[0, hd]] if n_txt else [])
+            return [((g.double() - w).norm() / w.norm()).item() for g, w in zip(got, want)]
+
+        for a, b in zip(errors(split), errors(plain)):
+            # 1e-7: one rounding of the fp32 result (2^-24), which both share
+            assert a <= max(b, 1e-7), (errors(split), errors(plain))
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("kind", ["k_inf", "k_nan", "v_inf", "q_ninf", "huge", "v_far", "tiny_v", "zeros"])
+def test_fp32_split_range(kind, D, gpu):
+    """Inputs outside the split's range give what the fp32-MFMA kernel gives:
+    non-finite values, products that overflow, V blocks of very different
+    size; and small or zero blocks keep fp32's relative accuracy."""
+    T, P, H = 6, 130, 2
+    m = _meta(T, P, 1, 1, 3, 1)
+    N = T * P
+    q, k, v = _draw([(1, N, H, D)] * 3, seed=D, dtype=torch.float32)
+    if kind == "k_inf":
+        k[0, 300, 0, 5] = float("-inf")
+    elif kind == "k_nan":
+        k[0, 10, 1, 3] = float("nan")
+    elif kind == "v_inf":
+        v[0, 500, 0, 7] = float("inf")
+    elif kind == "q_ninf":
+        q[0, 200, 0, 1] = float("-inf")
+    elif kind == "huge":
+        q[0, 200] *= 1e19
+        k[0, 150] *= 1e20
+    elif kind == "v_far":
+        v[0, :P] *= 1e-9
+    elif kind == "tiny_v":
+        v *= 1e-25
+    else:
+        k[0, :128] = 0
+        v[0, 64:256] = 0
+    plan = m.full_plan(gpu, N, N, 0, 0, D, torch.float32)
+    q, k, v = q.to(gpu), k.to(gpu), v.to(gpu)
+    a, _, la, _ = hip_ops.attn_fwd(q, k, v, plan, return_lse=True)
+    b, _, lb, _ = hip_ops.attn_fwd(q, k, v, plan, return_lse=True, scratch=False)
+    tol = 2e-5 * b[torch.isfinite(b)].abs().max().item()
+    torch.testing.assert_close(a, b, atol=tol, rtol=2e-5, equal_nan=True)
+    torch.testing.assert_close(la, lb, atol=2e-5, rtol=1e-6, equal_nan=True)
+
+
+def test_fp32_smaller_workspace_runs_the_fp32_kernel(gpu):
+    """A workspace too small for the split operands (1 KiB was enough for any
+    fp32 call) still runs, on the fp32 MFMAs: bit for bit the call without."""
+    T, P, H, D = 5, 100, 2, 64
+    m = _meta(T, P, 1, 1, 3, 1)
+    q, k, v = (x.to(gpu) for x in _draw([(1, T * P, H, D)] * 3, dtype=torch.float32))
+    plan = m.full_plan(gpu, T * P, T * P, 0, 0, D, torch.float32)
+    want = hip_ops.attn_fwd(q, k, v, plan, scratch=False)[0]
+    call = hip_ops.attn_args(q, k, v, plan)
+    ws = torch.empty(1024, dtype=torch.uint8, device=gpu)
+    call.args.workspace, call.args.workspace_bytes = ws.data_ptr(), 1024
+    capi.check("lvsa_attn_fwd", capi.lib().lvsa_attn_fwd(C.byref(call.args), hip_ops._stream(call.out.device)))
+    assert torch.equal(call.out, want)
 
 
 def test_fp32_wrapper_and_prefill(gpu):
