@@ -375,7 +375,7 @@ void attn_fwd_split_kernel(AttnParams p) {
   constexpr int NFR = D / 8;                       // fragments of a block's hi (lo) numbers
   constexpr int TILE = 2 * NFR * 1024;             // bytes of one K or V block
   constexpr int NIW = TILE / 1024 / kWaves;        // 1 KiB copies per wave and block
-  constexpr int LA = 1;                            // operand pairs read ahead of their MFMAs
+  constexpr int LA = 3;                            // operands read this many MFMAs ahead
   constexpr int LDS = KG * 2 * TILE > kF32Lds<D> ? KG * 2 * TILE : kF32Lds<D>;
   static_assert(KG == 1 || (KG - 1) * kWaves * (NT * 16 + 3) * 256 <= LDS, "the merge must fit the buffers");
   __shared__ __attribute__((aligned(1024))) char smem_raw[LDS];
@@ -468,6 +468,11 @@ void attn_fwd_split_kernel(AttnParams p) {
   constexpr float kMaxLag = 3.f;
 
   const int rounds = (t.e1 - t.e0 + KG - 1) / KG;
+  // Two groups run half a round apart (one barrier), so that on each SIMD one
+  // wave's P V meets the other's scores and softmax.
+  if constexpr (KG == 2) {
+    if (kg == 1) __syncthreads();
+  }
   for (int r = 0; r < rounds; ++r) {
     const bool have = e < t.e1;
     wait_vm0();
@@ -478,30 +483,43 @@ void attn_fwd_split_kernel(AttnParams p) {
       copy(cur + 1, vs);
       const uint2 now = ent;
       const int kexp = exps[cur], ve = exps[cur + 1];
-      // S^T of both key halves: the small products (hi lo, lo hi) in an
-      // accumulator of their own, so only hi hi rounds at the size of S
-      floatx16 s[2];
+      // S^T of both key halves: the small products (hi lo, lo hi) first, so
+      // only the D / 16 hi hi MFMAs round at the size of S
+      floatx16 s[2] = {floatx16{0}, floatx16{0}};
+      if constexpr (true) __builtin_amdgcn_s_setprio(1);
+      {
+        halfx8 a[4 * ND];
+        // operands 0 .. 4 ND - 1: (lo, hi) of both halves per k-step, then hi again
+        auto operand = [&](int i) __attribute__((always_inline)) {
+          const int c = i >> 2, half = i & 1;
+          return frag(ks, ((i & 2) ? 0 : NFR) + half * ND + c);
+        };
+        constexpr int NO = 4 * ND;
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        floatx16 big = floatx16{0}, small = floatx16{0};
-        halfx8 kh[ND], kl[ND];
-#pragma unroll
-        for (int c = -LA; c < ND; ++c) {
-          if (c + LA < ND) {
-            kh[c + LA] = frag(ks, half * ND + c + LA);
-            kl[c + LA] = frag(ks, NFR + half * ND + c + LA);
-            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // two LDS reads
+        for (int i = -LA; i < NO; ++i) {
+          if (i + LA < NO) {
+            a[i + LA] = operand(i + LA);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
           }
-          if (c >= 0) {
-            big = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[c], qh[c], big, 0, 0, 0);
-            small = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[c], qh[c], small, 0, 0, 0);
-            small = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[c], ql[c], small, 0, 0, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);   // three MFMAs
+          if (i >= 0) {
+            s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], (i & 2) ? ql[i >> 2] : qh[i >> 2], s[i & 1], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
           }
         }
+        halfx8 b[2 * ND];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[half][i] = big[i] + small[i];
+        for (int i = -LA; i < 2 * ND; ++i) {
+          if (i + LA < 2 * ND) {
+            b[i + LA] = frag(ks, ((i + LA) & 1) * ND + ((i + LA) >> 1));
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+          if (i >= 0) {
+            s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[i], qh[i >> 1], s[i & 1], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          }
+        }
       }
+      if constexpr (true) __builtin_amdgcn_s_setprio(0);
       if ((now.y & 3u) != kKindNone) {
         const uint32_t keep = block_keep_bits(p, now.x, now.y, my_tile_row, my_row, t.nrows, h, relw);
 #pragma unroll
@@ -575,11 +593,12 @@ void attn_fwd_split_kernel(AttnParams p) {
     if (more) copy(slot, ks);
     if (have) {
       halfx8 vh[NFR], vl[NFR];
+      constexpr int LP = 1;     // operand pairs read ahead of their three MFMAs
 #pragma unroll
-      for (int f = -LA; f < NFR; ++f) {
-        if (f + LA < NFR) {
-          vh[f + LA] = frag(vs, f + LA);
-          vl[f + LA] = frag(vs, NFR + f + LA);
+      for (int f = -LP; f < NFR; ++f) {
+        if (f + LP < NFR) {
+          vh[f + LP] = frag(vs, f + LP);
+          vl[f + LP] = frag(vs, NFR + f + LP);
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
         if (f >= 0) {
@@ -591,6 +610,9 @@ void attn_fwd_split_kernel(AttnParams p) {
         }
       }
     }
+  }
+  if constexpr (KG == 2) {
+    if (kg == 0) __syncthreads();
   }
 
   // Merge the groups: m, l and O at their true scale.
