@@ -36,24 +36,29 @@ void clear_error() { g_last_error.clear(); }
 namespace {
 
 constexpr int kMaskThreads = 1024;
-constexpr int kPlanThreads = 128;
+constexpr int kPlanThreads = 256;
 constexpr int kScanThreads = 1024;
 
-// Exclusive scan of one int per thread across the work-group.
+// Exclusive scan of one int per thread across the work-group (whole waves;
+// sh: an int per wave).
 __device__ int block_exclusive_scan(int v, int* sh, int* total) {
-  const int tid = threadIdx.x;
-  sh[tid] = v;
-  __syncthreads();
-  for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-    int add = (tid >= off) ? sh[tid - off] : 0;
-    __syncthreads();
-    sh[tid] += add;
-    __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  int incl = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int add = __shfl_up(incl, off);
+    if (lane >= off) incl += add;
   }
-  const int incl = sh[tid];
-  *total = sh[blockDim.x - 1];
+  if (lane == 63) sh[wave] = incl;
   __syncthreads();
-  return incl - v;
+  int before = 0, all = 0;
+  for (int w = 0; w < waves; ++w) {
+    const int x = sh[w];
+    if (w < wave) before += x;
+    all += x;
+  }
+  *total = all;
+  __syncthreads();
+  return before + incl - v;
 }
 
 // Window bounds of query frame f (lvsa/sparse_attention.py:40-104).
@@ -144,28 +149,20 @@ struct MaskGeom {
   int T, P, first, n_local, n_rows, words;
 };
 
-// One 32-frame word of relation row `f`: bit set for global frames ("full"
-// only) and for non-global window frames holding tokens on this rank (both).
-__device__ inline void relation_word(const MaskGeom& g, int f, int lo, int hi, int w, const uint8_t* gflag,
+// Bits of the frames [lo, hi] in the 32-frame word w.
+__device__ inline uint32_t range_word(int lo, int hi, int w) {
+  const int a = lo - 32 * w > 0 ? lo - 32 * w : 0, b = hi - 32 * w < 31 ? hi - 32 * w : 31;
+  return a > b ? 0u : (0xFFFFFFFFu >> (31 - b)) & (0xFFFFFFFFu << a);
+}
+
+// One 32-frame word of a relation row of window [lo, hi]: bit set for global
+// frames ("full" only) and for non-global window frames holding tokens on this
+// rank (both), which are the frames [first, first + n_local).
+__device__ inline void relation_word(const MaskGeom& g, int lo, int hi, int w, const uint32_t* gword,
                                      uint32_t* full, uint32_t* win) {
-  uint32_t a = 0, b = 0;
-  const int base = 32 * w;
-  for (int bit = 0; bit < 32; ++bit) {
-    const int fr = base + bit;
-    if (fr >= g.T) break;
-    if (gflag[fr]) {
-      a |= 1u << bit;
-    } else if (fr >= lo && fr <= hi) {
-      const int64_t s = (int64_t)fr * g.P > g.gts ? (int64_t)fr * g.P : g.gts;
-      const int64_t e = (int64_t)(fr + 1) * g.P < g.gts + g.local ? (int64_t)(fr + 1) * g.P : g.gts + g.local;
-      if (s < e) {
-        a |= 1u << bit;
-        b |= 1u << bit;
-      }
-    }
-  }
-  *full = a;
-  *win = b;
+  const int a = lo > g.first ? lo : g.first, b = hi < g.first + g.n_local - 1 ? hi : g.first + g.n_local - 1;
+  *win = range_word(a, b, w) & ~gword[w];
+  *full = gword[w] | *win;
 }
 
 __global__ __launch_bounds__(kMaskThreads) void mask_build_kernel(lvsa_mask_params p, MaskGeom g,
@@ -175,8 +172,9 @@ __global__ __launch_bounds__(kMaskThreads) void mask_build_kernel(lvsa_mask_para
   __shared__ int16_t whi[LVSA_MAX_FRAMES];
   __shared__ int rowoff[LVSA_MAX_FRAMES + 2];
   __shared__ uint32_t uni[LVSA_BITMAP_WORDS];
+  __shared__ uint32_t gword[LVSA_BITMAP_WORDS];   // the global flags as words
   __shared__ int uprefix[LVSA_BITMAP_WORDS + 1];
-  __shared__ int scan_sh[kMaskThreads];
+  __shared__ int scan_sh[kMaskThreads / 64];
   __shared__ int s_rowmax;
   __shared__ int s_kfi;
 
@@ -204,6 +202,12 @@ __global__ __launch_bounds__(kMaskThreads) void mask_build_kernel(lvsa_mask_para
     }
   }
   __syncthreads();
+
+  for (int w = tid; w < g.words; w += nt) {
+    uint32_t x = 0;
+    for (int b = 0; b < 32 && 32 * w + b < T; ++b) x |= (uint32_t)gflag[32 * w + b] << b;
+    gword[w] = x;
+  }
 
   // 2. sorted global list via a scan over contiguous per-thread segments.
   const int seg = (T + nt - 1) / nt;
@@ -233,7 +237,7 @@ __global__ __launch_bounds__(kMaskThreads) void mask_build_kernel(lvsa_mask_para
     int nnz = 0;
     for (int w = 0; w < g.words; ++w) {
       uint32_t full, win;
-      relation_word(g, f, wlo[f], whi[f], w, gflag, &full, &win);
+      relation_word(g, wlo[f], whi[f], w, gword, &full, &win);
       out.rel_full[(int64_t)r * g.words + w] = full;
       out.rel_window[(int64_t)r * g.words + w] = win;
       if (r < g.n_rows) {
@@ -292,7 +296,7 @@ __global__ __launch_bounds__(kMaskThreads) void mask_build_kernel(lvsa_mask_para
     int k = rowoff[r];
     for (int w = 0; w < g.words; ++w) {
       uint32_t full, win;
-      relation_word(g, f, wlo[f], whi[f], w, gflag, &full, &win);
+      relation_word(g, wlo[f], whi[f], w, gword, &full, &win);
       const uint32_t uw = uni[w];
       while (full) {
         const int b = __ffs(full) - 1;
@@ -315,9 +319,15 @@ __global__ __launch_bounds__(kMaskThreads) void mask_build_kernel(lvsa_mask_para
 
 // ───────────────────────────── block plan ──────────────────────────────────
 
+// Row r of the query source is token qo + r of relation row qf0 on (qo < R),
+// key row c token ko + c of key frame kf0 on (ko < C): sums below 2^32, so the
+// kernels divide in 32 bits.
 struct PlanCtx {
   lvsa_plan_params p;
   int n_vt, n_tt, nkc, nxc;
+  uint32_t qo, ko;
+  int qf0;
+  int64_t kf0;
 };
 
 __device__ inline uint32_t rel_word(const PlanCtx& c, int row, int w) {
@@ -328,6 +338,26 @@ __device__ inline uint32_t rel_word(const PlanCtx& c, int row, int w) {
 __device__ inline uint32_t rel_bit(const PlanCtx& c, int row, int64_t kf) {
   if (kf < 0) return 0u;
   return (rel_word(c, row, (int)(kf >> 5)) >> (kf & 31)) & 1u;
+}
+
+// Relation rows qf0..qf1 of query tile t.
+__device__ inline void tile_frames(const PlanCtx& c, int t, int64_t* r0, int* qf0, int* qf1) {
+  *r0 = (int64_t)t * c.p.block_q;
+  const int64_t r1 = (*r0 + c.p.block_q) < c.p.n_q ? (*r0 + c.p.block_q) : c.p.n_q;
+  *qf0 = c.qf0 + (int)((c.qo + (uint32_t)*r0) / (uint32_t)c.p.R);
+  *qf1 = c.qf0 + (int)((c.qo + (uint32_t)(r1 - 1)) / (uint32_t)c.p.R);
+}
+
+// Key blocks [jlo, jhi] of the frame source that key frame kf touches; false
+// when it has no row in it.
+__device__ inline bool frame_blocks(const PlanCtx& c, int64_t kf, int* jlo, int* jhi) {
+  int64_t a = (kf - c.kf0) * c.p.C - c.ko, e = a + c.p.C;
+  if (a < 0) a = 0;
+  if (e > c.p.n_k) e = c.p.n_k;
+  if (a >= e) return false;
+  *jlo = (int)((uint32_t)a / (uint32_t)c.p.block_k);
+  *jhi = (int)((uint32_t)(e - 1) / (uint32_t)c.p.block_k);
+  return true;
 }
 
 // Descriptor of a block of a dense source (text or extra rows): full, or a
@@ -345,7 +375,8 @@ __device__ uint32_t frame_desc(const PlanCtx& c, int64_t r0, int qf0, int qf1, i
   const lvsa_plan_params& p = c.p;
   const int64_t k0 = j * p.block_k;
   const int64_t k1 = (k0 + p.block_k) < p.n_k ? (k0 + p.block_k) : p.n_k;
-  const int64_t kfa = (p.k_tok0 + k0) / p.C, kfb = (p.k_tok0 + k1 - 1) / p.C;
+  const int64_t kfa = c.kf0 + (c.ko + (uint32_t)k0) / (uint32_t)p.C;
+  const int64_t kfb = c.kf0 + (c.ko + (uint32_t)(k1 - 1)) / (uint32_t)p.C;
   const bool tail = (k1 - k0) < p.block_k;
   const int nq = qf1 - qf0 + 1;
   const int64_t nk = kfb - kfa + 1 + (tail ? 1 : 0);
@@ -370,63 +401,119 @@ __device__ uint32_t frame_desc(const PlanCtx& c, int64_t r0, int qf0, int qf1, i
   return make_desc(kKindGeneric, 0, 0, 0);
 }
 
+// Entries of tile t, counted by one thread (tiles of few query frames).
+__device__ int tile_count(const PlanCtx& c, int t) {
+  if (t >= c.n_vt) return c.nkc + c.nxc;
+  int64_t r0;
+  int qf0, qf1;
+  tile_frames(c, t, &r0, &qf0, &qf1);
+  int count = 0, jnext = 0;
+  for (int w = 0; w < c.p.words; ++w) {
+    uint32_t u = 0;
+    for (int q = qf0; q <= qf1; ++q) u |= rel_word(c, q, w);
+    while (u) {
+      const int b = __ffs(u) - 1;
+      u &= u - 1;
+      int jlo, jhi;
+      if (!frame_blocks(c, 32 * (int64_t)w + b, &jlo, &jhi)) continue;
+      if (jlo < jnext) jlo = jnext;
+      if (jhi >= jlo) {
+        count += jhi - jlo + 1;
+        jnext = jhi + 1;
+      }
+    }
+  }
+  return count + c.nxc;
+}
+
+// One work-group per tile: writes its entries (kFill), or their number to
+// indptr[t + 1].  Latency bound.  The attended key frames are taken 64 at a
+// time, a lane each: the lane's blocks are those of its frame past the ones
+// of the attended frame below it, a wave scan gives their places in the list,
+// and the list's entries are then dealt to all lanes, so that the descriptors
+// (divisions and relation reads) are computed in parallel.  One thread per
+// tile walking its ~400 entries took 146 us for 13 frames of 1350 tokens (35
+// us for 33 of 256), which every new pattern waits for.
 template <bool kFill>
 __global__ __launch_bounds__(kPlanThreads) void plan_tiles_kernel(PlanCtx c, int32_t* indptr, uint32_t* entries,
                                                                   int64_t cap) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= c.n_vt + c.n_tt) return;
-  const lvsa_plan_params& p = c.p;
-  int64_t pos = kFill ? (int64_t)indptr[t] : 0;
+  const int t = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t begin = kFill ? (int64_t)indptr[t] : 0;
   const int64_t end = kFill ? (int64_t)indptr[t + 1] : 0;
   int64_t count = 0;
-  auto emit = [&](uint32_t w0, uint32_t w1) {
-    if (kFill && pos < end && pos < cap) {
+  auto emit = [&](int64_t i, uint32_t w0, uint32_t w1) {
+    const int64_t pos = begin + i;
+    if (pos < end && pos < cap) {
       entries[2 * pos] = w0;
       entries[2 * pos + 1] = w1;
     }
-    ++pos;
-    ++count;
   };
   if (t < c.n_vt) {
-    const int64_t r0 = (int64_t)t * p.block_q;
-    const int64_t r1 = (r0 + p.block_q) < p.n_q ? (r0 + p.block_q) : p.n_q;
-    const int qf0 = (int)((p.q_tok0 + r0) / p.R) - p.q_frame0;
-    const int qf1 = (int)((p.q_tok0 + r1 - 1) / p.R) - p.q_frame0;
-    int64_t jnext = 0;
-    for (int w = 0; w < p.words; ++w) {
+    int64_t r0;
+    int qf0, qf1;
+    tile_frames(c, t, &r0, &qf0, &qf1);
+    int last = -1;                       // last block taken so far
+    for (int w = 0; w < c.p.words; w += 2) {
+      // this lane's frame; every wave does the same scan
       uint32_t u = 0;
-      for (int q = qf0; q <= qf1; ++q) u |= rel_word(c, q, w);
-      while (u) {
-        const int b = __ffs(u) - 1;
-        u &= u - 1;
-        const int64_t kf = 32 * (int64_t)w + b;
-        int64_t a = kf * p.C - p.k_tok0, e = a + p.C;
-        if (a < 0) a = 0;
-        if (e > p.n_k) e = p.n_k;
-        if (a >= e) continue;
-        const int64_t jlo = a / p.block_k, jhi = (e - 1) / p.block_k;
-        for (int64_t j = (jlo > jnext ? jlo : jnext); j <= jhi; ++j)
-          emit((uint32_t)j, frame_desc(c, r0, qf0, qf1, j));
-        if (jhi + 1 > jnext) jnext = jhi + 1;
+      for (int q = qf0; q <= qf1; ++q) u |= rel_word(c, q, w + (lane >> 5));
+      int jlo = 0, jhi = -1;
+      const bool on = ((u >> (lane & 31)) & 1u) && frame_blocks(c, 32 * (int64_t)w + lane, &jlo, &jhi);
+      const uint64_t active = __ballot(on);
+      if (active == 0) continue;
+      const uint64_t below = active & ((1ull << lane) - 1ull);
+      const int prev = __shfl(jhi, below ? 63 - __clzll(below) : 0);
+      const int taken = below ? prev : last;
+      if (jlo <= taken) jlo = taken + 1;
+      const int n = on && jhi >= jlo ? jhi - jlo + 1 : 0;
+      int incl = n;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(incl, o);
+        if (lane >= o) incl += x;
       }
+      const int total = __shfl(incl, 63);
+      if (kFill) {
+        for (int base = 0; base < total; base += kPlanThreads) {
+          const int i = base + tid;
+          int f = 0;                     // the lane whose frame holds entry i: lanes with incl <= i
+          for (int o = 32; o > 0; o >>= 1)
+            if (__shfl(incl, f + o - 1) <= i) f += o;
+          const int j = __shfl(jlo, f) + i - (__shfl(incl, f) - __shfl(n, f));
+          if (i < total) emit(count + i, (uint32_t)j, frame_desc(c, r0, qf0, qf1, j));
+        }
+      }
+      count += total;
+      last = __shfl(jhi, 63 - __clzll(active));
     }
   } else {
-    for (int64_t j = 0; j < c.nkc; ++j) emit((uint32_t)j, dense_desc(c, p.n_k, j));
+    if (kFill)
+      for (int j = tid; j < c.nkc; j += kPlanThreads) emit(j, (uint32_t)j, dense_desc(c, c.p.n_k, j));
+    count = c.nkc;
   }
-  for (int64_t j = 0; j < c.nxc; ++j) emit(kSrcExtra | (uint32_t)j, dense_desc(c, p.n_x, j));
-  if (!kFill) indptr[t + 1] = (int32_t)count;
+  if (kFill)
+    for (int j = tid; j < c.nxc; j += kPlanThreads) emit(count + j, kSrcExtra | (uint32_t)j, dense_desc(c, c.p.n_x, j));
+  if (!kFill && tid == 0) indptr[t + 1] = (int32_t)(count + c.nxc);
 }
 
-// indptr[1..n] holds per-tile counts; turn it into row pointers, clamped to
-// the entry capacity (status[0] = 1 when the bound was exceeded).
-__global__ __launch_bounds__(kScanThreads) void plan_scan_kernel(int32_t* indptr, int n, int64_t cap,
+// Row pointers from per-tile counts, clamped to the entry capacity
+// (status[0] = 1 when the bound was exceeded): an exclusive scan by one
+// work-group.  kCount: it counts the tiles' entries first, a thread per tile
+// (up to kCountTiles tiles of at most kCountFrames query frames, where that is
+// faster than a launch of its own), else indptr[1..n] holds them.
+constexpr int kCountTiles = 4 * kScanThreads, kCountFrames = 4;
+template <bool kCount>
+__global__ __launch_bounds__(kScanThreads) void plan_scan_kernel(PlanCtx c, int32_t* indptr, int n, int64_t cap,
                                                                  int32_t* status) {
-  __shared__ int scan_sh[kScanThreads];
+  __shared__ int scan_sh[kScanThreads / 64];
   const int tid = threadIdx.x, nt = blockDim.x;
   const int seg = (n + nt - 1) / nt;
   const int a = min(n, tid * seg), b = min(n, a + seg);
   int s = 0;
-  for (int i = a; i < b; ++i) s += indptr[i + 1];
+  for (int i = a; i < b; ++i) {
+    if (kCount) indptr[i + 1] = tile_count(c, i);
+    s += indptr[i + 1];
+  }
   int total;
   int acc = block_exclusive_scan(s, scan_sh, &total);
   for (int i = a; i < b; ++i) {
@@ -603,6 +690,11 @@ static int plan_ctx(const lvsa_plan_params* p, PlanCtx* c) {
   c->n_tt = (int)ceil_div(p->n_tq, p->block_q);
   c->nkc = (int)ceil_div(p->n_k, p->block_k);
   c->nxc = (int)ceil_div(p->n_x, p->block_k);
+  const int64_t R = p->R > 0 ? p->R : 1, C = p->C > 0 ? p->C : 1;   // unused without video rows
+  c->qo = (uint32_t)(p->q_tok0 % R);
+  c->ko = (uint32_t)(p->k_tok0 % C);
+  c->qf0 = (int)(p->q_tok0 / R - p->q_frame0);
+  c->kf0 = p->k_tok0 / C;
   return LVSA_OK;
 }
 
@@ -642,13 +734,18 @@ int lvsa_plan_build(const lvsa_plan_params* p, int32_t* tile_indptr, uint32_t* e
     hipLaunchKernelGGL(plan_empty_kernel, dim3(1), dim3(1), 0, stream, tile_indptr, (int32_t*)workspace);
     return launch_status("lvsa_plan_build");
   }
-  const dim3 grid((unsigned)ceil_div(n, kPlanThreads));
-  hipLaunchKernelGGL(plan_tiles_kernel<false>, grid, dim3(kPlanThreads), 0, stream, c, tile_indptr, entries,
-                     max_entries);
-  hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, tile_indptr, n, max_entries,
-                     (int32_t*)workspace);
-  hipLaunchKernelGGL(plan_tiles_kernel<true>, grid, dim3(kPlanThreads), 0, stream, c, tile_indptr, entries,
-                     max_entries);
+  int32_t* status = (int32_t*)workspace;
+  if (n <= kCountTiles && (c.n_vt == 0 || (p->block_q - 1) / p->R + 2 <= kCountFrames)) {
+    hipLaunchKernelGGL(plan_scan_kernel<true>, dim3(1), dim3(kScanThreads), 0, stream, c, tile_indptr, n, max_entries,
+                       status);
+  } else {
+    hipLaunchKernelGGL(plan_tiles_kernel<false>, dim3((unsigned)n), dim3(kPlanThreads), 0, stream, c, tile_indptr,
+                       entries, max_entries);
+    hipLaunchKernelGGL(plan_scan_kernel<false>, dim3(1), dim3(kScanThreads), 0, stream, c, tile_indptr, n, max_entries,
+                       status);
+  }
+  hipLaunchKernelGGL(plan_tiles_kernel<true>, dim3((unsigned)n), dim3(kPlanThreads), 0, stream, c, tile_indptr,
+                     entries, max_entries);
   return launch_status("lvsa_plan_build");
 }
 

@@ -179,6 +179,27 @@ def test_plan_block_csr_at_baseline(name, T, P, W, kfi, offs, b, gpu):
             assert got == cols, (name, off, bq, bk)
 
 
+@pytest.mark.parametrize("T,P,W,kfi,bq,bk", [
+    (140, 3, 2, 8, 128, 64),     # tiles of 43 query frames: counted by a work-group each; 5 words
+    (33, 130, 2, 8, 1, 64),      # 4290 tiles: more than the scan kernel counts itself
+    (65, 200, 1, 5, 256, 64),    # the last of 3 words holds one frame
+    (97, 131, 3, 4, 128, 64),    # 4 words
+    (9, 64, 1, 4, 256, 64),      # frames on the block grid
+    (8, 257, 1, None, 384, 255), # every frame shares blocks with its neighbours
+], ids=str)
+def test_plan_block_lists(T, P, W, kfi, bq, bk, gpu):
+    """Block lists of both ways to count a plan and of one- and two-word frame scans."""
+    ref = om.build_frame_mask(T, P, W, 1, kfi, offset=1)
+    dm = hip_ops.mask_build(hip_ops.mask_params(T, P, W, 1, kfi, 1), gpu)
+    N = T * P
+    plan = hip_ops.plan_build(dm.rel_full, n_q=N, n_k=N, R=P, Cf=P, max_row_frames=ref.compact_n, block_q=bq,
+                              block_k=bk)
+    indptr, cols = om.block_csr(om.frame_relation(ref), P, N, N, bq, bk)
+    assert plan.tile_indptr.cpu().tolist() == indptr
+    assert plan.status[:2].tolist() == [0, indptr[-1]]
+    assert (plan.entries[: indptr[-1], 0].cpu().numpy().astype(np.int64) & 0x7FFFFFFF).tolist() == cols
+
+
 def test_window_golden_arbitrary_global_sets(golden, gpu):
     """The reference's window bounds for 600 arbitrary global sets: each set
     goes in as boundary guards (no anchors, no keyframe grid), so the device's
