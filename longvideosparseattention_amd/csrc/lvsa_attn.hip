@@ -13,73 +13,6 @@ using namespace lvsa;
 
 namespace {
 
-// Key blocks (of 64 keys) per text chunk when a text tile is split: about a
-// third of a Wan / HunyuanVideo video tile and below a CogVideoX one, so the
-// chunks fill the launch's last round at a granularity finer than a tile
-// (64 measured the same at CogVideoX and 0.3% slower at HunyuanVideo).
-constexpr int kTextChunkBlocks = 128;
-constexpr int kMaxTextChunks = 64;
-
-// Text chunks per text tile (1 = no split): of a 16-bit call with a workspace,
-// and of an fp32 call with room for its split operands.
-int text_chunks_any(const lvsa_attn_args* a) {
-  if (a->n_tq == 0) return 1;
-  const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
-  const int64_t c = ceil_div(blocks, kTextChunkBlocks);
-  return (int)(c < 1 ? 1 : (c > kMaxTextChunks ? kMaxTextChunks : c));
-}
-
-int text_chunks_of(const lvsa_attn_args* a) { return a->dtype == LVSA_FP32 ? 1 : text_chunks_any(a); }
-
-int64_t text_ws_bytes(const lvsa_attn_args* a, int chunks) {
-  if (a->n_tq == 0 || chunks <= 1) return 0;
-  return 4 * (text_ws_o_elems(chunks, a->B, a->H, a->n_tq, a->D) + 2LL * chunks * a->B * a->H * a->n_tq);
-}
-
-// Partials of the video split with `vsplit` slots per queue (O, then the
-// (running max, row sum) pairs).
-int64_t video_ws_bytes(const lvsa_attn_args* a, int vsplit) {
-  if (vsplit <= 0) return 0;
-  return 4 * (video_ws_o_elems(vsplit, a->block_q, a->D) + 2LL * kXcds * vsplit * 2 * a->block_q);
-}
-
-// Workspace of a call: the text-split partials (text_ws_bytes) at offset 0,
-// the video-split partials (video_ws_bytes) after them at a 256-byte
-// boundary, then the work-queue counters (kQueueBytes) at the next one.
-int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
-int64_t video_offset(const lvsa_attn_args* a, int chunks) { return align256(text_ws_bytes(a, chunks)); }
-int64_t queue_offset(const lvsa_attn_args* a, int chunks, int vsplit) {
-  return align256(video_offset(a, chunks) + video_ws_bytes(a, vsplit));
-}
-int64_t ws_bytes(const lvsa_attn_args* a, int vsplit) {
-  return queue_offset(a, text_chunks_of(a), vsplit) + kQueueBytes;
-}
-
-// fp32: the text-split partials, the counters (unused) and, from
-// f32_split_offset, K and V of every key block as fp16 pairs
-// (lvsa_attn_f32.hip).  0 blocks where that scratch would pass kMaxSplitBytes
-// (as much as K and V themselves: 2.3 GB for 121 frames of 1560 tokens, 12
-// heads, D = 128) or the grid's 2^31: such a call runs the fp32 kernel.
-constexpr int64_t kMaxSplitBytes = 16LL << 30;
-int64_t f32_split_slots(const lvsa_attn_args* a) {
-  if (a->dtype != LVSA_FP32) return 0;
-  const int64_t slots = 2LL * a->B * a->Hkv * (ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN));
-  return slots >= (int64_t)INT32_MAX || f32_split_bytes(slots, a->D) > kMaxSplitBytes ? 0 : slots;
-}
-int64_t f32_split_offset(const lvsa_attn_args* a) {
-  return align256(queue_offset(a, text_chunks_any(a), 0) + kQueueBytes);
-}
-int64_t f32_ws_bytes(const lvsa_attn_args* a) {
-  const int64_t slots = f32_split_slots(a);
-  return slots ? f32_split_offset(a) + f32_split_bytes(slots, a->D) : ws_bytes(a, 0);
-}
-
-// Zero the work-queue counters (a kernel, not a memset, so the call can be
-// captured in a HIP graph and replayed).
-__global__ __launch_bounds__(64) void queue_reset_kernel(uint32_t* q) {
-  if (threadIdx.x < 8) q[threadIdx.x * (kQueueStride / 4)] = 0u;
-}
-
 // Compute units of the current device (the persistent grid of the
 // single-stream kernel), cached per device.
 int cu_count() {
@@ -95,6 +28,103 @@ int cu_count() {
   return cached[dev];
 }
 
+// Key blocks of a video tile, guessed (the plan's counts are on the device):
+// about six frames of anchors and window and a keyframe in eight, and the
+// extra rows.  Only balance depends on it.
+int64_t guessed_tile_blocks(const lvsa_attn_args* a) {
+  const int64_t C = a->C > 0 ? a->C : 1, frames = ceil_div(a->n_k, C);
+  const int64_t attended = 6 + ceil_div(frames, 8);
+  const int64_t all = ceil_div(a->n_k, kBN);
+  const int64_t b = attended < frames ? ceil_div(attended * C, kBN) : all;
+  return (b < all ? b : all) + ceil_div(a->n_x, kBN);
+}
+
+// Key blocks (of 64 keys) per text chunk when a text tile is split: about a
+// third of a Wan / HunyuanVideo video tile and below a CogVideoX one, so the
+// chunks fill the launch's last round at a granularity finer than a tile
+// (64 measured the same at CogVideoX and 0.3% slower at HunyuanVideo).
+// Beside video tiles of fewer blocks a chunk has as many as they (at least
+// kMinTextChunkBlocks), unless that takes more than kMaxSmallText of scratch:
+// 24 frames of 130 tokens, 12 heads, 37 text tokens ran its one 50-block text
+// tile per head whole, three times as long as its video tiles.
+constexpr int kTextChunkBlocks = 128, kMinTextChunkBlocks = 16;
+constexpr int kMaxTextChunks = 64;
+constexpr int64_t kMaxSmallText = 16LL << 20;
+
+int64_t text_ws_bytes(const lvsa_attn_args* a, int chunks) {
+  if (a->n_tq == 0 || chunks <= 1) return 0;
+  return 4 * (text_ws_o_elems(chunks, a->B, a->H, a->n_tq, a->D) + 2LL * chunks * a->B * a->H * a->n_tq);
+}
+
+// Text chunks per text tile (1 = no split): of a 16-bit call with a workspace,
+// and of an fp32 call with room for its split operands.
+int text_chunks_any(const lvsa_attn_args* a) {
+  if (a->n_tq == 0) return 1;
+  const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
+  auto chunks = [&](int64_t per) {
+    const int64_t c = ceil_div(blocks, per);
+    return (int)(c < 1 ? 1 : (c > kMaxTextChunks ? kMaxTextChunks : c));
+  };
+  if (a->n_q > 0) {
+    const int64_t tile = guessed_tile_blocks(a);
+    if (tile < kTextChunkBlocks) {
+      const int c = chunks(tile > kMinTextChunkBlocks ? tile : kMinTextChunkBlocks);
+      if (text_ws_bytes(a, c) <= kMaxSmallText) return c;
+    }
+  }
+  return chunks(kTextChunkBlocks);
+}
+
+int text_chunks_of(const lvsa_attn_args* a) { return a->dtype == LVSA_FP32 ? 1 : text_chunks_any(a); }
+
+// The video split of a call: `tiles` per queue in `parts` parts each.
+struct VideoSplit {
+  int tiles = 0, parts = 0;
+};
+
+// Partials of the video split (O, then the (running max, row sum) pairs).
+int64_t video_ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
+  if (v.tiles <= 0) return 0;
+  return 4 * (video_ws_o_elems(v.tiles, v.parts, a->block_q, a->D) + 2LL * kXcds * v.tiles * v.parts * a->block_q);
+}
+
+// Workspace of a call: the text-split partials (text_ws_bytes) at offset 0,
+// the video-split partials (video_ws_bytes) after them at a 256-byte
+// boundary, then the work-queue counters (kQueueBytes) at the next one.
+int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
+int64_t video_offset(const lvsa_attn_args* a, int chunks) { return align256(text_ws_bytes(a, chunks)); }
+int64_t queue_offset(const lvsa_attn_args* a, int chunks, VideoSplit v) {
+  return align256(video_offset(a, chunks) + video_ws_bytes(a, v));
+}
+int64_t ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
+  return queue_offset(a, text_chunks_of(a), v) + kQueueBytes;
+}
+
+// fp32: the partials of both splits, the counters (unused) and, from
+// f32_split_offset, K and V of every key block as fp16 pairs
+// (lvsa_attn_f32.hip).  0 blocks where that scratch would pass kMaxSplitBytes
+// (as much as K and V themselves: 2.3 GB for 121 frames of 1560 tokens, 12
+// heads, D = 128) or the grid's 2^31: such a call runs the fp32 kernel.
+constexpr int64_t kMaxSplitBytes = 16LL << 30;
+int64_t f32_split_slots(const lvsa_attn_args* a) {
+  if (a->dtype != LVSA_FP32) return 0;
+  const int64_t slots = 2LL * a->B * a->Hkv * (ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN));
+  return slots >= (int64_t)INT32_MAX || f32_split_bytes(slots, a->D) > kMaxSplitBytes ? 0 : slots;
+}
+int64_t f32_split_offset(const lvsa_attn_args* a, VideoSplit v) {
+  return align256(queue_offset(a, text_chunks_any(a), v) + kQueueBytes);
+}
+int64_t f32_ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
+  const int64_t slots = f32_split_slots(a);
+  return slots ? f32_split_offset(a, v) + f32_split_bytes(slots, a->D) : ws_bytes(a, VideoSplit{});
+}
+
+// Zero the work-queue counters (a kernel, not a memset, so the call can be
+// captured in a HIP graph and replayed).
+__global__ __launch_bounds__(64) void queue_reset_kernel(uint32_t* q) {
+  if (threadIdx.x < 8) q[threadIdx.x * (kQueueStride / 4)] = 0u;
+}
+
 // Whether a 16-bit head size 64 plan of 256-row tiles runs the dual map
 // (LVSA_D64_WAVES=8 selects 8 waves of 32 rows instead, for comparisons).
 bool dual_map(const lvsa_attn_args* a) {
@@ -102,24 +132,68 @@ bool dual_map(const lvsa_attn_args* a) {
   return a->D == 64 && a->block_q == kPPBM && a->dtype != LVSA_FP32 && !(w && strcmp(w, "8") == 0);
 }
 
-// Video tiles split in key-range halves at the end of each work queue, with
-// the dual map: its two work-groups per CU take whole tiles at half the CU's
-// rate, so a last round of whole tiles leaves CUs idle for longer.  As many
-// per queue as the queue has work-groups on its XCD, halved (32), so that the
-// last round runs half tiles, and at most the queue's video tiles
-// (CogVideoX 0.9% faster; the 8-wave maps, one work-group per CU, gain
-// nothing from it: Wan 4x and HunyuanVideo within +-0.5%).  0 for other maps,
-// fp32, calls too small for the work queues, or with LVSA_VIDEO_SPLIT=0.
-int vsplit_pref(const lvsa_attn_args* a) {
+// Work-groups of the call's kernel that run at once.  fp32: one per CU with
+// two key groups for at most that many items (launch_f32).
+int64_t concurrent_groups(const lvsa_attn_args* a, int64_t cus, int64_t vwork) {
+  if (a->dtype == LVSA_FP32) {
+    const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_any(a) * a->H * a->B;
+    return cus * (work <= cus ? 1 : a->D == 64 ? 3 : a->D <= 128 ? 2 : 1);
+  }
+  if (a->block_q == kBM && a->D <= 128) return 2 * cus;
+  return cus * (dual_map(a) ? 2 : 1);
+}
+
+// Video tiles that run as parts of their key ranges at the end of the launch,
+// so that its last round is finer than whole tiles.  None with
+// LVSA_VIDEO_SPLIT=0.
+// - The dual map over the work queues: its two work-groups per CU take whole
+//   tiles at half the CU's rate, so a last round of whole tiles leaves CUs
+//   idle for longer.  As many tiles per queue as the queue has work-groups on
+//   its XCD, halved (32), in two parts (CogVideoX 0.9% faster).
+// - Otherwise launches of fewer than kSplitRounds rounds, whose last round is
+//   not full: its tiles in the number of parts that ends soonest by a model of
+//   the last round (below), where that saves 7% and 5 us of it.  33 frames of 390
+//   tokens, 12 heads, D = 128 (612 tiles, 2.4 rounds): 383 -> 338 us and 10
+//   for the merge; 9 frames of 256 (108 tiles, one round): 46 -> 36 + 10, so
+//   whole.  Longer launches gain little from their last round and pay the same
+//   merge (Wan 4x and HunyuanVideo, 24 and 20 rounds, within +-0.5%).
+constexpr int kSplitRounds = 5, kMaxParts = 8;
+constexpr int64_t kMaxVideoSplitBytes = 48LL << 20;
+VideoSplit video_split_of(const lvsa_attn_args* a) {
+  VideoSplit v;
   const char* e = getenv("LVSA_VIDEO_SPLIT");
-  if ((e && strcmp(e, "0") == 0) || !dual_map(a) || a->n_q == 0) return 0;
-  const int per_cu = 2;
   const int64_t cus = cu_count();
+  if ((e && strcmp(e, "0") == 0) || a->n_q == 0 || a->block_q <= 0 || a->block_q == kStream12BM || cus <= 0) return v;
   const int64_t vwork = ceil_div(a->n_q, a->block_q) * a->H * a->B;
-  const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_of(a) * a->H * a->B;
-  if (cus <= 0 || work <= per_cu * cus) return 0;
-  const int64_t s = per_cu * cus / (2 * kXcds), per_queue = ceil_div(vwork, kXcds);
-  return (int)(s < per_queue ? s : per_queue);
+  const int64_t groups = concurrent_groups(a, cus, vwork);
+  if (dual_map(a)) {
+    const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_of(a) * a->H * a->B;
+    if (work > groups) {
+      const int64_t s = groups / (2 * kXcds), per_queue = ceil_div(vwork, kXcds);
+      v.tiles = (int)(s < per_queue ? s : per_queue);
+      v.parts = 2;
+      return v;
+    }
+  }
+  const int64_t rest = vwork % groups;
+  if (vwork >= kSplitRounds * groups || rest == 0) return v;
+  // Microseconds, as measured on launches of one round: about 1 per key block
+  // (fp32: 2.5 times that), 8 to start and end a launch and 5 per item; the
+  // merge 3 and its partials at 3 TB/s.
+  const double block_us = (0.75 + 0.3 * a->block_q * a->D / 32768.0) * (a->dtype == LVSA_FP32 ? 2.5 : 1.0);
+  const int64_t blocks = guessed_tile_blocks(a);
+  const double whole = 8.0 + blocks * block_us + 5.0;
+  double best = whole - (5.0 > 0.07 * whole ? 5.0 : 0.07 * whole);
+  for (int k = 2; k <= kMaxParts && blocks >= 6 * k; ++k) {
+    const VideoSplit w{(int)ceil_div(rest, kXcds), k};
+    const int64_t bytes = video_ws_bytes(a, w);
+    const double t = 8.0 + ceil_div(rest * k, groups) * (blocks * block_us / k + 5.0) + 3.0 + bytes / 3e6;
+    if (t < best && bytes <= kMaxVideoSplitBytes) {
+      best = t;
+      v = w;
+    }
+  }
+  return v;
 }
 
 // Exact log-sum-exp merge of the text chunks (lvsa-vllm-omni/lvsa_vllm_omni/
@@ -165,9 +239,10 @@ __global__ __launch_bounds__(256) void attn_text_merge_kernel(const float* ws, i
     lse_t[bh * n_tq + row] = L > 0.f ? (M + __log2f(L)) * 0.69314718055994530942f : -INFINITY;
 }
 
-// Merge of the two halves of the split video tiles (vsplit slots per queue):
-// one thread per (slot, row, 4 columns), the exact log-sum-exp combination
-// of attn_text_merge_kernel, written where the unsplit tile writes O and LSE.
+// Merge of the parts of the split video tiles (vsplit slots per queue): one
+// thread per (slot, row, 4 columns), the exact log-sum-exp combination of
+// attn_text_merge_kernel, written where the unsplit tile writes O and LSE.
+// Bound by the partials it reads.
 template <typename E>
 __global__ __launch_bounds__(256) void attn_video_merge_kernel(AttnParams p, int block_q, int D) {
   const int g4 = D / 4;
@@ -183,20 +258,29 @@ __global__ __launch_bounds__(256) void attn_video_merge_kernel(AttnParams p, int
   const int r = (int)((t % per_slot) / g4), dq = (int)(t % g4);
   const int64_t row = (int64_t)tile * block_q + r;
   if (row >= p.n_q) return;
-  const float2* ml = reinterpret_cast<const float2*>(p.vws + video_ws_o_elems(p.vsplit, block_q, D));
-  const int64_t i0 = (2 * slot) * block_q + r, i1 = i0 + block_q;
-  const float2 a0 = ml[i0], a1 = ml[i1];
-  const float M = fmaxf(a0.x, a1.x);
-  const float w0 = __builtin_amdgcn_exp2f(a0.x - M), w1 = __builtin_amdgcn_exp2f(a1.x - M);
-  const float L = w0 * a0.y + w1 * a1.y;
-  const float4 o0 = *reinterpret_cast<const float4*>(p.vws + i0 * D + 4 * dq);
-  const float4 o1 = *reinterpret_cast<const float4*>(p.vws + i1 * D + 4 * dq);
+  const float2* ml = reinterpret_cast<const float2*>(p.vws + video_ws_o_elems(p.vsplit, q.parts, block_q, D));
+  const int64_t i0 = (q.parts * slot) * block_q + r;
+  float M = -INFINITY;
+  for (int c = 0; c < q.parts; ++c) M = fmaxf(M, ml[i0 + (int64_t)c * block_q].x);
+  float L = 0.f;
+  float4 acc = float4{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < q.parts; ++c) {
+    const int64_t i = i0 + (int64_t)c * block_q;
+    const float2 mc = ml[i];
+    const float wt = __builtin_amdgcn_exp2f(mc.x - M);
+    const float4 o = *reinterpret_cast<const float4*>(p.vws + i * D + 4 * dq);
+    L += wt * mc.y;
+    acc.x += wt * o.x;
+    acc.y += wt * o.y;
+    acc.z += wt * o.z;
+    acc.w += wt * o.w;
+  }
   const float inv = L > 0.f ? 1.0f / L : 0.f;
-  E* op = reinterpret_cast<E*>(p.o + 2 * (batch * p.o_str[0] + row * p.o_str[1] + head * p.o_str[2])) + 4 * dq;
-  op[0] = (E)((w0 * o0.x + w1 * o1.x) * inv);
-  op[1] = (E)((w0 * o0.y + w1 * o1.y) * inv);
-  op[2] = (E)((w0 * o0.z + w1 * o1.z) * inv);
-  op[3] = (E)((w0 * o0.w + w1 * o1.w) * inv);
+  E* op = reinterpret_cast<E*>(p.o + sizeof(E) * (batch * p.o_str[0] + row * p.o_str[1] + head * p.o_str[2])) + 4 * dq;
+  op[0] = (E)(acc.x * inv);
+  op[1] = (E)(acc.y * inv);
+  op[2] = (E)(acc.z * inv);
+  op[3] = (E)(acc.w * inv);
   if (p.lse && dq == 0)
     p.lse[((int64_t)batch * p.H + head) * p.n_q + row] =
         L > 0.f ? (M + __log2f(L)) * 0.69314718055994530942f : -INFINITY;
@@ -293,9 +377,16 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   // fp32 with room for the split operands: K and V as fp16 pairs, text tiles
   // in chunks; without it (a smaller workspace, or none) the fp32 MFMAs and
   // whole text tiles.
-  const int64_t split_slots = fp32 && a->workspace && a->workspace_bytes >= f32_ws_bytes(a) ? f32_split_slots(a) : 0;
+  VideoSplit vsplit = a->workspace ? video_split_of(a) : VideoSplit{};
+  int64_t split_slots = 0;
+  if (fp32 && a->workspace) {
+    split_slots = f32_split_slots(a);
+    if (split_slots && a->workspace_bytes < f32_ws_bytes(a, vsplit)) vsplit = VideoSplit{};
+    if (split_slots && a->workspace_bytes < f32_ws_bytes(a, vsplit)) split_slots = 0;
+    if (!split_slots) vsplit = VideoSplit{};
+  }
   const int chunks = !a->workspace ? 1 : split_slots ? text_chunks_any(a) : text_chunks_of(a);
-  const int64_t ws_need = a->workspace ? ws_bytes(a, 0) : 0;   // without the video split
+  const int64_t ws_need = a->workspace ? ws_bytes(a, VideoSplit{}) : 0;   // without the video split
   LVSA_REQUIRE(a->workspace_bytes >= ws_need, LVSA_ERR_CAPACITY,
                "lvsa_attn_fwd: workspace of %lld bytes < %lld needed (lvsa_attn_workspace_query)",
                (long long)a->workspace_bytes, (long long)ws_need);
@@ -359,11 +450,15 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   p.split_exp = nullptr;
   p.split_slots = (int)split_slots;
   if (split_slots) {
-    p.split = (char*)a->workspace + f32_split_offset(a);
+    p.split = (char*)a->workspace + f32_split_offset(a, vsplit);
     p.split_exp = (int32_t*)(p.split + split_slots * 4LL * kBN * a->D);
   }
-  p.vsplit = 0;
-  p.vws = nullptr;
+  // the video split when the workspace holds its partials (the size
+  // lvsa_attn_workspace_query returns), none otherwise
+  if (!fp32 && vsplit.tiles > 0 && a->workspace_bytes < ws_bytes(a, vsplit)) vsplit = VideoSplit{};
+  p.vsplit = vsplit.tiles;
+  p.vparts = vsplit.parts;
+  p.vws = vsplit.tiles > 0 ? (float*)((char*)a->workspace + video_offset(a, chunks)) : nullptr;
   // The single-stream kernel (D = 64, 96 and 128 here; 192 and 256 below)
   // serves plans without generic descriptors:
   // 256-row tiles touch at most two query frames when frames have >= 255
@@ -430,18 +525,11 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   // work-group per CU (two with the dual map) over the work queues (counters
   // zeroed first).
   p.queues = nullptr;
-  p.grid = (int)work;
+  p.grid = static_grid(p);
   const int cus = cu_count();
   const int per_cu = p.dual ? 2 : 1;
   if (p.use_stream && a->workspace && cus > 0 && work > per_cu * cus) {
-    // the video split when the workspace holds its partials (the size
-    // lvsa_attn_workspace_query returns), none otherwise
-    const int vs = vsplit_pref(a);
-    if (vs > 0 && a->workspace_bytes >= ws_bytes(a, vs)) {
-      p.vsplit = vs;
-      p.vws = (float*)((char*)a->workspace + video_offset(a, chunks));
-    }
-    p.queues = (uint32_t*)((char*)a->workspace + queue_offset(a, chunks, p.vsplit));
+    p.queues = (uint32_t*)((char*)a->workspace + queue_offset(a, chunks, vsplit));
     p.grid = per_cu * cus;
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, stream, p.queues);
     const int qrc = launch_status("lvsa_attn_fwd (queue reset)");
@@ -460,7 +548,8 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   if (p.vsplit > 0) {
     const int64_t threads = (int64_t)kXcds * p.vsplit * bq * (a->D / 4);
     const dim3 grid((unsigned)ceil_div(threads, 256));
-    if (bf16) hipLaunchKernelGGL(attn_video_merge_kernel<__bf16>, grid, dim3(256), 0, stream, p, bq, a->D);
+    if (fp32) hipLaunchKernelGGL(attn_video_merge_kernel<float>, grid, dim3(256), 0, stream, p, bq, a->D);
+    else if (bf16) hipLaunchKernelGGL(attn_video_merge_kernel<__bf16>, grid, dim3(256), 0, stream, p, bq, a->D);
     else hipLaunchKernelGGL(attn_video_merge_kernel<_Float16>, grid, dim3(256), 0, stream, p, bq, a->D);
     rc = launch_status("lvsa_attn_fwd (video merge)");
     if (rc != LVSA_OK) return rc;
@@ -485,7 +574,7 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
 }
 
 namespace lvsa {
-int64_t attn_workspace_min_bytes(const lvsa_attn_args* a) { return ws_bytes(a, 0); }
+int64_t attn_workspace_min_bytes(const lvsa_attn_args* a) { return ws_bytes(a, VideoSplit{}); }
 }  // namespace lvsa
 
 extern "C" int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes) {
@@ -495,6 +584,7 @@ extern "C" int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes
                "lvsa_attn_workspace_query: bad sizes");
   LVSA_REQUIRE(a->D == 64 || a->D == 96 || a->D == 128 || a->D == 192 || a->D == 256, LVSA_ERR_UNSUPPORTED,
                "lvsa_attn_workspace_query: head_dim %d not supported", a->D);
-  *bytes = a->dtype == LVSA_FP32 ? f32_ws_bytes(a) : ws_bytes(a, vsplit_pref(a));
+  const VideoSplit v = video_split_of(a);
+  *bytes = a->dtype == LVSA_FP32 ? f32_ws_bytes(a, v) : ws_bytes(a, v);
   return LVSA_OK;
 }

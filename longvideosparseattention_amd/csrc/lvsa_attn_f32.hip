@@ -60,6 +60,7 @@ __device__ __forceinline__ Tile f32_tile(const AttnParams& p, const WorkItem& it
     t.nrows = p.n_q;
     t.r0 = (int64_t)it.tile * kBM;
     t.lse = p.lse ? p.lse + ((int64_t)it.batch * p.H + it.head) * p.n_q : nullptr;
+    if (it.vhalf >= 0) video_partial_dst<D>(p, it, kBM, t.r0, t.obase, t.ors, t.lse);
   } else {
     t.qbase = p.qt + 4 * (it.batch * p.qt_str[0] + it.head * p.qt_str[2]);
     t.obase = p.ot + 4 * (it.batch * p.ot_str[0] + it.head * p.ot_str[2]);
@@ -70,7 +71,7 @@ __device__ __forceinline__ Tile f32_tile(const AttnParams& p, const WorkItem& it
     t.lse = p.lse_t ? p.lse_t + ((int64_t)it.batch * p.H + it.head) * p.n_tq : nullptr;
     if (p.text_chunks > 1) text_partial_dst<D>(p, it, t.obase, t.ors, t.lse);
   }
-  t.partial = it.text && p.text_chunks > 1;
+  t.partial = (it.text && p.text_chunks > 1) || it.vhalf >= 0;
   item_entries(p, it, t.e0, t.e1);
   return t;
 }
@@ -245,6 +246,7 @@ __global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void attn_fwd_f32_kerne
   __shared__ __attribute__((aligned(16))) float lds[kF32Lds<D> / 4];
   __shared__ uint32_t relw[kBM * kRelPitch];
   const WorkItem it = map_work(p);
+  if (it.tile < 0) return;
   const Tile t = f32_tile<D>(p, it);
   // published by the first block's barrier
   if (p.rel_lds && !it.text) load_rel_rows<kBM>(p, relw, t.r0, t.nrows, threadIdx.x, kThreads);
@@ -390,6 +392,7 @@ void attn_fwd_split_kernel(AttnParams p) {
   lds_char* vs = ks + TILE;
 
   const WorkItem it = map_work(p);
+  if (it.tile < 0) return;
   const Tile t = f32_tile<D>(p, it);
   const int64_t my_row = t.r0 + 32 * rw + i32;
   const int my_tile_row = 32 * rw + i32;
@@ -670,7 +673,7 @@ void attn_fwd_split_kernel(AttnParams p) {
 
 template <int D>
 int launch_f32_d(const AttnParams& p, int cus, hipStream_t stream) {
-  const dim3 grid(p.total_work);
+  const dim3 grid(p.grid);
   if (!p.split) {
     hipLaunchKernelGGL(attn_fwd_f32_kernel<D>, grid, dim3(kThreads), 0, stream, p);
     return launch_status("lvsa_attn_fwd (fp32)");

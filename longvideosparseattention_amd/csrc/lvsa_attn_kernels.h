@@ -84,13 +84,13 @@ struct AttnParams {
   // D = 64, 256-row tiles on the single-stream kernel: the dual map (4 waves
   // of 64 rows, two work-groups per CU) rather than 8 waves of 32 rows
   int dual;
-  // Key-range split of each queue's last video tiles (with the work queues):
-  // the last min(vsplit, videos of the queue) video items of queue x run as
-  // two halves of their entry lists, after the queue's whole tiles, and write
-  // unnormalised partials to slots x * vsplit + s of vws (fp32 O [slot][half]
-  // [block_q][D], then (running max, row sum) [slot][half][block_q]) for
-  // attn_video_merge_kernel.  0: no split.
-  int vsplit;
+  // Key-range split of each queue's last video tiles: the last min(vsplit,
+  // videos of the queue) video items of queue x run as vparts (0: two) equal
+  // parts of their entry lists, after the queue's whole tiles, and write
+  // unnormalised partials to slots x * vsplit + s of vws (fp32 O
+  // [slot][part][block_q][D], then (running max, row sum)
+  // [slot][part][block_q]) for attn_video_merge_kernel.  0: no split.
+  int vsplit, vparts;
   float* vws;
   // Work queues (single-stream kernel with a workspace): `grid` persistent
   // work-groups, one per CU (two with the dual map), take work items from 8 queues, one per XCD,
@@ -252,64 +252,26 @@ __device__ __forceinline__ void wait_vm0() {
   __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
-// The work item of this work-group.  Video tiles are remapped so that
-// consecutive tiles of one head run on one XCD (work-groups are dispatched to
-// the 8 XCDs round-robin, and each XCD has its own L2): XCD x takes a
-// contiguous range of the video items.  Text items keep the dispatch order.
+// A work item: a query tile of one head, a chunk of a text tile, or a part of
+// a split video tile.
 struct WorkItem {
   int tile, head, batch, chunk;
   bool text;
-  int vhalf, vslot;   // a split video tile: half 0 or 1 and its partial slot; vhalf -1: whole
+  int vhalf, vslot;   // a split video tile: its part and its partial slot; vhalf -1: whole
 };
-__device__ __forceinline__ WorkItem map_work(const AttnParams& p) {
-  WorkItem it;
-  const int b = blockIdx.x;
-  const int tb0 = p.text_first ? 0 : p.n_vwork;  // first block of the text items
-  const int vb0 = p.text_first ? p.n_twork : 0;  // first block of the video items
-  if (b >= tb0 && b < tb0 + p.n_twork) {
-    int t = b - tb0;
-    it.chunk = t % p.text_chunks;
-    t /= p.text_chunks;
-    it.tile = p.n_vt + t % p.n_tt;
-    t /= p.n_tt;
-    it.head = t % p.H;
-    it.batch = t / p.H;
-    it.text = true;
-    it.vhalf = -1;
-    it.vslot = 0;
-    return it;
-  }
-  const int x = b % kXcds;
-  const int per = p.n_vwork / kXcds, rem = p.n_vwork % kXcds;
-  // video items on XCD y: per, plus one for the first `rem` XCDs in dispatch
-  // order after block vb0
-  int start = 0;
-  for (int y = 0; y < x; ++y) start += per + ((((y - vb0) % kXcds + kXcds) % kXcds) < rem ? 1 : 0);
-  const int first = vb0 + (((x - vb0) % kXcds + kXcds) % kXcds);  // first video block on XCD x
-  const int w = start + (b - first) / kXcds;
-  it.tile = w % p.n_vt;
-  const int rest = w / p.n_vt;
-  it.head = rest % p.H;
-  it.batch = rest / p.H;
-  it.chunk = 0;
-  it.text = false;
-  it.vhalf = -1;
-  it.vslot = 0;
-  return it;
-}
 
 // Work queues.  Queue x (one per XCD) holds, in this order: the unsplit text
 // items t = x, x + 8, ... (the longest, first), the video items of the same
 // XCD-contiguous range map_work gives XCD x (consecutive tiles of a head, so
 // the K/V blocks they share stay in that XCD's L2), the last n_split of them
-// as two halves each (key-range halves of their entry lists), and the split
-// text chunks t = x, x + 8, ... (the shortest, last).  The halves and the
-// chunks make the launch's last round finer than whole tiles.  A work-group takes items from the
-// queue of its own XCD and, once that is empty, from the next ones in turn:
+// as vparts key ranges each, and the split text chunks t = x, x + 8, ... (the
+// shortest, last).  The parts and the chunks make the launch's last round
+// finer than whole tiles.  A work-group takes items from the queue of its own XCD and, once that is empty, from the next ones in turn:
 // XCDs that run faster take over the items of the slower ones at the end, so
 // the launch does not wait for the slowest XCD's fixed share.
 struct QueueShape {
-  int n_first, v0, n_video, n_split, n_last;   // n_split of the n_video video items run as two halves
+  int n_first, v0, n_video, n_split, n_last;   // n_split of the n_video video items run as `parts` parts
+  int parts;
 };
 __host__ __device__ inline QueueShape queue_shape(const AttnParams& p, int x) {
   QueueShape q;
@@ -320,11 +282,14 @@ __host__ __device__ inline QueueShape queue_shape(const AttnParams& p, int x) {
   q.v0 = x * per + (x < rem ? x : rem);
   q.n_video = per + (x < rem ? 1 : 0);
   q.n_split = p.vsplit < q.n_video ? p.vsplit : q.n_video;
+  q.parts = p.vparts > 2 ? p.vparts : 2;
   return q;
 }
 
 // Items in queue x.
-__host__ __device__ inline int queue_items(const QueueShape& q) { return q.n_first + q.n_video + q.n_split + q.n_last; }
+__host__ __device__ inline int queue_items(const QueueShape& q) {
+  return q.n_first + q.n_video + q.n_split * (q.parts - 1) + q.n_last;
+}
 
 __host__ __device__ inline WorkItem text_item(const AttnParams& p, int t) {
   WorkItem it;
@@ -346,15 +311,15 @@ __host__ __device__ inline WorkItem queue_item(const AttnParams& p, int x, int j
   if (j < q.n_first) return text_item(p, x + kXcds * j);
   j -= q.n_first;
   const int n_whole = q.n_video - q.n_split;
-  if (j >= n_whole + 2 * q.n_split) return text_item(p, x + kXcds * (j - n_whole - 2 * q.n_split));
+  if (j >= n_whole + q.parts * q.n_split) return text_item(p, x + kXcds * (j - n_whole - q.parts * q.n_split));
   WorkItem it;
   it.vhalf = -1;
   it.vslot = 0;
   int w = q.v0 + j;
-  if (j >= n_whole) {                 // half j & 1 of split tile s of the queue
-    const int s = (j - n_whole) >> 1;
+  if (j >= n_whole) {                 // a part of split tile s of the queue
+    const int s = (j - n_whole) / q.parts;
     w = q.v0 + n_whole + s;
-    it.vhalf = (j - n_whole) & 1;
+    it.vhalf = (j - n_whole) - s * q.parts;
     it.vslot = x * p.vsplit + s;
   }
   it.tile = w % p.n_vt;
@@ -363,6 +328,26 @@ __host__ __device__ inline WorkItem queue_item(const AttnParams& p, int x, int j
   it.batch = rest / p.H;
   it.chunk = 0;
   it.text = false;
+  return it;
+}
+
+// The work item of this work-group without work queues: item b / 8 of queue
+// b % 8 (work-groups are dispatched to the 8 XCDs round-robin), so that
+// consecutive tiles of one head run on one XCD, as with the queues.  tile -1:
+// past the end of a shorter queue (the grid is 8 times the longest).
+__host__ __device__ inline int static_grid(const AttnParams& p) {
+  int n = 0;
+  for (int x = 0; x < kXcds; ++x) {
+    const int m = queue_items(queue_shape(p, x));
+    n = m > n ? m : n;
+  }
+  return kXcds * n;
+}
+__device__ __forceinline__ WorkItem map_work(const AttnParams& p) {
+  const int x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+  WorkItem it;
+  it.tile = -1;
+  if (j < queue_items(queue_shape(p, x))) it = queue_item(p, x, j);
   return it;
 }
 
@@ -403,23 +388,24 @@ __device__ __forceinline__ void store_text_partial(char* wo, float* ml, int h, c
   if (h == 0) *reinterpret_cast<float2*>(ml) = float2{m_run, l_tot};
 }
 
-// Elements of the O partials of the video split: vsplit slots per queue, two
-// halves per slot, block_q rows of D.
-__host__ __device__ inline int64_t video_ws_o_elems(int vsplit, int block_q, int D) {
-  return (int64_t)kXcds * vsplit * 2 * block_q * D;
+// Elements of the O partials of the video split: vsplit slots per queue,
+// `parts` parts per slot, block_q rows of D.
+__host__ __device__ inline int64_t video_ws_o_elems(int vsplit, int parts, int block_q, int D) {
+  return (int64_t)kXcds * vsplit * parts * block_q * D;
 }
 
-// A half of a split video tile writes its partials where a tile writes its
+// A part of a split video tile writes its partials where a tile writes its
 // output: row base, row stride and LSE pointer redirected to its slot, offset
 // so that the tile's first row r0 lands on the slot's row 0.
 template <int D>
 __device__ __forceinline__ void video_partial_dst(const AttnParams& p, const WorkItem& it, int block_q, int64_t r0,
                                                   char*& obase, int64_t& ors, float*& lse) {
-  const int64_t slot = 2 * (int64_t)it.vslot + it.vhalf;
+  const int parts = p.vparts > 2 ? p.vparts : 2;
+  const int64_t slot = (int64_t)parts * it.vslot + it.vhalf;
   const uintptr_t ws = reinterpret_cast<uintptr_t>(p.vws);
   ors = 4 * D;
   obase = reinterpret_cast<char*>(ws + 4 * (slot * block_q - r0) * D);
-  lse = reinterpret_cast<float*>(ws + 4 * (video_ws_o_elems(p.vsplit, block_q, D) + 2 * (slot * block_q - r0)));
+  lse = reinterpret_cast<float*>(ws + 4 * (video_ws_o_elems(p.vsplit, parts, block_q, D) + 2 * (slot * block_q - r0)));
 }
 
 // A split text item writes its partials where a tile writes its output: the
@@ -435,19 +421,16 @@ __device__ __forceinline__ void text_partial_dst(const AttnParams& p, const Work
   lse = p.ws + text_ws_o_elems(p.text_chunks, p.B, p.H, p.n_tq, D) + 2 * slot;
 }
 
-// Entry range [e0, e1) of the work item: the tile's plan entries, chunk
-// `chunk` of text_chunks equal parts of them, or half `vhalf` of a split
-// video tile's (the first half takes the odd entry).
+// Entry range [e0, e1) of the work item: the tile's plan entries, or chunk
+// `chunk` of text_chunks (part `vhalf` of a split video tile's parts) equal
+// shares of them.
 __device__ __forceinline__ void item_entries(const AttnParams& p, const WorkItem& it, int& e0, int& e1) {
   e0 = p.tile_indptr[it.tile];
   e1 = p.tile_indptr[it.tile + 1];
-  if (it.vhalf >= 0) {
-    const int mid = e0 + (e1 - e0 + 1) / 2;
-    if (it.vhalf == 0) e1 = mid;
-    else e0 = mid;
-  } else if (it.text && p.text_chunks > 1) {
-    const int len = (e1 - e0 + p.text_chunks - 1) / p.text_chunks;
-    const int a = e0 + it.chunk * len;
+  const int shares = it.vhalf >= 0 ? (p.vparts > 2 ? p.vparts : 2) : it.text ? p.text_chunks : 1;
+  if (shares > 1) {
+    const int len = (e1 - e0 + shares - 1) / shares;
+    const int a = e0 + (it.vhalf >= 0 ? it.vhalf : it.chunk) * len;
     e0 = a < e1 ? a : e1;
     e1 = e0 + len < e1 ? e0 + len : e1;
   }
@@ -568,6 +551,7 @@ __global__ __launch_bounds__(kThreads, D >= 192 ? 1 : 2) void attn_fwd_kernel(At
   const int i32 = lane & 31;      // query row of this lane within the wave
 
   const WorkItem it = map_work(p);
+  if (it.tile < 0) return;
   const int tile = it.tile, head = it.head, batch = it.batch;
   const bool text = it.text;
   const int hk = head / p.group;
@@ -586,6 +570,7 @@ __global__ __launch_bounds__(kThreads, D >= 192 ? 1 : 2) void attn_fwd_kernel(At
     nrows = p.n_q;
     r0 = (int64_t)tile * kBM;
     lse = p.lse ? p.lse + ((int64_t)batch * p.H + head) * p.n_q : nullptr;
+    if (it.vhalf >= 0) video_partial_dst<D>(p, it, kBM, r0, obase, ors, lse);
   } else {
     qbase = p.qt + 2 * (batch * p.qt_str[0] + head * p.qt_str[2]);
     obase = p.ot + 2 * (batch * p.ot_str[0] + head * p.ot_str[2]);
@@ -596,7 +581,7 @@ __global__ __launch_bounds__(kThreads, D >= 192 ? 1 : 2) void attn_fwd_kernel(At
     lse = p.lse_t ? p.lse_t + ((int64_t)batch * p.H + head) * p.n_tq : nullptr;
     if (p.text_chunks > 1) text_partial_dst<D>(p, it, obase, ors, lse);
   }
-  const bool partial = text && p.text_chunks > 1;
+  const bool partial = (text && p.text_chunks > 1) || it.vhalf >= 0;
   int e0, e1;
   item_entries(p, it, e0, e1);
 
@@ -1009,6 +994,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void attn_fwd_pp_kernel(AttnParams p
   const int i32 = lane & 31;
 
   const WorkItem it = map_work(p);
+  if (it.tile < 0) return;
   const int tile = it.tile, head = it.head, batch = it.batch;
   const bool text = it.text;
   const int hk = head / p.group;
@@ -1027,6 +1013,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void attn_fwd_pp_kernel(AttnParams p
     nrows = p.n_q;
     r0 = (int64_t)tile * kPPBM;
     lse = p.lse ? p.lse + ((int64_t)batch * p.H + head) * p.n_q : nullptr;
+    if (it.vhalf >= 0) video_partial_dst<D>(p, it, kPPBM, r0, obase, ors, lse);
   } else {
     qbase = p.qt + 2 * (batch * p.qt_str[0] + head * p.qt_str[2]);
     obase = p.ot + 2 * (batch * p.ot_str[0] + head * p.ot_str[2]);
@@ -1037,7 +1024,7 @@ __global__ __launch_bounds__(kPPThreads, 1) void attn_fwd_pp_kernel(AttnParams p
     lse = p.lse_t ? p.lse_t + ((int64_t)batch * p.H + head) * p.n_tq : nullptr;
     if (p.text_chunks > 1) text_partial_dst<D>(p, it, obase, ors, lse);
   }
-  const bool partial = text && p.text_chunks > 1;
+  const bool partial = (text && p.text_chunks > 1) || it.vhalf >= 0;
   int e0, e1;
   item_entries(p, it, e0, e1);
   const int n = e1 - e0;
@@ -1515,17 +1502,17 @@ template <int D, typename E>
 int launch(const AttnParams& prm, int block_q, hipStream_t stream) {
   if constexpr (D == 96) {
     (void)block_q;
-    hipLaunchKernelGGL((attn_fwd_pp_kernel<D, E>), dim3(prm.total_work), dim3(kPPThreads), 0, stream, prm);
+    hipLaunchKernelGGL((attn_fwd_pp_kernel<D, E>), dim3(prm.grid), dim3(kPPThreads), 0, stream, prm);
     return launch_status("lvsa_attn_fwd");
   }
   if constexpr (D == 64 || D == 128) {
     if (block_q == kPPBM) {
-      hipLaunchKernelGGL((attn_fwd_pp_kernel<D, E>), dim3(prm.total_work), dim3(kPPThreads), 0, stream, prm);
+      hipLaunchKernelGGL((attn_fwd_pp_kernel<D, E>), dim3(prm.grid), dim3(kPPThreads), 0, stream, prm);
       return launch_status("lvsa_attn_fwd");
     }
   }
   if constexpr (D != 96) {
-    hipLaunchKernelGGL((attn_fwd_kernel<D, E>), dim3(prm.total_work), dim3(kThreads), 0, stream, prm);
+    hipLaunchKernelGGL((attn_fwd_kernel<D, E>), dim3(prm.grid), dim3(kThreads), 0, stream, prm);
   }
   return launch_status("lvsa_attn_fwd");
 }

@@ -439,6 +439,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && D == 64) ? 2 : 1) void attn_fw
     } else {
       if (!first) break;
       it = map_work(p);
+      if (it.tile < 0) break;
     }
     stream_item<D, NW, E, DW>(p, it, lds0);   // one call site: one copy of the key loop
     __syncthreads();

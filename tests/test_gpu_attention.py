@@ -897,6 +897,43 @@ def test_work_queues_match_static_grid(cfg, gpu, monkeypatch):
         _close(ot1[:1], rto, "queued text rows")
 
 
+PARTS = [
+    # T, P, H, Hkv, D, n_txt, dtype: fewer rounds than kSplitRounds with a part-filled last one
+    (9, 512, 4, 2, 128, 0, torch.bfloat16),     # 72 tiles on 256 CUs: every tile in parts, no queues
+    (33, 400, 6, 6, 128, 40, torch.float16),    # 312 tiles: the work queues, text chunks
+    (9, 600, 3, 1, 64, 0, torch.bfloat16),      # the dual map below its queue launch
+    (9, 600, 3, 3, 96, 5, torch.bfloat16),
+    (9, 500, 4, 2, 192, 0, torch.bfloat16),     # dual-wide map
+    (9, 500, 2, 2, 256, 9, torch.float16),      # wide map, 128-row tiles
+    (50, 200, 3, 3, 128, 0, torch.bfloat16),    # ping-pong kernel, generic masks
+    (50, 126, 1, 1, 256, 0, torch.bfloat16),    # 4-wave kernel
+    (9, 500, 2, 1, 128, 0, torch.float32),      # fp32, two key groups
+    (13, 900, 9, 9, 64, 70, torch.float32),     # fp32, more tiles than concurrent work-groups
+    (9, 500, 2, 1, 256, 0, torch.float32),
+]
+
+
+@pytest.mark.parametrize("cfg", PARTS, ids=[str(c[:6]) for c in PARTS])
+def test_video_tiles_in_parts(cfg, gpu, monkeypatch):
+    """Last-round tiles as key-range parts merged by log-sum-exp, against whole
+    tiles (LVSA_VIDEO_SPLIT=0): O and LSE within the rounding of the merge."""
+    T, P, H, Hkv, D, n_txt, dt = cfg
+    N = T * P
+    m = _meta(T, P, 2, 1, 8, 3)
+    q, k, v, qt, kt, vt = (x.to(gpu) for x in _draw(
+        [(1, N, H, D), (1, N, Hkv, D), (1, N, Hkv, D), (1, n_txt, H, D), (1, n_txt, Hkv, D), (1, n_txt, Hkv, D)],
+        seed=33, dtype=dt))
+    kw = dict(k_text=kt, v_text=vt, q_text=qt) if n_txt else {}
+    parts = lv.lvsa_attention(q, k, v, m, return_lse=True, **kw)
+    monkeypatch.setenv("LVSA_VIDEO_SPLIT", "0")
+    whole = lv.lvsa_attention(q, k, v, m, return_lse=True, **kw)
+    assert not torch.equal(parts[0], whole[0]), "no tile was split"
+    # one rounding of the output type (|O| < 1) each; fp32: a few of the merge
+    tol = {torch.bfloat16: 4e-3, torch.float16: 1e-3, torch.float32: 2e-6}[dt]
+    for a, b in zip(parts, whole):
+        torch.testing.assert_close(a.float(), b.float(), atol=tol, rtol=tol)
+
+
 TALL = [
     # T, P, W, kfi, off, H, Hkv, D, n_txt, dtype, B  (head size 64, frames >= 383 rows: 384-row tiles possible)
     (13, 1350, 1, 4, 0, 6, 6, 64, 226, torch.bfloat16, 1),     # CogVideoX frame and text sizes
