@@ -43,10 +43,11 @@ int64_t guessed_tile_blocks(const lvsa_attn_args* a) {
 // third of a Wan / HunyuanVideo video tile and below a CogVideoX one, so the
 // chunks fill the launch's last round at a granularity finer than a tile
 // (64 measured the same at CogVideoX and 0.3% slower at HunyuanVideo).
-// Beside video tiles of fewer blocks a chunk has as many as they (at least
-// kMinTextChunkBlocks), unless that takes more than kMaxSmallText of scratch:
-// 24 frames of 130 tokens, 12 heads, 37 text tokens ran its one 50-block text
-// tile per head whole, three times as long as its video tiles.
+// Text tiles of one such chunk beside shorter video tiles run in chunks as
+// long as those (at least kMinTextChunkBlocks), unless that takes more than
+// kMaxSmallText of scratch or than the caller's: 24 frames of 130 tokens, 12
+// heads, 37 text tokens ran its one 50-block text tile per head whole, three
+// times as long as its video tiles (69.6 us per call, 59.1 in chunks).
 constexpr int kTextChunkBlocks = 128, kMinTextChunkBlocks = 16;
 constexpr int kMaxTextChunks = 64;
 constexpr int64_t kMaxSmallText = 16LL << 20;
@@ -56,26 +57,25 @@ int64_t text_ws_bytes(const lvsa_attn_args* a, int chunks) {
   return 4 * (text_ws_o_elems(chunks, a->B, a->H, a->n_tq, a->D) + 2LL * chunks * a->B * a->H * a->n_tq);
 }
 
-// Text chunks per text tile (1 = no split): of a 16-bit call with a workspace,
-// and of an fp32 call with room for its split operands.
-int text_chunks_any(const lvsa_attn_args* a) {
+// Text chunks per text tile (1 = no split).
+int text_chunks_of(const lvsa_attn_args* a) {
   if (a->n_tq == 0) return 1;
   const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
-  auto chunks = [&](int64_t per) {
-    const int64_t c = ceil_div(blocks, per);
-    return (int)(c < 1 ? 1 : (c > kMaxTextChunks ? kMaxTextChunks : c));
-  };
-  if (a->n_q > 0) {
+  const int64_t c = ceil_div(blocks, kTextChunkBlocks);
+  if (c <= 1 && a->n_q > 0) {
     const int64_t tile = guessed_tile_blocks(a);
-    if (tile < kTextChunkBlocks) {
-      const int c = chunks(tile > kMinTextChunkBlocks ? tile : kMinTextChunkBlocks);
-      if (text_ws_bytes(a, c) <= kMaxSmallText) return c;
-    }
+    const int f = (int)ceil_div(blocks, tile > kMinTextChunkBlocks ? tile : kMinTextChunkBlocks);
+    if (text_ws_bytes(a, f) <= kMaxSmallText) return f < 1 ? 1 : f;
   }
-  return chunks(kTextChunkBlocks);
+  return (int)(c < 1 ? 1 : (c > kMaxTextChunks ? kMaxTextChunks : c));
 }
 
-int text_chunks_of(const lvsa_attn_args* a) { return a->dtype == LVSA_FP32 ? 1 : text_chunks_any(a); }
+// Chunks that every workspace has to hold the partials of: those of long text
+// tiles in 16 bit.
+int text_chunks_least(const lvsa_attn_args* a) {
+  const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
+  return a->dtype == LVSA_FP32 || blocks <= kTextChunkBlocks ? 1 : text_chunks_of(a);
+}
 
 // The video split of a call: `tiles` per queue in `parts` parts each.
 struct VideoSplit {
@@ -88,35 +88,44 @@ int64_t video_ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
   return 4 * (video_ws_o_elems(v.tiles, v.parts, a->block_q, a->D) + 2LL * kXcds * v.tiles * v.parts * a->block_q);
 }
 
-// Workspace of a call: the text-split partials (text_ws_bytes) at offset 0,
-// the video-split partials (video_ws_bytes) after them at a 256-byte
-// boundary, then the work-queue counters (kQueueBytes) at the next one.
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
-int64_t video_offset(const lvsa_attn_args* a, int chunks) { return align256(text_ws_bytes(a, chunks)); }
-int64_t queue_offset(const lvsa_attn_args* a, int chunks, VideoSplit v) {
-  return align256(video_offset(a, chunks) + video_ws_bytes(a, v));
-}
-int64_t ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
-  return queue_offset(a, text_chunks_of(a), v) + kQueueBytes;
-}
 
-// fp32: the partials of both splits, the counters (unused) and, from
-// f32_split_offset, K and V of every key block as fp16 pairs
-// (lvsa_attn_f32.hip).  0 blocks where that scratch would pass kMaxSplitBytes
-// (as much as K and V themselves: 2.3 GB for 121 frames of 1560 tokens, 12
-// heads, D = 128) or the grid's 2^31: such a call runs the fp32 kernel.
+// fp32: blocks of K and V as fp16 pairs (lvsa_attn_f32.hip).  0 where that
+// scratch would pass kMaxSplitBytes (as much as K and V themselves: 2.3 GB for
+// 121 frames of 1560 tokens, 12 heads, D = 128) or the grid's 2^31: such a
+// call runs the fp32 kernel.
 constexpr int64_t kMaxSplitBytes = 16LL << 30;
 int64_t f32_split_slots(const lvsa_attn_args* a) {
   if (a->dtype != LVSA_FP32) return 0;
   const int64_t slots = 2LL * a->B * a->Hkv * (ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN));
   return slots >= (int64_t)INT32_MAX || f32_split_bytes(slots, a->D) > kMaxSplitBytes ? 0 : slots;
 }
-int64_t f32_split_offset(const lvsa_attn_args* a, VideoSplit v) {
-  return align256(queue_offset(a, text_chunks_any(a), v) + kQueueBytes);
+
+// Workspace of a call: the text-split partials at offset 0, the video-split
+// partials, the work-queue counters (kQueueBytes) and the fp32 pairs after
+// them, each at a 256-byte boundary.
+struct Scratch {
+  int chunks;
+  VideoSplit v;
+  int64_t slots, video, queue, split, bytes;
+};
+Scratch scratch_of(const lvsa_attn_args* a, int chunks, VideoSplit v, int64_t slots) {
+  Scratch s{chunks, v, slots, 0, 0, 0, 0};
+  s.video = align256(text_ws_bytes(a, chunks));
+  s.queue = align256(s.video + video_ws_bytes(a, v));
+  s.bytes = s.queue + kQueueBytes;
+  s.split = align256(s.bytes);
+  if (slots) s.bytes = s.split + f32_split_bytes(slots, a->D);
+  return s;
 }
-int64_t f32_ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
+VideoSplit video_split_of(const lvsa_attn_args* a);
+// What lvsa_attn_workspace_query asks for, and the least that a workspace must
+// be (whole tiles, fp32 on the fp32 MFMAs).
+Scratch scratch_least(const lvsa_attn_args* a) { return scratch_of(a, text_chunks_least(a), VideoSplit{}, 0); }
+Scratch scratch_full(const lvsa_attn_args* a, bool video_split = true) {
   const int64_t slots = f32_split_slots(a);
-  return slots ? f32_split_offset(a, v) + f32_split_bytes(slots, a->D) : ws_bytes(a, VideoSplit{});
+  if (a->dtype == LVSA_FP32 && slots == 0) return scratch_least(a);
+  return scratch_of(a, text_chunks_of(a), video_split ? video_split_of(a) : VideoSplit{}, slots);
 }
 
 // Zero the work-queue counters (a kernel, not a memset, so the call can be
@@ -136,7 +145,7 @@ bool dual_map(const lvsa_attn_args* a) {
 // two key groups for at most that many items (launch_f32).
 int64_t concurrent_groups(const lvsa_attn_args* a, int64_t cus, int64_t vwork) {
   if (a->dtype == LVSA_FP32) {
-    const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_any(a) * a->H * a->B;
+    const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_of(a) * a->H * a->B;
     return cus * (work <= cus ? 1 : a->D == 64 ? 3 : a->D <= 128 ? 2 : 1);
   }
   if (a->block_q == kBM && a->D <= 128) return 2 * cus;
@@ -374,19 +383,18 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
                  "lvsa_attn_fwd: query rows map to relation rows [%lld, %lld], the relation has %d rows",
                  (long long)first, (long long)last, a->rel_rows);
   }
-  // fp32 with room for the split operands: K and V as fp16 pairs, text tiles
-  // in chunks; without it (a smaller workspace, or none) the fp32 MFMAs and
-  // whole text tiles.
-  VideoSplit vsplit = a->workspace ? video_split_of(a) : VideoSplit{};
-  int64_t split_slots = 0;
-  if (fp32 && a->workspace) {
-    split_slots = f32_split_slots(a);
-    if (split_slots && a->workspace_bytes < f32_ws_bytes(a, vsplit)) vsplit = VideoSplit{};
-    if (split_slots && a->workspace_bytes < f32_ws_bytes(a, vsplit)) split_slots = 0;
-    if (!split_slots) vsplit = VideoSplit{};
+  // As much of the scratch as the workspace holds: all, without the video
+  // split, or the least.
+  Scratch ws{1, VideoSplit{}, 0, 0, 0, 0, 0};
+  int64_t ws_need = 0;
+  if (a->workspace) {
+    const Scratch least = scratch_least(a);
+    ws_need = least.bytes;
+    ws = scratch_full(a);
+    if (ws.bytes > a->workspace_bytes) ws = scratch_full(a, false);
+    if (ws.bytes > a->workspace_bytes) ws = least;
   }
-  const int chunks = !a->workspace ? 1 : split_slots ? text_chunks_any(a) : text_chunks_of(a);
-  const int64_t ws_need = a->workspace ? ws_bytes(a, VideoSplit{}) : 0;   // without the video split
+  const int chunks = ws.chunks;
   LVSA_REQUIRE(a->workspace_bytes >= ws_need, LVSA_ERR_CAPACITY,
                "lvsa_attn_fwd: workspace of %lld bytes < %lld needed (lvsa_attn_workspace_query)",
                (long long)a->workspace_bytes, (long long)ws_need);
@@ -448,17 +456,14 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   p.ws = chunks > 1 ? (float*)a->workspace : nullptr;
   p.split = nullptr;
   p.split_exp = nullptr;
-  p.split_slots = (int)split_slots;
-  if (split_slots) {
-    p.split = (char*)a->workspace + f32_split_offset(a, vsplit);
-    p.split_exp = (int32_t*)(p.split + split_slots * 4LL * kBN * a->D);
+  p.split_slots = (int)ws.slots;
+  if (ws.slots) {
+    p.split = (char*)a->workspace + ws.split;
+    p.split_exp = (int32_t*)(p.split + ws.slots * 4LL * kBN * a->D);
   }
-  // the video split when the workspace holds its partials (the size
-  // lvsa_attn_workspace_query returns), none otherwise
-  if (!fp32 && vsplit.tiles > 0 && a->workspace_bytes < ws_bytes(a, vsplit)) vsplit = VideoSplit{};
-  p.vsplit = vsplit.tiles;
-  p.vparts = vsplit.parts;
-  p.vws = vsplit.tiles > 0 ? (float*)((char*)a->workspace + video_offset(a, chunks)) : nullptr;
+  p.vsplit = ws.v.tiles;
+  p.vparts = ws.v.parts;
+  p.vws = ws.v.tiles > 0 ? (float*)((char*)a->workspace + ws.video) : nullptr;
   // The single-stream kernel (D = 64, 96 and 128 here; 192 and 256 below)
   // serves plans without generic descriptors:
   // 256-row tiles touch at most two query frames when frames have >= 255
@@ -529,7 +534,7 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   const int cus = cu_count();
   const int per_cu = p.dual ? 2 : 1;
   if (p.use_stream && a->workspace && cus > 0 && work > per_cu * cus) {
-    p.queues = (uint32_t*)((char*)a->workspace + queue_offset(a, chunks, vsplit));
+    p.queues = (uint32_t*)((char*)a->workspace + ws.queue);
     p.grid = per_cu * cus;
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, stream, p.queues);
     const int qrc = launch_status("lvsa_attn_fwd (queue reset)");
@@ -574,7 +579,7 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
 }
 
 namespace lvsa {
-int64_t attn_workspace_min_bytes(const lvsa_attn_args* a) { return ws_bytes(a, VideoSplit{}); }
+int64_t attn_workspace_min_bytes(const lvsa_attn_args* a) { return scratch_least(a).bytes; }
 }  // namespace lvsa
 
 extern "C" int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes) {
@@ -584,7 +589,6 @@ extern "C" int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes
                "lvsa_attn_workspace_query: bad sizes");
   LVSA_REQUIRE(a->D == 64 || a->D == 96 || a->D == 128 || a->D == 192 || a->D == 256, LVSA_ERR_UNSUPPORTED,
                "lvsa_attn_workspace_query: head_dim %d not supported", a->D);
-  const VideoSplit v = video_split_of(a);
-  *bytes = a->dtype == LVSA_FP32 ? f32_ws_bytes(a, v) : ws_bytes(a, v);
+  *bytes = scratch_full(a).bytes;
   return LVSA_OK;
 }
