@@ -76,14 +76,21 @@ class BlockSparseAttentionWrapper:
         indptr = indptr.to(device)
         indices = indices.to(device)
         n_blocks_k = N // C
-        self._bitmap, status = hip_ops.csr_to_bitmap(indptr, indices, n_blocks_k)
+        self._bitmap, self._status = hip_ops.csr_to_bitmap(indptr, indices, n_blocks_k)
+        self._status_checked = False
+        self._status_host = None
+        if not torch.cuda.is_current_stream_capturing():
+            # copied back while the block plan is built, so that the first
+            # run() waits for neither
+            self._status_host = torch.empty(1, dtype=torch.int32, pin_memory=True)
+            self._status_host.copy_(self._status[:1], non_blocking=True)
+            self._status_ready = torch.cuda.Event()
+            self._status_ready.record(torch.cuda.current_stream(device))
         self._plans = {}
         self._plan_args = dict(n_q=M, n_k=N, R=R, Cf=C, max_row_frames=max(1, n_blocks_k), device=device)
         self._plan = self._plan_for(head_dim, _torch_dtype(q_data_type))
         self._shape = (M, N, num_qo_heads, num_kv_heads, head_dim)
         self._scale = sm_scale
-        self._status = status
-        self._status_checked = False
 
     def _plan_for(self, head_dim: int, dtype: Optional[torch.dtype]) -> hip_ops.BlockPlan:
         # one block plan per tile height: fp32 runs 128-row tiles
@@ -101,7 +108,12 @@ class BlockSparseAttentionWrapper:
         # stream capture (the plan is reused by every run()).
         if self._status_checked or torch.cuda.is_current_stream_capturing():
             return
-        if int(self._status[0].item()):
+        if self._status_host is None:
+            bad = int(self._status[0].item())
+        else:
+            self._status_ready.synchronize()
+            bad = int(self._status_host[0])
+        if bad:
             raise ValueError("indices hold column ids outside [0, N/C)")
         self._status_checked = True
 

@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes as C
 import math
 import os
+import struct
 from dataclasses import dataclass
 from typing import Optional, Sequence, Tuple
 
@@ -121,7 +122,25 @@ def dual_wide_ok(plan: "BlockPlan", *srcs: Optional[torch.Tensor]) -> bool:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def _call(device: torch.device, name: str, *args) -> None:
+    """One C entry point on ``device``'s current stream (its last argument)."""
+    fn = getattr(capi.lib(), name)
+    if torch.cuda.current_device() == device.index:
+        rc = fn(*args, _stream(device))
+    else:
+        with torch.cuda.device(device):
+            rc = fn(*args, _stream(device))
+    if rc:
+        capi.check(name, rc)
+
+
+def _indexed(device: torch.device) -> torch.device:
+    """``device`` with its index filled in (the current GPU's for plain "cuda")."""
+    device = torch.device(device)
+    return torch.device("cuda", torch.cuda.current_device()) if device.index is None else device
 
 
 def _require_device(t: torch.Tensor, name: str) -> None:
@@ -130,10 +149,6 @@ def _require_device(t: torch.Tensor, name: str) -> None:
             f"{name} must be a GPU (HIP) tensor: the LVSA MI355X backend has no CPU path "
             f"(got {getattr(t, 'device', type(t))})"
         )
-
-
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
 
 
 # ───────────────────────────── mask builder ────────────────────────────────
@@ -191,10 +206,8 @@ def auto_kfi(T: int, W: int, n_first: int, reference_frames: int = 21, sparsity_
             raise RuntimeError("lvsa_auto_kfi runs on the GPU only")
         out = torch.empty(1, dtype=torch.int32, device=device)
     _require_device(out, "kfi output")
-    with torch.cuda.device(out.device):
-        capi.check("lvsa_auto_kfi", capi.lib().lvsa_auto_kfi(
-            int(T), int(W), int(n_first), int(reference_frames), float(sparsity_scale), out.data_ptr(),
-            _stream(out.device)))
+    _call(out.device, "lvsa_auto_kfi", int(T), int(W), int(n_first), int(reference_frames), float(sparsity_scale),
+          out.data_ptr())
     return out
 
 
@@ -208,6 +221,7 @@ def mask_build(p: capi.MaskParams, device: torch.device) -> DeviceMask:
     device = torch.device(device)
     if device.type != "cuda":
         raise RuntimeError("lvsa_mask_build runs on the GPU only")
+    device = _indexed(device)
     s = mask_sizes(p)
     i32 = dict(dtype=torch.int32, device=device)
     T = p.T
@@ -228,8 +242,7 @@ def mask_build(p: capi.MaskParams, device: torch.device) -> DeviceMask:
         dm.global_frames.data_ptr(), dm.window_bounds.data_ptr(), dm.rel_full.data_ptr(),
         dm.rel_window.data_ptr(), dm.info.data_ptr(),
     )
-    with torch.cuda.device(device):
-        capi.check("lvsa_mask_build", capi.lib().lvsa_mask_build(C.byref(p), C.byref(out), _stream(device)))
+    _call(device, "lvsa_mask_build", C.byref(p), C.byref(out))
     return dm
 
 
@@ -319,7 +332,7 @@ def plan_build(rel: Optional[torch.Tensor], *, n_q: int, n_k: int, n_x: int = 0,
         rel = rel.contiguous()
     if device is None or torch.device(device).type != "cuda":
         raise RuntimeError("lvsa_plan_build runs on the GPU only")
-    device = torch.device(device)
+    device = _indexed(device)
     if block_q is None:
         block_q = attn_block_q(head_dim, dtype, video_rows=n_q > 0)
     p = capi.PlanParams()
@@ -336,30 +349,42 @@ def plan_build(rel: Optional[torch.Tensor], *, n_q: int, n_k: int, n_x: int = 0,
     indptr = torch.empty(sz.n_tiles + 1, **i32)
     entries = torch.empty(max(sz.max_entries, 1), 2, **i32)
     status = torch.empty(max(sz.workspace_bytes // 4, 4), **i32)
-    with torch.cuda.device(device):
-        capi.check("lvsa_plan_build", capi.lib().lvsa_plan_build(
-            C.byref(p), indptr.data_ptr(), entries.data_ptr(), sz.max_entries,
-            status.data_ptr(), status.numel() * 4, _stream(device)))
-    return BlockPlan(indptr, entries, status, sz.n_tiles, sz.n_video_tiles, p, rel, max_row_frames)
+    _call(device, "lvsa_plan_build", C.byref(p), indptr.data_ptr(), entries.data_ptr(), sz.max_entries,
+          status.data_ptr(), status.numel() * 4)
+    plan = BlockPlan(indptr, entries, status, sz.n_tiles, sz.n_video_tiles, p, rel, max_row_frames)
+    # A tile lists a key block at most once, so a capacity of every block per
+    # tile cannot overflow and verify() has nothing to read back.
+    plan._verified = sz.max_entries >= sz.n_tiles * (-(-n_k // block_k) + -(-n_x // block_k))
+    return plan
 
 
 # ─────────────────────────── attention forward ─────────────────────────────
 
 
-def _prep(t: torch.Tensor, name: str, dtype: torch.dtype) -> torch.Tensor:
-    _require_device(t, name)
+def _rows(t: torch.Tensor, name: str, dtype: torch.dtype):
+    """A ``[B, S, H, D]`` tensor the kernels can read (16-byte rows and row
+    strides; other layouts are repacked on the device), its address and its
+    first three strides."""
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+        _require_device(t, name)
     if t.dim() != 4:
         raise ValueError(f"{name} must be [B, S, H, D], got shape {tuple(t.shape)}")
     if t.dtype != dtype:
         raise TypeError(f"{name} has dtype {t.dtype}, expected {dtype}")
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((s * t.element_size()) % 16 == 0
-                                                              for s in t.stride()[:3])
-    # The kernel reads 16-byte row chunks; other layouts are repacked on the device.
-    return t if ok else t.clone(memory_format=torch.contiguous_format)
+    s0, s1, s2, s3 = t.stride()
+    ptr = t.data_ptr()
+    if s3 != 1 or (ptr | ((s0 | s1 | s2) * t.element_size())) & 15:
+        t = t.clone(memory_format=torch.contiguous_format)
+        s0, s1, s2, _ = t.stride()
+        ptr = t.data_ptr()
+    return t, ptr, s0, s1, s2
 
 
-def _str3(t: Optional[torch.Tensor]):
-    return capi._Str3(*(t.stride()[:3] if t is not None else (0, 0, 0)))
+# lvsa_attn_args as one struct.pack_into: setting its 60 fields one by one
+# through ctypes was a fifth of a small call's host time.
+_ATTN_ARGS = struct.Struct("@10P24q8ifii2P2iP4i2qiPq")
+assert _ATTN_ARGS.size == C.sizeof(capi.AttnArgs)
+_ABSENT = (0, 0, 0)
 
 
 @dataclass
@@ -384,28 +409,31 @@ def attn_args(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan
     dtype = q.dtype
     if dtype not in _DTYPES:
         raise TypeError(f"unsupported dtype {dtype}: bf16, fp16 or fp32 inputs")
-    q = _prep(q, "query", dtype)
-    k = _prep(k, "key", dtype)
-    v = _prep(v, "value", dtype)
+    q, q_ptr, *q_str = _rows(q, "query", dtype)
+    k, k_ptr, *k_str = _rows(k, "key", dtype)
+    v, v_ptr, *v_str = _rows(v, "value", dtype)
     B, n_q, H, D = q.shape
-    Hkv = k.shape[2]
+    kshape = k.shape
+    _, n_k, Hkv, _ = kshape
     kernel_head_dim(D)  # raises for an unsupported head size
-    if k.shape[0] != B or k.shape[3] != D or v.shape != k.shape:
+    if kshape[0] != B or kshape[3] != D or v.shape != kshape:
         raise ValueError(f"key/value shapes {tuple(k.shape)} / {tuple(v.shape)} do not match query {tuple(q.shape)}")
     if H % Hkv:
         raise ValueError(f"num heads {H} must be a multiple of kv heads {Hkv}")
-    n_x = 0
+    n_x = kx_ptr = vx_ptr = 0
+    kx_str = vx_str = _ABSENT
     if kx is not None and kx.shape[1] > 0:
-        kx = _prep(kx, "extra key", dtype)
-        vx = _prep(vx, "extra value", dtype)
+        kx, kx_ptr, *kx_str = _rows(kx, "extra key", dtype)
+        vx, vx_ptr, *vx_str = _rows(vx, "extra value", dtype)
         if kx.shape[0] != B or kx.shape[2] != Hkv or kx.shape[3] != D or vx.shape != kx.shape:
             raise ValueError("extra key/value shape mismatch")
         n_x = kx.shape[1]
     else:
         kx = vx = None
-    n_tq = 0
+    n_tq = qt_ptr = 0
+    qt_str = _ABSENT
     if qt is not None and qt.shape[1] > 0:
-        qt = _prep(qt, "text query", dtype)
+        qt, qt_ptr, *qt_str = _rows(qt, "text query", dtype)
         if qt.shape[0] != B or qt.shape[2] != H or qt.shape[3] != D:
             raise ValueError("text query shape mismatch")
         n_tq = qt.shape[1]
@@ -419,10 +447,10 @@ def attn_args(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan
     if plan.block_k != capi.ATTN_BLOCK_K:
         raise ValueError(f"plan built with block_k={plan.block_k}; the attention kernels walk key blocks of "
                          f"{capi.ATTN_BLOCK_K} rows")
-    if (pp.n_q, pp.n_k, pp.n_x, pp.n_tq) != (n_q, k.shape[1], n_x, n_tq):
+    if (pp.n_q, pp.n_k, pp.n_x, pp.n_tq) != (n_q, n_k, n_x, n_tq):
         raise ValueError(
             f"plan built for (n_q, n_k, n_x, n_tq)={(pp.n_q, pp.n_k, pp.n_x, pp.n_tq)}, "
-            f"called with {(n_q, k.shape[1], n_x, n_tq)}")
+            f"called with {(n_q, n_k, n_x, n_tq)}")
     if out is None:
         out = torch.empty_like(q, memory_format=torch.contiguous_format)
     if qt is not None and out_t is None:
@@ -430,25 +458,17 @@ def attn_args(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan
     lse = torch.empty(B, H, n_q, dtype=torch.float32, device=q.device) if return_lse else None
     lse_t = (torch.empty(B, H, n_tq, dtype=torch.float32, device=q.device)
              if (return_lse and qt is not None) else None)
+    o_str = out.stride()
+    ot_ptr, ot_str = (0, _ABSENT) if out_t is None else (out_t.data_ptr(), out_t.stride()[:3])
     a = capi.AttnArgs()
-    a.q, a.k, a.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
-    a.kx, a.vx, a.qt = _ptr(kx), _ptr(vx), _ptr(qt)
-    a.o, a.ot = out.data_ptr(), _ptr(out_t)
-    a.lse, a.lse_t = _ptr(lse), _ptr(lse_t)
-    a.q_str, a.k_str, a.v_str = _str3(q), _str3(k), _str3(v)
-    a.kx_str, a.vx_str, a.qt_str = _str3(kx), _str3(vx), _str3(qt)
-    a.o_str, a.ot_str = _str3(out), _str3(out_t)
-    a.B, a.H, a.Hkv, a.D = B, H, Hkv, D
-    a.n_q, a.n_k, a.n_x, a.n_tq = n_q, k.shape[1], n_x, n_tq
-    a.scale = float(scale) if scale is not None else 1.0 / math.sqrt(D)
-    a.dtype = _DTYPES[dtype]
-    a.block_q = plan.block_q
-    a.tile_indptr, a.entries = plan.tile_indptr.data_ptr(), plan.entries.data_ptr()
-    a.n_tiles, a.n_video_tiles = plan.n_tiles, plan.n_video_tiles
-    a.rel = pp.rel
-    a.words, a.R, a.C, a.q_frame0 = pp.words, pp.R, pp.C, pp.q_frame0
-    a.q_tok0, a.k_tok0 = pp.q_tok0, pp.k_tok0
-    a.rel_rows = pp.rel_rows
+    _ATTN_ARGS.pack_into(
+        a, 0, q_ptr, k_ptr, v_ptr, kx_ptr, vx_ptr, qt_ptr, out.data_ptr(), ot_ptr,
+        0 if lse is None else lse.data_ptr(), 0 if lse_t is None else lse_t.data_ptr(),
+        *q_str, *k_str, *v_str, *kx_str, *vx_str, *qt_str, o_str[0], o_str[1], o_str[2], *ot_str,
+        B, H, Hkv, D, n_q, n_k, n_x, n_tq,
+        float(scale) if scale is not None else 1.0 / math.sqrt(D), _DTYPES[dtype], pp.block_q,
+        plan.tile_indptr.data_ptr(), plan.entries.data_ptr(), plan.n_tiles, plan.n_video_tiles,
+        pp.rel or 0, pp.words, pp.R, pp.C, pp.q_frame0, pp.q_tok0, pp.k_tok0, pp.rel_rows, 0, 0)
     plan.verify()
     return AttnCall(a, out, out_t, lse, lse_t, (q, k, v, kx, vx, qt, plan))
 
@@ -471,15 +491,22 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan,
     call = attn_args(q, k, v, plan, kx=kx, vx=vx, qt=qt, scale=scale, return_lse=return_lse, out=out,
                      out_t=out_t)
     a = call.args
-    ws_bytes = C.c_int64(0)
-    capi.check("lvsa_attn_workspace_query", capi.lib().lvsa_attn_workspace_query(C.byref(a), C.byref(ws_bytes)))
-    ws = None
-    if ws_bytes.value > 0 and scratch:
-        # work-queue counters (zeroed by the call) and the text-split partials
-        ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=call.out.device)
-        a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes.value
-    with torch.cuda.device(call.out.device):
-        capi.check("lvsa_attn_fwd", capi.lib().lvsa_attn_fwd(C.byref(a), _stream(call.out.device)))
+    device = call.out.device
+    if scratch:
+        ws_bytes = C.c_int64(0)
+        # on the call's GPU: the scratch follows its compute units
+        if torch.cuda.current_device() == device.index:
+            rc = capi.lib().lvsa_attn_workspace_query(C.byref(a), C.byref(ws_bytes))
+        else:
+            with torch.cuda.device(device):
+                rc = capi.lib().lvsa_attn_workspace_query(C.byref(a), C.byref(ws_bytes))
+        if rc:
+            capi.check("lvsa_attn_workspace_query", rc)
+        if ws_bytes.value > 0:
+            # work-queue counters (zeroed by the call), partials, fp32 pairs
+            ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=device)
+            a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes.value
+    _call(device, "lvsa_attn_fwd", C.byref(a))
     return call.out, call.out_t, call.lse, call.lse_t
 
 
@@ -504,10 +531,8 @@ def gather_frames(src: torch.Tensor, frames: torch.Tensor, P: int) -> torch.Tens
         raise TypeError(f"unsupported element size {es}")
     sstr = (C.c_int64 * 3)(*src.stride()[:3])
     dstr = (C.c_int64 * 3)(*dst.stride()[:3])
-    with torch.cuda.device(src.device):
-        capi.check("lvsa_gather_frames", capi.lib().lvsa_gather_frames(
-            src.data_ptr(), sstr, dst.data_ptr(), dstr, frames.data_ptr(), n, P, B, H, D, es,
-            _stream(src.device)))
+    _call(src.device, "lvsa_gather_frames", src.data_ptr(), sstr, dst.data_ptr(), dstr, frames.data_ptr(), n, P, B, H,
+          D, es)
     return dst
 
 
@@ -524,8 +549,6 @@ def csr_to_bitmap(indptr: torch.Tensor, indices: torch.Tensor, n_cols: int) -> T
     words = max(1, -(-n_cols // 32))
     bitmap = torch.empty(max(n_rows, 1), words, dtype=torch.int32, device=device)
     status = torch.empty(4, dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
-        capi.check("lvsa_csr_to_bitmap", capi.lib().lvsa_csr_to_bitmap(
-            indptr.data_ptr(), indices.data_ptr() if indices.numel() else None, n_rows, n_cols,
-            bitmap.data_ptr(), words, status.data_ptr(), _stream(device)))
+    _call(device, "lvsa_csr_to_bitmap", indptr.data_ptr(), indices.data_ptr() if indices.numel() else None, n_rows,
+          n_cols, bitmap.data_ptr(), words, status.data_ptr())
     return bitmap[:n_rows], status

@@ -108,6 +108,33 @@ def get_window_bounds(
     return adaptive_window_bounds(f, W, T)
 
 
+def _all_window_bounds(T: int, W: int, expand: bool, is_global: bytearray) -> List[Tuple[int, int]]:
+    """:func:`get_window_bounds` of every frame, counting the non-global
+    frames of a window by prefix sums."""
+    if W == 0:
+        return [(f, f - 1) for f in range(T)]
+    upto = [0]
+    for g in is_global:
+        upto.append(upto[-1] + 1 - g)
+    target = min(2 * W + 1, upto[T]) if expand else 0
+    bounds = []
+    for f in range(T):
+        lo, hi = adaptive_window_bounds(f, W, T)
+        missing = target - (upto[hi + 1] - upto[lo])
+        if missing > 0:
+            for x in _outward(lo, hi, T):
+                if x < lo:
+                    lo = x
+                else:
+                    hi = x
+                if not is_global[x]:
+                    missing -= 1
+                    if missing == 0:
+                        break
+        bounds.append((lo, hi))
+    return bounds
+
+
 def compute_boundary_guard_frames(
     total_frames: int,
     local_seq: int,
@@ -242,11 +269,11 @@ class _DeviceState:
 
     def join(self, device: torch.device) -> None:
         """Order the current stream of ``device`` after every build so far."""
-        if self.ready is None or torch.cuda.is_current_stream_capturing():
+        if self.ready is None or self.joined.get(hip_ops._stream(device), 0) == self.version:
+            return
+        if torch.cuda.is_current_stream_capturing():
             return
         s = torch.cuda.current_stream(device)
-        if self.joined.get(s.cuda_stream, 0) == self.version:
-            return
         s.wait_event(self.ready)
         for t in self._tensors():
             t.record_stream(s)
@@ -394,46 +421,44 @@ class LVSAMetadata:
         G = sorted(set(compute_global_indices(T, n_first_frames, kfi, keyframe_offset)) | set(guards))
         Gs = set(G)
         nG = len(G)
-        bounds = [get_window_bounds(f, W, T, expand_window, Gs, nG) for f in range(T)]
-
-        def on_rank(fr: int) -> Tuple[int, int]:
-            return max(fr * P, gts) - gts, min((fr + 1) * P, gts + local_seq) - gts
+        is_global = bytearray(T)
+        for g in G:
+            is_global[g] = 1
+        bounds = _all_window_bounds(T, W, expand_window, is_global)
 
         first, last = gts // P, (gts + local_seq - 1) // P
-        local_frames = [(fr, *on_rank(fr)) for fr in range(first, last + 1)]
-        window_ctx: Dict[int, List[Tuple[int, int]]] = {}
-        for fr, _, _ in local_frames:
-            lo, hi = bounds[fr]
-            window_ctx[fr] = [on_rank(wf) for wf in range(lo, hi + 1)
-                              if wf not in Gs and on_rank(wf)[0] < on_rank(wf)[1]]
-
-        attended_rows = []
-        for fr in range(first, last + 1):
-            lo, hi = bounds[fr]
-            attended_rows.append(sorted(Gs.union(range(lo, hi + 1))))
-        attended_C = max(len(r) for r in attended_rows)
-
+        # every frame's rows on this rank (empty or reversed off it)
+        on_rank = [(max(fr * P, gts) - gts, min((fr + 1) * P, gts + local_seq) - gts) for fr in range(T)]
+        local_frames = [(fr, *on_rank[fr]) for fr in range(first, last + 1)]
         # CSR geometry: MB rows from the first local frame; compact ids number
         # the union of all rows (lvsa/sparse_attention.py:550-635).
         MB = -(-local_seq // P)
-        union: Set[int] = set()
+        window_ctx: Dict[int, List[Tuple[int, int]]] = {}
+        attended_rows = []
+        union: Set[int] = set(Gs)
         nnz = 0
         row_max = 0
-        for qi in range(MB):
-            fr = first + qi
+        for fr in range(first, last + 1):
             lo, hi = bounds[fr]
-            row = Gs | {wf for wf in range(lo, hi + 1) if wf not in Gs and on_rank(wf)[0] < on_rank(wf)[1]}
-            union |= row
-            nnz += len(row)
-            row_max = max(row_max, len(row))
+            window = [wf for wf in range(lo, hi + 1) if not is_global[wf]]
+            here = [wf for wf in window if first <= wf <= last]
+            window_ctx[fr] = [on_rank[wf] for wf in here]
+            attended_rows.append(sorted(G + window))
+            if fr < first + MB:
+                union.update(here)
+                nnz += nG + len(here)
+                row_max = max(row_max, nG + len(here))
+        attended_C = max(len(r) for r in attended_rows)
         compact = sorted(union)
-        gpos = {g: i for i, g in enumerate(G)}
-        gcop = [(gpos[fr] * P, ci * P) for ci, fr in enumerate(compact) if fr in Gs]
-        lcop = [(fr * P - gts, ci * P) for ci, fr in enumerate(compact) if fr not in Gs]
+        gcop = []
+        lcop = []
+        for ci, fr in enumerate(compact):
+            if is_global[fr]:
+                gcop.append((len(gcop) * P, ci * P))
+            else:
+                lcop.append((fr * P - gts, ci * P))
 
-        gmask = torch.zeros(T, dtype=torch.int8)
-        if G:
-            gmask[torch.tensor(G)] = 1
+        gmask = torch.tensor(list(is_global), dtype=torch.int8)
         return cls(
             total_latent_frames=T, num_patches=P, window_size=W, n_first_frames=n_first_frames,
             key_frame_interval=kfi, expand_window=expand_window, rank=rank, world=world,
@@ -557,6 +582,9 @@ class LVSAMetadata:
             plan = hip_ops.plan_build(
                 st.mask.rel_window, n_q=n_q, n_k=n_k, n_x=n_extra, R=P, Cf=P, q_tok0=gts, k_tok0=gts,
                 q_frame0=gts // P, max_row_frames=max(1, 2 * self.window_size + 1), block_q=block_q)
+            # rel_window holds at most 2W + 1 frames per row and every other tile list is
+            # bounded by its blocks, so the capacity is exact: nothing to read back
+            plan._verified = True
             st.plans[key] = plan
             st.built(st.mask.info.device)
         return plan
@@ -576,6 +604,8 @@ class LVSAMetadata:
             plan = hip_ops.plan_build(
                 st.mask.rel_full, n_q=n_q, n_k=n_k, n_x=n_text_k, n_tq=n_text_q, R=P, Cf=P,
                 max_row_frames=max(1, self.max_row_frames), block_q=block_q)
+            # max_row_frames is the longest row of this pattern: the capacity is exact
+            plan._verified = True
             st.plans[key] = plan
             st.built(st.mask.info.device)
         return plan
