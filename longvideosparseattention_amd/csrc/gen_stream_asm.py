@@ -74,6 +74,11 @@ Register map (VGPRs; the kernel's operands pin them), D = 128 (D = 64):
   rows, K and V in two-stage rings of their own: block j copies K(j+1) and V(j)
   and waits for all copies at the next barrier, K and V tracking their key
   sources separately (SWITCHK / SWITCHV).  218 (194) VGPRs.
+  The half map (D = 128 and 64, Layout nw = 4, dual = False) is the 8-wave
+  map's wave, registers and softmax in work-groups of 4 waves and 128 query
+  rows, two per CU: D = 128 with the wide map's two-stage K and V rings and
+  copy schedule (O in VGPRs, one lane offset per tensor), D = 64 with the
+  four-stage ring.
   D = 192 by default runs the dual-wide map (Layout nw = 4, dual = True): the
   wide map's copies, rings and AGPR-held O with the dual map's two 32-row
   halves per wave (256-row tiles): O of half r in a[96 r : 96 r + 95], Q of
@@ -115,15 +120,18 @@ class Layout:
     map: 64 rows per wave in two 32-row halves (NR = 2), the compact map's
     slots and temporaries, at most 256 VGPRs (two waves per SIMD).  `dual`
     with D = 192 is the dual-wide map: the wide map with two 32-row halves
-    per wave, half 1's Q in the AGPRs after O (QA)."""
+    per wave, half 1's Q in the AGPRs after O (QA).  `nw` = 4 with D = 128, or
+    with D = 64 and `dual` False, is the half map: 128-row work-groups of the
+    8-wave map's waves."""
 
     def __init__(self, D: int, nw: int = 8, rs: bool = False, dual: bool | None = None):
         dual = (nw == 4 and D == 64) if dual is None else dual
         assert (D, nw, dual) in ((64, 8, False), (96, 8, False), (128, 8, False), (64, 12, False), (192, 4, False),
-                                 (256, 4, False), (64, 4, True), (192, 4, True))
+                                 (256, 4, False), (64, 4, True), (192, 4, True), (128, 4, False), (64, 4, False))
         self.D = D
         self.nw = nw
         self.wide = nw == 4 and D >= 192
+        self.ring2 = nw == 4 and D >= 128  # two-stage rings: block j copies K(j+1) and V(j)
         self.dual = dual                  # two 32-row halves per wave (64 rows)
         self.NR = 2 if self.dual else 1   # 32-row halves per wave
         assert rs or not self.dual
@@ -138,7 +146,7 @@ class Layout:
         # reading out of range (zeros) and never read
         self.RB = 2 * {96: 128, 192: 256}.get(D, D)   # bytes per K/V row in LDS
         self.TILE = 64 * self.RB          # one K or V block
-        self.NST = 2 if self.wide else 4  # LDS stages per tensor
+        self.NST = 2 if self.ring2 else 4  # LDS stages per tensor
         self.VBASE = self.NST * self.TILE  # V stages follow the K stages
         self.NCP = self.TILE // 1024 // (4 if nw == 4 else 8)   # 1 KiB copies per tensor, wave and block
         # rows between a wave's consecutive copies of one tensor (8 or 4 waves x 1 KiB)
@@ -608,7 +616,7 @@ class Gen:
             f"s_mov_b32 {sr(rs + 3)}, 0x20000",
             f"s_lshl_b32 {sr(st16)}, {sr(st)}, 4",
             f"v_mad_u32_u24 {vr(off)}, {vr(L.DMAROW)}, {sr(st)}, {vr(L.C16)}",
-            f"v_mad_u32_u24 {vr(off + 1)}, {vr(L.DMAROW + 2)}, {sr(st)}, {vr(L.C16 + 2)}",
+            *([f"v_mad_u32_u24 {vr(off + 1)}, {vr(L.DMAROW + 2)}, {sr(st)}, {vr(L.C16 + 2)}"] if L.wide else []),
             "s_nop 1",
             f"s_setpc_b64 {sr(S_RET, 2)}",
         ]
@@ -653,6 +661,11 @@ class Gen:
             lds = (L.VBASE if v else 0) + stage * L.TILE + ii * 4096
             so = sr((S_SOVW if v else S_SOK) + (ii >> 1))
             lane = (L.DV if v else L.DK) + (ii & 1)
+        elif L.ring2:
+            # copy ii of wave w: LDS KiB 4*ii + w, rows 16*ii + 4*w + lane/16
+            lds = (L.VBASE if v else 0) + stage * L.TILE + ii * 4096
+            so = sr((S_SOVW if v else S_SOK) + ii)
+            lane = L.DV if v else L.DK
         else:
             lds = (L.VBASE if v else 0) + stage * L.TILE + ii * L.CPROWS * L.RB
             so = sr((S_SOV if v else S_SOK) + ii)
@@ -773,10 +786,10 @@ class Gen:
         L = self.L
         vst, cst = (stage + 3) & 3, (stage + 2) & 3       # entry slots of blocks j-1 and j+2
         # LDS stages of K(j) and V(j-1) (wide: two-stage rings of their own)
-        kld, vld = (stage & 1, (stage + 1) & 1) if L.wide else (stage, vst)
+        kld, vld = (stage & 1, (stage + 1) & 1) if L.ring2 else (stage, vst)
         site = f"I{stage}"
         M = 2 * L.NQK                     # MFMAs per sub-iteration (QK and PV interleaved)
-        self.e(f"; ── block j, K stage {stage}", f"s_waitcnt vmcnt({0 if L.wide else 2 * L.NCP})",
+        self.e(f"; ── block j, K stage {stage}", f"s_waitcnt vmcnt({0 if L.ring2 else 2 * L.NCP})",
                "s_barrier", "s_waitcnt lgkmcnt(0)")
         mf = []
         half_q = L.NQK // 2               # QK k-steps per 16-key PV step
@@ -794,7 +807,7 @@ class Gen:
                 mf += qks[c:c + step] + rest[c:c + step]
             mf += rest[L.NQK:]
         assert mf[:len(self.lead_pv(vst))] == self.lead_pv(vst)
-        if L.wide:
+        if L.ring2:
             # K(j+1) into the K stage K(j-1) left, V(j) into the V stage V(j-2) left
             fill = {0: self.decode_wide(S_ENT + 2 * ((stage + 1) & 3), site, False) +
                     self.decode_wide(S_ENT + 2 * stage, site, True)}
@@ -806,7 +819,8 @@ class Gen:
             if L.dual:
                 at_copy = tuple(self.dual_copy[0] + self.dual_copy[1] * k for k in range(2 * L.NCP))
             else:
-                at_copy = {8: (6, 10, 22, 26), 6: (4, 8, 16, 20), 4: (5, 13)}[L.NQK]
+                at_copy = {8: (6, 10, 22, 26), 6: (4, 8, 16, 20), 4: (5, 13) if L.NCP == 1 else (2, 5, 9, 13)}[L.NQK]
+                assert len(at_copy) == 2 * L.NCP
             for k, at in enumerate(at_copy):
                 self.place_copy(fill, at, cst, k)
         u, ue = self.u, self.ue
@@ -829,9 +843,9 @@ class Gen:
     def first_iteration(self) -> None:
         """Block 0: QK of its two sub-blocks, softmax of sub-block 0, copies of block 2."""
         L = self.L
-        self.e("; ── block 0", f"s_waitcnt vmcnt({0 if L.wide else 2 * L.NCP})", "s_barrier", "s_waitcnt lgkmcnt(0)")
+        self.e("; ── block 0", f"s_waitcnt vmcnt({0 if L.ring2 else 2 * L.NCP})", "s_barrier", "s_waitcnt lgkmcnt(0)")
         mf = [("qk", 0, 0, c, L.SA) for c in range(L.NQK)] + [("qk", 0, 1, c, L.SB) for c in range(L.NQK)]
-        if L.wide:
+        if L.ring2:
             # K(1) into K stage 1, V(0) into V stage 0, spread over the block's QK MFMAs
             fill = {0: self.decode_wide(S_ENT + 2, "F", False) + self.decode_wide(S_ENT, "F", True)}
             n = len(mf)
@@ -852,8 +866,8 @@ class Gen:
         """After block n-1 (in `stage`): softmax of sub-block 2n-1, PV of block n-1."""
         L = self.L
         self.e(f"{lbl(f'DRAIN{stage}')}:")
-        vld = stage & 1 if L.wide else stage
-        if L.wide:
+        vld = stage & 1 if L.ring2 else stage
+        if L.ring2:
             # V(n-1) was copied during block n-1: wait for every wave's copies
             self.e("s_waitcnt vmcnt(0)", "s_barrier")
         nh = L.NQK                        # PV MFMAs per half: 2 16-key steps x NDT d-tiles
@@ -883,7 +897,7 @@ class Gen:
           f"s_mov_b32 {sr(S_J)}, 0",
           f"s_mov_b32 {sr(S_CUR)}, 2",
           "s_waitcnt lgkmcnt(0)")
-        if L.wide:
+        if L.ring2:
             # K(0) into K stage 0; V(0) and K(1) follow in block 0
             e(f"s_mov_b32 {sr(S_CURV)}, 2")
             e(*self.decode_wide(S_ENT, "S0", False))
@@ -905,7 +919,7 @@ class Gen:
             self.drain(stage)
         e(*self.stubs)
         e(*self.rare_routine(L.SA, L.PA, "RARE_A"), *self.rare_routine(L.SB, L.PB, "RARE_B"))
-        e(*(self.switch_wide(False) + self.switch_wide(True) if L.wide else self.switch_routine()))
+        e(*(self.switch_wide(False) + self.switch_wide(True) if L.ring2 else self.switch_routine()))
         e(*self.mask_routine(L.SA, "MASK_A"), *self.mask_routine(L.SB, "MASK_B"))
         e(f"{lbl('END')}:")
         return self.lines
@@ -914,12 +928,15 @@ class Gen:
 # (head size, waves, two 32-row halves per wave): the dual map of D = 64 and
 # the dual-wide map of D = 192 run 64 rows per wave
 MAPS = ((128, 8, False), (96, 8, False), (64, 8, False), (64, 12, False), (64, 4, True), (256, 4, False),
-        (192, 4, False), (192, 4, True))
+        (192, 4, False), (192, 4, True), (128, 4, False), (64, 4, False))
 
 
 def map_key(D: int, nw: int, dual: bool) -> tuple:
-    """PRODUCT_MAP / per-map option key: (D, nw), or (D, nw, "dual") for the
-    dual-wide map (the one (D, nw) pair with two maps)."""
+    """PRODUCT_MAP / per-map option key: (D, nw); (D, nw, "dual") for the
+    dual-wide map and (64, 4, "half") for the half map of D = 64, whose (D, nw)
+    pairs have two maps."""
+    if (D, nw, dual) == (64, 4, False):
+        return (D, nw, "half")
     return (D, nw, "dual") if dual and D >= 192 else (D, nw)
 
 
@@ -929,7 +946,8 @@ def map_opts(D: int, nw: int, dual: bool) -> dict:
 
 
 def prefix(D: int, nw: int, dual: bool = False) -> str:
-    return f"LVSA_STREAM{D}" + ("" if nw == 8 else f"W{nw}") + ("D" if dual and D >= 192 else "")
+    half = nw == 4 and D <= 128 and not dual
+    return f"LVSA_STREAM{D}" + ("" if nw == 8 else f"W{nw}") + ("D" if dual and D >= 192 else "H" if half else "")
 
 
 def operands(D: int, nw: int = 8, rs: bool = False, dual: bool | None = None) -> list[str]:
@@ -1023,8 +1041,11 @@ PRODUCT = {128: dict(lead=2, early_load=True, dot_init=True, and_scc=True, copy_
 # or 6, the softmax from slot 3 or 8, no paired LDS waits, copies every MFMA
 # pair and 12 tail wait states all landed between -0.3% and +0.75%, and
 # copies every third MFMA pair +4.4%.
+# The half map of D = 128 opens no block with P V: V of the block before lands
+# with the barrier.
 PRODUCT_MAP = {(64, 12): dict(sm_start=1, tail_nop=8),
-               (64, 4): dict(sm_start=1, tail_nop=8, dual_copy=(6, 8))}
+               (64, 4): dict(sm_start=1, tail_nop=8, dual_copy=(6, 8)),
+               (128, 4): dict(lead=0)}
 
 
 def render(per_d: dict | None = None, **opts) -> str:
@@ -1099,7 +1120,7 @@ def census(D: int, nw: int, dual: bool = False, dt: str = "bf16") -> dict:
 
 def print_census() -> None:
     cols = [(128, 8, False), (96, 8, False), (64, 12, False), (64, 8, False), (64, 4, True), (192, 4, False),
-            (192, 4, True), (256, 4, False)]
+            (192, 4, True), (256, 4, False), (128, 4, False), (64, 4, False)]
     res = {col: census(*col) for col in cols}
     print("| per 32-key sub-block, per wave | " +
           " | ".join(f"D={d}, {n} waves" + (" (64 rows)" if dual else "") for d, n, dual in cols) + " |")

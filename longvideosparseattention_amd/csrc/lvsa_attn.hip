@@ -77,15 +77,16 @@ int text_chunks_least(const lvsa_attn_args* a) {
   return a->dtype == LVSA_FP32 || blocks <= kTextChunkBlocks ? 1 : text_chunks_of(a);
 }
 
-// The video split of a call: `tiles` per queue in `parts` parts each.
+// The video split of a call: `tiles` tiles of `rows` rows per queue in `parts`
+// parts each.
 struct VideoSplit {
-  int tiles = 0, parts = 0;
+  int tiles = 0, parts = 0, rows = 0;
 };
 
 // Partials of the video split (O, then the (running max, row sum) pairs).
 int64_t video_ws_bytes(const lvsa_attn_args* a, VideoSplit v) {
   if (v.tiles <= 0) return 0;
-  return 4 * (video_ws_o_elems(v.tiles, v.parts, a->block_q, a->D) + 2LL * kXcds * v.tiles * v.parts * a->block_q);
+  return 4 * (video_ws_o_elems(v.tiles, v.parts, v.rows, a->D) + 2LL * kXcds * v.tiles * v.parts * v.rows);
 }
 
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
@@ -134,22 +135,93 @@ __global__ __launch_bounds__(64) void queue_reset_kernel(uint32_t* q) {
   if (threadIdx.x < 8) q[threadIdx.x * (kQueueStride / 4)] = 0u;
 }
 
-// Whether a 16-bit head size 64 plan of 256-row tiles runs the dual map
-// (LVSA_D64_WAVES=8 selects 8 waves of 32 rows instead, for comparisons).
-bool dual_map(const lvsa_attn_args* a) {
+// Whether the short last key block of the frame-structured source crosses a
+// frame boundary: it holds the t = n_k - 64 floor((n_k - 1) / 64) < 64 last
+// keys, tokens [k_tok0 + n_k - t, k_tok0 + n_k), and the last boundary at or
+// below its end lies e = (k_tok0 + n_k) mod C tokens before that end.  The
+// plan builder describes such a block as "generic" (two frames and the rows
+// past the end of the source).
+bool stream_tail_crosses_frame(int64_t n_q, int64_t n_k, int64_t k_tok0, int C) {
+  if (n_q == 0 || n_k <= 0 || C <= 0) return false;
+  const int64_t t = n_k - kBN * ((n_k - 1) / kBN);
+  const int64_t e = (k_tok0 + n_k) % C;
+  return t < kBN && e > 0 && e < t;
+}
+
+// Which kernel a call runs, and on tiles of how many rows.
+struct Route {
+  bool stream, dual, half;   // the single-stream kernel, and its map
+  int shift;                 // two tiles per plan tile
+  int rows;                  // query rows per tile
+  int per_cu;                // work-groups per CU
+  bool src32, tail_cross;
+};
+Route route_of(const lvsa_attn_args* a) {
+  const bool fp32 = a->dtype == LVSA_FP32;
+  const int R = a->R > 0 ? a->R : 1, C = a->C > 0 ? a->C : 1;
+  Route r{false, false, false, 0, a->block_q, 1, false, false};
+  // The single-stream kernel (every 16-bit head size) serves plans without
+  // generic descriptors: 256-row tiles touch at most two query frames when
+  // frames have >= 255 rows (128-row tiles: 127), and 64-key blocks (even
+  // short last ones) at most two key frames when frames have >= 64 keys.
+  // LVSA_ATTN_KERNEL=pp selects the compiler-built kernels instead
+  // (comparisons).
+  const char* kenv = getenv("LVSA_ATTN_KERNEL");
+  const bool force_pp = kenv != nullptr && strcmp(kenv, "pp") == 0;
+  // Its copies address a whole key source through one buffer resource with
+  // 32-bit byte offsets; at D = 96 and 192 the lanes of the unused chunks of
+  // a row add 0x7FFF0000 to theirs, which must lie past the end of the
+  // source (zeros, no access) or inside it (a harmless read into chunks no
+  // read touches): the rows must stay below 2^31 bytes there.
+  const int64_t lim = (a->D == 96 || a->D == 192) ? (1LL << 31) : (1LL << 32);
+  auto fits32 = [lim](int64_t rows, int64_t row_elems) { return (rows + kBN) * row_elems * 2 < lim; };
+  r.src32 = fits32(a->n_k, a->k_str[1]) && fits32(a->n_k, a->v_str[1]) &&
+            (a->n_x == 0 || (fits32(a->n_x, a->kx_str[1]) && fits32(a->n_x, a->vx_str[1])));
+  // Its lane copy offsets are 24-bit products (row x row stride in bytes).
+  auto fits24 = [](int64_t row_elems) { return row_elems * 2 < (1LL << 24); };
+  const bool str24 = fits24(a->k_str[1]) && fits24(a->v_str[1]) &&
+                     (a->n_x == 0 || (fits24(a->kx_str[1]) && fits24(a->vx_str[1])));
+  // Its loop masks "two-part" descriptors only.  A short last key block of
+  // the frame source that crosses a frame boundary (a source starting
+  // mid-frame, as on a context-parallel shard) has three parts (two frames
+  // and the rows past the end) and is planned "generic".
+  r.tail_cross = stream_tail_crosses_frame(a->n_q, a->n_k, a->k_tok0, C);
+  if (fp32 || force_pp || !r.src32 || !str24 || r.tail_cross) return r;
+  if (a->n_q > 0 && (R < a->block_q - 1 || C < kBN)) return r;
+  // 12-wave tiles of 384 rows (D = 64); 256-row tiles of D <= 128 and, on the
+  // dual-wide map, 192; the wide map's 128-row tiles of D = 192 and 256
+  r.stream = true;
+  if (a->D > 128 || a->block_q == kStream12BM) return r;
+  // D = 64 on 256-row tiles: the dual map (64 rows per wave, 4 waves, two
+  // work-groups per CU); LVSA_D64_WAVES=8 selects 8 waves of 32 rows instead
+  // (comparisons).
   const char* w = getenv("LVSA_D64_WAVES");
-  return a->D == 64 && a->block_q == kPPBM && a->dtype != LVSA_FP32 && !(w && strcmp(w, "8") == 0);
+  const bool waves8 = a->D == 64 && w && strcmp(w, "8") == 0;
+  if (a->block_q == kBM) {
+    r.half = a->D != 96;
+  } else if (a->D != 96 && !waves8) {
+    // A plan of few 256-row tiles runs as twice as many 128-row ones: while
+    // those are at most one per CU at D = 128 (108 tiles: 51 -> 39 us, 124 with
+    // text 151 -> 106; 143 to 176 within -2% to +8%), two at D = 64 (108 tiles:
+    // 42 -> 35 us, 256: 60 -> 52; 336 with text 103 -> 114).
+    const int64_t tiles = (ceil_div(a->n_q, kPPBM) + ceil_div(a->n_tq, kPPBM) * text_chunks_of(a)) * a->H * a->B;
+    r.half = tiles <= (a->D == 128 ? cu_count() / 2 : cu_count());
+    r.shift = r.half ? 1 : 0;
+  }
+  r.dual = a->D == 64 && !r.half && !waves8;
+  if (r.half) r.rows = kBM;
+  if (r.half || r.dual) r.per_cu = 2;
+  return r;
 }
 
 // Work-groups of the call's kernel that run at once.  fp32: one per CU with
 // two key groups for at most that many items (launch_f32).
-int64_t concurrent_groups(const lvsa_attn_args* a, int64_t cus, int64_t vwork) {
+int64_t concurrent_groups(const lvsa_attn_args* a, const Route& r, int64_t cus, int64_t vwork) {
   if (a->dtype == LVSA_FP32) {
-    const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_of(a) * a->H * a->B;
+    const int64_t work = vwork + ceil_div(a->n_tq, r.rows) * text_chunks_of(a) * a->H * a->B;
     return cus * (work <= cus ? 1 : a->D == 64 ? 3 : a->D <= 128 ? 2 : 1);
   }
-  if (a->block_q == kBM && a->D <= 128) return 2 * cus;
-  return cus * (dual_map(a) ? 2 : 1);
+  return cus * (!r.stream && r.rows == kBM && a->D <= 128 ? 2 : r.per_cu);
 }
 
 // Video tiles that run as parts of their key ranges at the end of the launch,
@@ -173,14 +245,16 @@ VideoSplit video_split_of(const lvsa_attn_args* a) {
   const char* e = getenv("LVSA_VIDEO_SPLIT");
   const int64_t cus = cu_count();
   if ((e && strcmp(e, "0") == 0) || a->n_q == 0 || a->block_q <= 0 || a->block_q == kStream12BM || cus <= 0) return v;
-  const int64_t vwork = ceil_div(a->n_q, a->block_q) * a->H * a->B;
-  const int64_t groups = concurrent_groups(a, cus, vwork);
-  if (dual_map(a)) {
-    const int64_t work = vwork + ceil_div(a->n_tq, a->block_q) * text_chunks_of(a) * a->H * a->B;
+  const Route route = route_of(a);
+  const int64_t vwork = ceil_div(a->n_q, route.rows) * a->H * a->B;
+  const int64_t groups = concurrent_groups(a, route, cus, vwork);
+  if (route.dual) {
+    const int64_t work = vwork + ceil_div(a->n_tq, route.rows) * text_chunks_of(a) * a->H * a->B;
     if (work > groups) {
       const int64_t s = groups / (2 * kXcds), per_queue = ceil_div(vwork, kXcds);
       v.tiles = (int)(s < per_queue ? s : per_queue);
       v.parts = 2;
+      v.rows = route.rows;
       return v;
     }
   }
@@ -189,12 +263,12 @@ VideoSplit video_split_of(const lvsa_attn_args* a) {
   // Microseconds, as measured on launches of one round: about 1 per key block
   // (fp32: 2.5 times that), 8 to start and end a launch and 5 per item; the
   // merge 3 and its partials at 3 TB/s.
-  const double block_us = (0.75 + 0.3 * a->block_q * a->D / 32768.0) * (a->dtype == LVSA_FP32 ? 2.5 : 1.0);
+  const double block_us = (0.75 + 0.3 * route.rows * a->D / 32768.0) * (a->dtype == LVSA_FP32 ? 2.5 : 1.0);
   const int64_t blocks = guessed_tile_blocks(a);
   const double whole = 8.0 + blocks * block_us + 5.0;
   double best = whole - (5.0 > 0.07 * whole ? 5.0 : 0.07 * whole);
   for (int k = 2; k <= kMaxParts && blocks >= 6 * k; ++k) {
-    const VideoSplit w{(int)ceil_div(rest, kXcds), k};
+    const VideoSplit w{(int)ceil_div(rest, kXcds), k, route.rows};
     const int64_t bytes = video_ws_bytes(a, w);
     const double t = 8.0 + ceil_div(rest * k, groups) * (blocks * block_us / k + 5.0) + 3.0 + bytes / 3e6;
     if (t < best && bytes <= kMaxVideoSplitBytes) {
@@ -295,19 +369,6 @@ __global__ __launch_bounds__(256) void attn_video_merge_kernel(AttnParams p, int
         L > 0.f ? (M + __log2f(L)) * 0.69314718055994530942f : -INFINITY;
 }
 
-// Whether the short last key block of the frame-structured source crosses a
-// frame boundary: it holds the t = n_k - 64 floor((n_k - 1) / 64) < 64 last
-// keys, tokens [k_tok0 + n_k - t, k_tok0 + n_k), and the last boundary at or
-// below its end lies e = (k_tok0 + n_k) mod C tokens before that end.  The
-// plan builder describes such a block as "generic" (two frames and the rows
-// past the end of the source).
-bool stream_tail_crosses_frame(int64_t n_q, int64_t n_k, int64_t k_tok0, int C) {
-  if (n_q == 0 || n_k <= 0 || C <= 0) return false;
-  const int64_t t = n_k - kBN * ((n_k - 1) / kBN);
-  const int64_t e = (k_tok0 + n_k) % C;
-  return t < kBN && e > 0 && e < t;
-}
-
 bool aligned16(const void* ptr, const int64_t* str, int n, int elem_bytes) {
   if (((uintptr_t)ptr) % 16) return false;
   for (int i = 0; i < n; ++i)
@@ -349,10 +410,10 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
                LVSA_ERR_UNSUPPORTED,
                "lvsa_attn_fwd: 384-row tiles need head_dim 64 in bf16/fp16 and frames of >= 383 query and >= 64 "
                "key rows (head_dim %d, R %d, C %d); build the plan with block_q 256", a->D, a->R, a->C);
-  const int n_vt = (int)ceil_div(a->n_q, a->block_q), n_tt = (int)ceil_div(a->n_tq, a->block_q);
-  LVSA_REQUIRE(a->n_video_tiles == n_vt && a->n_tiles == n_vt + n_tt, LVSA_ERR_INVALID_ARG,
+  const int plan_vt = (int)ceil_div(a->n_q, a->block_q), plan_tt = (int)ceil_div(a->n_tq, a->block_q);
+  LVSA_REQUIRE(a->n_video_tiles == plan_vt && a->n_tiles == plan_vt + plan_tt, LVSA_ERR_INVALID_ARG,
                "lvsa_attn_fwd: plan has %d/%d tiles, expected %d/%d for block_q %d", a->n_video_tiles,
-               a->n_tiles, n_vt, n_vt + n_tt, a->block_q);
+               a->n_tiles, plan_vt, plan_vt + plan_tt, a->block_q);
   LVSA_REQUIRE(a->n_q == 0 || (a->q && a->o), LVSA_ERR_INVALID_ARG, "lvsa_attn_fwd: null q/o");
   LVSA_REQUIRE(a->n_tq == 0 || (a->qt && a->ot), LVSA_ERR_INVALID_ARG, "lvsa_attn_fwd: null text q/o");
   LVSA_REQUIRE(a->n_k == 0 || (a->k && a->v), LVSA_ERR_INVALID_ARG, "lvsa_attn_fwd: null k/v");
@@ -395,6 +456,8 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
     if (ws.bytes > a->workspace_bytes) ws = least;
   }
   const int chunks = ws.chunks;
+  const Route route = route_of(a);
+  const int n_vt = (int)ceil_div(a->n_q, route.rows), n_tt = (int)ceil_div(a->n_tq, route.rows);
   LVSA_REQUIRE(a->workspace_bytes >= ws_need, LVSA_ERR_CAPACITY,
                "lvsa_attn_fwd: workspace of %lld bytes < %lld needed (lvsa_attn_workspace_query)",
                (long long)a->workspace_bytes, (long long)ws_need);
@@ -464,75 +527,37 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   p.vsplit = ws.v.tiles;
   p.vparts = ws.v.parts;
   p.vws = ws.v.tiles > 0 ? (float*)((char*)a->workspace + ws.video) : nullptr;
-  // The single-stream kernel (D = 64, 96 and 128 here; 192 and 256 below)
-  // serves plans without generic descriptors:
-  // 256-row tiles touch at most two query frames when frames have >= 255
-  // rows, and 64-key blocks (even short last ones) at most two key frames
-  // when frames have >= 64 keys.  LVSA_ATTN_KERNEL=pp selects the ping-pong
-  // kernel instead (comparisons).
-  const char* kenv = getenv("LVSA_ATTN_KERNEL");
-  const bool force_pp = kenv != nullptr && strcmp(kenv, "pp") == 0;
-  // Its copies address a whole key source through one buffer resource with
-  // 32-bit byte offsets; at D = 96 and 192 the lanes of the unused chunks of
-  // a row add 0x7FFF0000 to theirs, which must lie past the end of the
-  // source (zeros, no access) or inside it (a harmless read into chunks no
-  // read touches): the rows must stay below 2^31 bytes there.
-  const int64_t lim = (a->D == 96 || a->D == 192) ? (1LL << 31) : (1LL << 32);
-  auto fits32 = [lim](int64_t rows, int64_t row_elems) { return (rows + kBN) * row_elems * 2 < lim; };
-  const bool src32 = fits32(a->n_k, a->k_str[1]) && fits32(a->n_k, a->v_str[1]) &&
-                     (a->n_x == 0 || (fits32(a->n_x, a->kx_str[1]) && fits32(a->n_x, a->vx_str[1])));
-  // Its lane copy offsets are 24-bit products (row x row stride in bytes).
-  const bool str24 = fits24(a->k_str[1]) && fits24(a->v_str[1]) &&
-                     (a->n_x == 0 || (fits24(a->kx_str[1]) && fits24(a->vx_str[1])));
-  // Its loop masks "two-part" descriptors only.  A short last key block of
-  // the frame source that crosses a frame boundary (a source starting
-  // mid-frame, as on a context-parallel shard) has three parts (two frames
-  // and the rows past the end) and is planned "generic".
-  const bool tail_cross = stream_tail_crosses_frame(a->n_q, a->n_k, a->k_tok0, p.C);
-  const bool stream_src = src32 && str24 && !tail_cross;
   // A plan holds generic blocks only where a tile touches more than two query
   // frames or a key block more than two parts.
-  const bool generic = a->n_q > 0 && (p.R < a->block_q - 1 || p.C < kBN || tail_cross);
+  const bool generic = a->n_q > 0 && (p.R < a->block_q - 1 || p.C < kBN || route.tail_cross);
   p.rel_lds = generic && p.words <= kRelWords;
-  p.use_stream = (!fp32 && (a->D == 128 || a->D == 96 || a->D == 64) && a->block_q == kPPBM && !force_pp &&
-                  stream_src && (a->n_q == 0 || (p.R >= 255 && p.C >= 64))) ? 1 : 0;
-  // D = 192 and 256: the wide single-stream loop on the 4-wave kernel's
-  // 128-row tiles, which touch at most two query frames when frames have
-  // >= 127 rows.
-  if (!fp32 && (a->D == 192 || a->D == 256) && a->block_q == kBM && !force_pp && stream_src &&
-      (a->n_q == 0 || (p.R >= 127 && p.C >= 64)))
-    p.use_stream = 1;
   // D = 192 on 256-row tiles: the loop's dual-wide map, the only kernel for
   // them (frames of >= 255 query rows).
-  if (a->D == 192 && a->block_q == kPPBM) {
-    LVSA_REQUIRE(!force_pp && stream_src && (a->n_q == 0 || (p.R >= 255 && p.C >= 64)), LVSA_ERR_UNSUPPORTED,
-                 "lvsa_attn_fwd: head_dim 192 on 256-row tiles needs frames of >= 255 query and >= 64 key rows, "
-                 "key sources below 2^31 bytes with row strides below 16 MiB, the last key block of the frame "
-                 "source inside one frame, and no LVSA_ATTN_KERNEL=pp (R %d, C %d); build the plan with block_q 128",
-                 p.R, p.C);
-    p.use_stream = 1;
-  }
+  LVSA_REQUIRE(a->D != 192 || a->block_q != kPPBM || route.stream, LVSA_ERR_UNSUPPORTED,
+               "lvsa_attn_fwd: head_dim 192 on 256-row tiles needs frames of >= 255 query and >= 64 key rows, "
+               "key sources below 2^31 bytes with row strides below 16 MiB, the last key block of the frame "
+               "source inside one frame, and no LVSA_ATTN_KERNEL=pp (R %d, C %d); build the plan with block_q 128",
+               p.R, p.C);
   if (a->block_q == kStream12BM) {
-    LVSA_REQUIRE(src32, LVSA_ERR_UNSUPPORTED,
+    LVSA_REQUIRE(route.src32, LVSA_ERR_UNSUPPORTED,
                  "lvsa_attn_fwd: 384-row tiles address each key source with 32-bit byte offsets (source too large); "
                  "build the plan with block_q 256");
-    LVSA_REQUIRE(!tail_cross, LVSA_ERR_UNSUPPORTED,
+    LVSA_REQUIRE(!route.tail_cross, LVSA_ERR_UNSUPPORTED,
                  "lvsa_attn_fwd: 384-row tiles need the last key block of the frame source inside one frame "
                  "(n_k %lld, k_tok0 %lld, C %d); build the plan with block_q 256",
                  (long long)a->n_k, (long long)a->k_tok0, p.C);
-    p.use_stream = 1;
   }
-  // D = 64 on 256-row tiles: the dual map (64 rows per wave, 4 waves, two
-  // work-groups per CU); LVSA_D64_WAVES=8 selects 8 waves of 32 rows instead
-  // (comparisons).
-  p.dual = (p.use_stream && dual_map(a)) ? 1 : 0;
+  p.use_stream = route.stream || a->block_q == kStream12BM;
+  p.dual = route.dual;
+  p.half = route.half;
+  p.plan_shift = route.shift;
   // With a workspace, the single-stream kernel runs one persistent
-  // work-group per CU (two with the dual map) over the work queues (counters
-  // zeroed first).
+  // work-group per CU (two with the dual and the half map) over the work
+  // queues (counters zeroed first).
   p.queues = nullptr;
   p.grid = static_grid(p);
   const int cus = cu_count();
-  const int per_cu = p.dual ? 2 : 1;
+  const int per_cu = route.per_cu;
   if (p.use_stream && a->workspace && cus > 0 && work > per_cu * cus) {
     p.queues = (uint32_t*)((char*)a->workspace + ws.queue);
     p.grid = per_cu * cus;
@@ -551,11 +576,11 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   else rc = launch_d64(p, bq, bf16, stream);
   if (rc != LVSA_OK) return rc;
   if (p.vsplit > 0) {
-    const int64_t threads = (int64_t)kXcds * p.vsplit * bq * (a->D / 4);
+    const int64_t threads = (int64_t)kXcds * p.vsplit * route.rows * (a->D / 4);
     const dim3 grid((unsigned)ceil_div(threads, 256));
-    if (fp32) hipLaunchKernelGGL(attn_video_merge_kernel<float>, grid, dim3(256), 0, stream, p, bq, a->D);
-    else if (bf16) hipLaunchKernelGGL(attn_video_merge_kernel<__bf16>, grid, dim3(256), 0, stream, p, bq, a->D);
-    else hipLaunchKernelGGL(attn_video_merge_kernel<_Float16>, grid, dim3(256), 0, stream, p, bq, a->D);
+    if (fp32) hipLaunchKernelGGL(attn_video_merge_kernel<float>, grid, dim3(256), 0, stream, p, route.rows, a->D);
+    else if (bf16) hipLaunchKernelGGL(attn_video_merge_kernel<__bf16>, grid, dim3(256), 0, stream, p, route.rows, a->D);
+    else hipLaunchKernelGGL(attn_video_merge_kernel<_Float16>, grid, dim3(256), 0, stream, p, route.rows, a->D);
     rc = launch_status("lvsa_attn_fwd (video merge)");
     if (rc != LVSA_OK) return rc;
   }

@@ -84,6 +84,10 @@ struct AttnParams {
   // D = 64, 256-row tiles on the single-stream kernel: the dual map (4 waves
   // of 64 rows, two work-groups per CU) rather than 8 waves of 32 rows
   int dual;
+  // D = 64 and 128 on the single-stream kernel: the half map, tiles of 128
+  // rows; with plan_shift 1 the plan's tiles have 256 and two tiles share one
+  // entry list
+  int half, plan_shift;
   // Key-range split of each queue's last video tiles: the last min(vsplit,
   // videos of the queue) video items of queue x run as vparts (0: two) equal
   // parts of their entry lists, after the queue's whole tiles, and write
@@ -425,8 +429,11 @@ __device__ __forceinline__ void text_partial_dst(const AttnParams& p, const Work
 // `chunk` of text_chunks (part `vhalf` of a split video tile's parts) equal
 // shares of them.
 __device__ __forceinline__ void item_entries(const AttnParams& p, const WorkItem& it, int& e0, int& e1) {
-  e0 = p.tile_indptr[it.tile];
-  e1 = p.tile_indptr[it.tile + 1];
+  const int t = !p.plan_shift ? it.tile
+                : it.text     ? ((p.n_vt + 1) >> 1) + ((it.tile - p.n_vt) >> 1)
+                              : it.tile >> 1;
+  e0 = p.tile_indptr[t];
+  e1 = p.tile_indptr[t + 1];
   const int shares = it.vhalf >= 0 ? (p.vparts > 2 ? p.vparts : 2) : it.text ? p.text_chunks : 1;
   if (shares > 1) {
     const int len = (e1 - e0 + shares - 1) / shares;

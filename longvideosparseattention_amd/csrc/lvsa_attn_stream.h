@@ -5,7 +5,9 @@
 // or 12 waves and 384 rows; for D = 192 and 256 the wide map, 4 waves and 128
 // rows, one wave per SIMD with O in AGPRs and K and V in two-stage rings, and
 // for D = 192 by default the dual-wide map, the wide map with 64 rows per wave
-// as two 32-row halves and 256-row tiles),
+// as two 32-row halves and 256-row tiles; and for D = 64 and 128 the half map,
+// 4 waves of 32 rows on 128-row tiles, two work-groups per CU, for frames of
+// 127 to 254 rows and launches too small for 256-row tiles),
 // each wave issuing S = K Q^T, the softmax and O += V^T P^T of consecutive
 // 32-key sub-blocks as one instruction stream
 // (the key loop is hand-scheduled assembly generated by gen_stream_asm.py into
@@ -17,8 +19,8 @@
 //
 // The loop handles plan descriptors "none" and "two-part" only; lvsa_attn_fwd
 // sends geometries that can produce generic descriptors (query frames below
-// 255 rows, 127 for the 128-row tiles of the wide map, or key frames below 64
-// rows) to attn_fwd_pp_kernel / attn_fwd_kernel, and accepts 384-row tiles
+// 255 rows, 127 for the 128-row tiles of the wide and half maps, or key frames
+// below 64 rows) to attn_fwd_pp_kernel / attn_fwd_kernel, and accepts 384-row tiles
 // only for query frames of at least 383 rows (256-row tiles at D = 192, which
 // only the dual-wide map runs, for at least 255).
 #pragma once
@@ -99,19 +101,22 @@ __device__ __forceinline__ void vset(U32Split<LO, HI>& v, int i, uint32_t x) {
 // generated key loop over the item's plan entries with the K/V ring at LDS
 // address lds0, the normalised O (or the text partial) and the LSE to memory.
 // DW selects the dual-wide map of D = 192 (4 waves of 64 rows on the wide
-// map's rings, 256-row tiles).
-template <int D, int NW, typename E, bool DW = false>
+// map's rings, 256-row tiles), HALF the half map of D = 64 and 128 (4 waves of
+// 32 rows, 128-row tiles, two work-groups per CU).
+template <int D, int NW, typename E, bool DW = false, bool HALF = false>
 __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem& it, uint32_t lds0) {
   static_assert(((D == 128 || D == 96) && NW == 8) || (D == 64 && (NW == 8 || NW == 12 || NW == 4)) ||
-                    ((D == 192 || D == 256) && NW == 4),
-                "the generated loops exist for D = 128 and 96 with 8 waves, D = 64 with 4, 8 or 12 and "
-                "D = 192 and 256 with 4");
+                    ((D == 192 || D == 256) && NW == 4) || (D == 128 && NW == 4 && HALF),
+                "the generated loops exist for D = 128 and 96 with 8 waves, D = 64 with 4, 8 or 12, "
+                "D = 192 and 256 with 4 and D = 128 with 4 (the half map)");
+  static_assert(!HALF || ((D == 64 || D == 128) && NW == 4), "the half map is D = 64 or 128 with 4 waves");
   static_assert(!DW || (D == 192 && NW == 4), "the dual-wide map is D = 192 with 4 waves");
   using Op = Ops<E>;
-  constexpr bool kWide = NW == 4 && D >= 192;   // one wave per SIMD, O in AGPRs, K and V rings of two stages
+  constexpr bool kWide = NW == 4 && D >= 192;   // one wave per SIMD, O in AGPRs
+  constexpr bool kRing2 = NW == 4 && D >= 128;  // K and V rings of two stages
   // 64 rows per wave (two 32-row halves): D = 64 with two work-groups per CU,
   // and the dual-wide map
-  constexpr bool kDual = (NW == 4 && D == 64) || DW;
+  constexpr bool kDual = (NW == 4 && D == 64 && !HALF) || DW;
   constexpr int NR = kDual ? 2 : 1;             // 32-row halves per wave
   constexpr int BM = 32 * NR * NW;              // query rows per tile
   // LDS layout: D = 96 rows on the D = 128 pitch, D = 192 rows on the D = 256 pitch
@@ -196,7 +201,7 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
     for (int dt = 0; dt < NT; ++dt) {
       const int chunk = 4 * dt + 2 * dgrp + ((lane & 3) >> 1);
       const int inb = (lane & 1) * 8;
-      constexpr int VB = (kWide ? 2 : kPPStages) * TILE;   // V stages follow the K stages
+      constexpr int VB = (kRing2 ? 2 : kPPStages) * TILE;   // V stages follow the K stages
       voff[dt] = lds0 + VB + rowA * RB + ((chunk ^ sw_a) << 4) + inb;
       voff[NT + dt] = lds0 + VB + (rowA + 8) * RB + ((chunk ^ sw_b) << 4) + inb;
     }
@@ -243,6 +248,8 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
   }
   u32x4 misc;                        // tile row, 4*h, -inf, mask temp
   misc[0] = (uint32_t)(32 * NR * wave + i32);   // tile row (the dual map: of half 0; half 1 is 32 below)
+  // the half map's tile may be the second half of a plan tile of 2 * BM rows
+  if constexpr (HALF) misc[0] += text ? 0u : (uint32_t)(BM * (tile & p.plan_shift));
   misc[1] = (uint32_t)(4 * h);
   misc[2] = 0xff800000u;
   misc[3] = 0u;
@@ -294,7 +301,27 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is written by the copies
     constexpr bool bf = std::is_same<E, __bf16>::value;
-    if constexpr (D == 128 && bf) {
+    if constexpr (HALF && D == 128 && bf) {
+      asm volatile(LVSA_STREAM128W4H_LOOP_BF16
+                   : LVSA_STREAM128W4H_OUTPUTS(o0, o1, o2, o3, ml, misc)
+                   : LVSA_STREAM128W4H_INPUTS(qv, koff, voff, dma, sa, sb, sc, ones)
+                   : LVSA_STREAM128W4H_CLOBBERS);
+    } else if constexpr (HALF && D == 128) {
+      asm volatile(LVSA_STREAM128W4H_LOOP_F16
+                   : LVSA_STREAM128W4H_OUTPUTS(o0, o1, o2, o3, ml, misc)
+                   : LVSA_STREAM128W4H_INPUTS(qv, koff, voff, dma, sa, sb, sc, ones)
+                   : LVSA_STREAM128W4H_CLOBBERS);
+    } else if constexpr (HALF && bf) {
+      asm volatile(LVSA_STREAM64W4H_LOOP_BF16
+                   : LVSA_STREAM64W4H_OUTPUTS(o0, o1, ml, misc)
+                   : LVSA_STREAM64W4H_INPUTS(qv, koff, voff, dma, sa, sb, sc, ones)
+                   : LVSA_STREAM64W4H_CLOBBERS);
+    } else if constexpr (HALF) {
+      asm volatile(LVSA_STREAM64W4H_LOOP_F16
+                   : LVSA_STREAM64W4H_OUTPUTS(o0, o1, ml, misc)
+                   : LVSA_STREAM64W4H_INPUTS(qv, koff, voff, dma, sa, sb, sc, ones)
+                   : LVSA_STREAM64W4H_CLOBBERS);
+    } else if constexpr (D == 128 && bf) {
       asm volatile(LVSA_STREAM128_LOOP_BF16
                    : LVSA_STREAM128_OUTPUTS(o0, o1, o2, o3, ml, misc)
                    : LVSA_STREAM128_INPUTS(qv, koff, voff, dma, sa, sb, sc, ones)
@@ -417,13 +444,15 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
 // other waves.  The barrier after an item keeps the next item's first copies
 // out of the LDS ring until every wave has left the key loop.  The dual map
 // (D = 64, 4 waves) runs two work-groups per CU: 256 VGPRs per wave and a
-// 64 KiB ring each.  DW: the dual-wide map of D = 192 (stream_item).
-template <int D, int NW, typename E, bool DW = false>
-__global__ __launch_bounds__(64 * NW, (NW == 4 && D == 64) ? 2 : 1) void attn_fwd_stream_kernel(AttnParams p) {
+// 64 KiB ring each; so does the half map.  DW: the dual-wide map of D = 192,
+// HALF: the half map (stream_item).
+template <int D, int NW, typename E, bool DW = false, bool HALF = false>
+__global__ __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) void attn_fwd_stream_kernel(AttnParams p) {
   // one K or V block (D = 96 on the D = 128 pitch, D = 192 on the D = 256 pitch)
   constexpr int TILE = kBN * 2 * (D == 96 ? 128 : D == 192 ? 256 : D);
-  // K and V stages: four each, two each in the wide map (4 waves, D = 192 and 256)
-  __shared__ __attribute__((aligned(1024))) char smem_raw[2 * ((NW == 4 && D >= 192) ? 2 : kPPStages) * TILE];
+  // K and V stages: four each, two each in the wide map (4 waves, D = 192 and
+  // 256) and the half map of D = 128
+  __shared__ __attribute__((aligned(1024))) char smem_raw[2 * ((NW == 4 && D >= 128) ? 2 : kPPStages) * TILE];
   __shared__ int next_item;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char*)smem_raw;
   int qx = 0, dry = 0;                    // thread 0: queue being drained, queues found empty
@@ -441,7 +470,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && D == 64) ? 2 : 1) void attn_fw
       it = map_work(p);
       if (it.tile < 0) break;
     }
-    stream_item<D, NW, E, DW>(p, it, lds0);   // one call site: one copy of the key loop
+    stream_item<D, NW, E, DW, HALF>(p, it, lds0);   // one call site: one copy of the key loop
     __syncthreads();
   }
 }

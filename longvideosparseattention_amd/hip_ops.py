@@ -51,7 +51,12 @@ def attn_block_q(head_dim: int = 128, dtype: Optional[torch.dtype] = None, frame
     256 for head sizes 64, 96 and 128 in 16-bit: the single-stream kernels
     (head size 64: the dual map, 4 waves of 64 rows, two work-groups per CU)
     when query frames span at least 255 rows and key frames at least 64, the
-    8-wave ping-pong kernel otherwise.  256 for 192 in 16-bit where the
+    8-wave ping-pong kernel otherwise.  128 for 64 and 128 in 16-bit on
+    shorter query frames, of which a 256-row tile would touch more than two:
+    the single-stream kernel's half map from 127 rows on (24 frames of 130
+    tokens, 12 heads, D = 128: 63.6 -> 52.4 us; 48 of 200, 16 heads: 242 ->
+    223; D = 64: 50.0 -> 39.5 and 167 -> 144), the 4-wave kernel below (48 of
+    100: 117 -> 110; 48 of 40, 12 heads: 40 -> 34).  256 for 192 in 16-bit where the
     single-stream kernel's dual-wide map (4 waves of 64 rows) takes the
     geometry: query frames of at least 255 rows (``frame_rows``), key frames
     of at least 64 (``key_rows``), and a key source of ``n_k`` rows from
@@ -89,6 +94,9 @@ def attn_block_q(head_dim: int = 128, dtype: Optional[torch.dtype] = None, frame
         return 384 if ok else 256
     if env:
         return int(env)
+    if kd != 96 and 0 < frame_rows < 255 and os.environ.get("LVSA_ATTN_KERNEL") != "pp" and \
+            not stream_tail_crosses_frame(1, n_k, k_tok0, key_rows):
+        return 128
     return 256
 
 

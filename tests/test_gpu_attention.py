@@ -899,13 +899,13 @@ def test_work_queues_match_static_grid(cfg, gpu, monkeypatch):
 
 PARTS = [
     # T, P, H, Hkv, D, n_txt, dtype: fewer rounds than kSplitRounds with a part-filled last one
-    (9, 512, 4, 2, 128, 0, torch.bfloat16),     # 72 tiles on 256 CUs: every tile in parts, no queues
+    (9, 512, 4, 2, 128, 0, torch.bfloat16),     # the half map on a 256-row plan, no queues
     (33, 400, 6, 6, 128, 40, torch.float16),    # 312 tiles: the work queues, text chunks
-    (9, 600, 3, 1, 64, 0, torch.bfloat16),      # the dual map below its queue launch
+    (9, 600, 3, 1, 64, 0, torch.bfloat16),      # the half map of D = 64
     (9, 600, 3, 3, 96, 5, torch.bfloat16),
     (9, 500, 4, 2, 192, 0, torch.bfloat16),     # dual-wide map
     (9, 500, 2, 2, 256, 9, torch.float16),      # wide map, 128-row tiles
-    (50, 200, 3, 3, 128, 0, torch.bfloat16),    # ping-pong kernel, generic masks
+    (50, 200, 3, 3, 96, 0, torch.bfloat16),     # ping-pong kernel, generic masks
     (50, 126, 1, 1, 256, 0, torch.bfloat16),    # 4-wave kernel
     (9, 500, 2, 1, 128, 0, torch.float32),      # fp32, two key groups
     (13, 900, 9, 9, 64, 70, torch.float32),     # fp32, more tiles than concurrent work-groups
@@ -932,6 +932,45 @@ def test_video_tiles_in_parts(cfg, gpu, monkeypatch):
     tol = {torch.bfloat16: 4e-3, torch.float16: 1e-3, torch.float32: 2e-6}[dt]
     for a, b in zip(parts, whole):
         torch.testing.assert_close(a.float(), b.float(), atol=tol, rtol=tol)
+
+
+HALF = [
+    # T, P, H, Hkv, n_txt, dtype, B: the half map's plans
+    (9, 127, 2, 1, 5, torch.bfloat16, 1),     # shortest frames, 128-row plan; a last tile of 119 rows
+    (7, 254, 3, 3, 0, torch.float16, 2),      # longest frames with a 128-row plan
+    (11, 128, 2, 2, 130, torch.bfloat16, 1),  # frames on the tiles; two text tiles
+    (5, 255, 2, 2, 3, torch.bfloat16, 1),     # 256-row plan, two tiles per entry list, row splits in both halves
+    (5, 385, 4, 2, 200, torch.float16, 1),    # ... text tiles of both halves; an odd number of 128-row tiles
+    (1, 257, 1, 1, 0, torch.bfloat16, 1),     # one row in the last plan tile
+    (40, 200, 16, 4, 37, torch.bfloat16, 1),  # more tiles than two per CU: the work queues
+]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("cfg", HALF, ids=[str(c[:5]) for c in HALF])
+def test_half_map(cfg, D, gpu):
+    """The half map (D = 64 and 128, 128-row tiles) against the fp32 oracle."""
+    T, P, H, Hkv, n_txt, dt, B = cfg
+    N = T * P
+    m = _meta(T, P, 1, 1, 4, 2)
+    q, k, v, qt, kt, vt = _draw([(B, N, H, D), (B, N, Hkv, D), (B, N, Hkv, D), (B, n_txt, H, D),
+                                 (B, n_txt, Hkv, D), (B, n_txt, Hkv, D)], seed=P, dtype=dt)
+    g = [x.to(gpu) for x in (q, k, v, qt, kt, vt)]
+    kw = dict(k_text=g[4], v_text=g[5], q_text=g[3]) if n_txt else {}
+    res = lv.lvsa_attention(g[0], g[1], g[2], m, return_lse=True, **kw)
+    o, lse = (res[0], res[2]) if n_txt else res
+    rows = [set(r) for r in om.build_frame_mask(T, P, 1, 1, 4, offset=2).rows]
+    frames = None if T < 20 else [0, 1, T // 2, T - 1]
+    ro, rl = oa.per_frame_sdpa(g[0].float(), g[1].float(), g[2].float(), rows, P,
+                               k_extra=g[4].float() if n_txt else None, v_extra=g[5].float() if n_txt else None,
+                               frames=frames)
+    _close(o, ro, str(cfg))
+    if frames is None:
+        torch.testing.assert_close(lse, rl.to(gpu), atol=2e-2, rtol=0)
+    if n_txt:
+        rto, rtl = oa.text_row_attention(g[3].float(), g[1].float(), g[2].float(), g[4].float(), g[5].float())
+        _close(res[1], rto, str(cfg) + " text rows")
+        torch.testing.assert_close(res[3], rtl.to(gpu), atol=2e-2, rtol=0)
 
 
 TALL = [

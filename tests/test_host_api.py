@@ -160,6 +160,26 @@ def test_head_sizes_of_the_plugin():
         hip_ops.kernel_head_dim(80)
 
 
+def test_block_q_short_frames(monkeypatch):
+    """Head sizes 64 and 128 plan 128-row tiles for query frames below 255
+    rows, which the entry point runs on the half map or the 4-wave kernel."""
+    from longvideosparseattention_amd import hip_ops
+
+    monkeypatch.delenv("LVSA_ATTN_BLOCK_Q", raising=False)
+    monkeypatch.delenv("LVSA_ATTN_KERNEL", raising=False)
+    for d in (64, 128):
+        assert hip_ops.attn_block_q(d, torch.bfloat16, 254, 254) == 128
+        assert hip_ops.attn_block_q(d, torch.float16, 30, 30) == 128
+        assert hip_ops.attn_block_q(d, torch.bfloat16, 255, 255) == 256
+        assert hip_ops.attn_block_q(d) == 256                                       # no geometry
+        # the short last block crosses a frame boundary: planned generic
+        assert hip_ops.attn_block_q(d, torch.bfloat16, 130, 130, n_k=150, k_tok0=0) == 256
+        assert hip_ops.attn_block_q(d, torch.float32, 130, 130) == 128
+    assert hip_ops.attn_block_q(96, torch.bfloat16, 130, 130) == 256
+    monkeypatch.setenv("LVSA_ATTN_KERNEL", "pp")
+    assert hip_ops.attn_block_q(128, torch.bfloat16, 130, 130) == 256
+
+
 def test_block_q_head_192(monkeypatch):
     """Head size 192 in 16-bit: 256-row tiles (the dual-wide map) for query
     frames >= 255 rows, key frames >= 64 and a short last key block inside

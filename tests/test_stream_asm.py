@@ -290,3 +290,27 @@ def test_wide_loop_dual_rare_path_and_fp16():
     err, lse_err, _ = run_loop([(j, _tail(150, j)) for j in range(3)], 150, 0, seed=7, dt="f16", D=192, nw=4,
                                dual=True)
     assert err <= 2e-3 and lse_err <= 2e-3, (err, lse_err)
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_half_map(case, D):
+    """The half map: the 8-wave map's waves in work-groups of 4 (128 query
+    rows); D = 128 on two-stage rings (K of block j + 1 and V of block j copied
+    during block j), D = 64 on the four-stage ring."""
+    make, nk, n_x = CASES[case]
+    n = len(make())
+    err, lse_err, copies = run_loop(make(), nk, n_x, D=D, nw=4, dual=False)
+    assert err <= 4e-3 and lse_err <= 2e-3, (case, err, lse_err)
+    assert copies == (4 * 4 * (1 + 2 * n) if D == 128 else 4 * 2 * 2 * (n + 2))
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_half_map_source_switches_rare_path_and_fp16(D):
+    ent = [(0, 0), (0x80000000, _tail(5, 0)), (1, 0), (2, _tail(150, 2))]
+    err, lse_err, _ = run_loop(ent, 150, 5, seed=8, D=D, nw=4, dual=False)
+    assert err <= 4e-3 and lse_err <= 2e-3, (err, lse_err)
+    err, lse_err, _ = run_loop([(j, 0) for j in range(3)], 192, 0, seed=3, D=D, nw=4, dual=False, always_rare=True)
+    assert err <= 4e-3 and lse_err <= 2e-3, (err, lse_err)
+    err, lse_err, _ = run_loop([(j, _tail(150, j)) for j in range(3)], 150, 0, seed=4, dt="f16", D=D, nw=4, dual=False)
+    assert err <= 2e-3 and lse_err <= 2e-3, (err, lse_err)
