@@ -148,9 +148,23 @@ bool stream_tail_crosses_frame(int64_t n_q, int64_t n_k, int64_t k_tok0, int C) 
   return t < kBN && e > 0 && e < t;
 }
 
+// LVSA_VIDEO_SPLIT=0: no video tile's keys are split (comparisons).
+bool no_key_split() {
+  const char* e = getenv("LVSA_VIDEO_SPLIT");
+  return e && strcmp(e, "0") == 0;
+}
+
+// Items of the longest queue (XCD) of a launch with tiles of `rows` rows, video
+// tiles whole.
+int64_t queue_fill(const lvsa_attn_args* a, int rows) {
+  return ceil_div(ceil_div(a->n_q, rows) * a->H * a->B, kXcds) +
+         ceil_div(ceil_div(a->n_tq, rows) * text_chunks_of(a) * a->H * a->B, kXcds);
+}
+
 // Which kernel a call runs, and on tiles of how many rows.
 struct Route {
   bool stream, dual, half;   // the single-stream kernel, and its map
+  bool pairs;                // the half map with two key groups
   int shift;                 // two tiles per plan tile
   int rows;                  // query rows per tile
   int per_cu;                // work-groups per CU
@@ -159,7 +173,7 @@ struct Route {
 Route route_of(const lvsa_attn_args* a) {
   const bool fp32 = a->dtype == LVSA_FP32;
   const int R = a->R > 0 ? a->R : 1, C = a->C > 0 ? a->C : 1;
-  Route r{false, false, false, 0, a->block_q, 1, false, false};
+  Route r{false, false, false, false, 0, a->block_q, 1, false, false};
   // The single-stream kernel (every 16-bit head size) serves plans without
   // generic descriptors: 256-row tiles touch at most two query frames when
   // frames have >= 255 rows (128-row tiles: 127), and 64-key blocks (even
@@ -201,16 +215,24 @@ Route route_of(const lvsa_attn_args* a) {
     r.half = a->D != 96;
   } else if (a->D != 96 && !waves8) {
     // A plan of few 256-row tiles runs as twice as many 128-row ones: while
-    // those are at most one per CU at D = 128 (108 tiles: 51 -> 39 us, 124 with
-    // text 151 -> 106; 143 to 176 within -2% to +8%), two at D = 64 (108 tiles:
+    // each has a CU of its own at D = 128 (108 plan tiles: 51 -> 39 us, 124
+    // with text 151 -> 106; 143 to 176 within -2% to +8%), two at D = 64 (108:
     // 42 -> 35 us, 256: 60 -> 52; 336 with text 103 -> 114).
-    const int64_t tiles = (ceil_div(a->n_q, kPPBM) + ceil_div(a->n_tq, kPPBM) * text_chunks_of(a)) * a->H * a->B;
-    r.half = tiles <= (a->D == 128 ? cu_count() / 2 : cu_count());
+    r.half = queue_fill(a, kBM) * kXcds <= cu_count() * (a->D == 128 ? 1 : 2);
     r.shift = r.half ? 1 : 0;
   }
   r.dual = a->D == 64 && !r.half && !waves8;
-  if (r.half) r.rows = kBM;
-  if (r.half || r.dual) r.per_cu = 2;
+  if (r.half) {
+    r.rows = kBM;
+    // Two key groups while every item has a CU of its own: a single group's
+    // four waves are one per SIMD there, which hides little of the softmax
+    // (D = 64, 108 plan tiles: 36 -> 26 us; D = 128, 84 items 43 -> 33 us, 192
+    // 42 -> 39, 216 42 -> 44: two groups read K and V twice as fast, and at
+    // D = 128 that many of them run into the L2).  Like the video split, off
+    // with LVSA_VIDEO_SPLIT=0.
+    r.pairs = queue_fill(a, kBM) * kXcds <= cu_count() * (a->D == 128 ? 3 : 4) / 4 && !no_key_split();
+  }
+  if (r.half || r.dual) r.per_cu = r.pairs ? 1 : 2;
   return r;
 }
 
@@ -242,9 +264,8 @@ constexpr int kSplitRounds = 5, kMaxParts = 8;
 constexpr int64_t kMaxVideoSplitBytes = 48LL << 20;
 VideoSplit video_split_of(const lvsa_attn_args* a) {
   VideoSplit v;
-  const char* e = getenv("LVSA_VIDEO_SPLIT");
   const int64_t cus = cu_count();
-  if ((e && strcmp(e, "0") == 0) || a->n_q == 0 || a->block_q <= 0 || a->block_q == kStream12BM || cus <= 0) return v;
+  if (no_key_split() || a->n_q == 0 || a->block_q <= 0 || a->block_q == kStream12BM || cus <= 0) return v;
   const Route route = route_of(a);
   const int64_t vwork = ceil_div(a->n_q, route.rows) * a->H * a->B;
   const int64_t groups = concurrent_groups(a, route, cus, vwork);
@@ -261,16 +282,21 @@ VideoSplit video_split_of(const lvsa_attn_args* a) {
   const int64_t rest = vwork % groups;
   if (vwork >= kSplitRounds * groups || rest == 0) return v;
   // Microseconds, as measured on launches of one round: about 1 per key block
-  // (fp32: 2.5 times that), 8 to start and end a launch and 5 per item; the
-  // merge 3 and its partials at 3 TB/s.
-  const double block_us = (0.75 + 0.3 * route.rows * a->D / 32768.0) * (a->dtype == LVSA_FP32 ? 2.5 : 1.0);
+  // (fp32: 2.5 times that, key groups: 0.6), 8 to start and end a launch and 5
+  // per item; the merge 3 and its partials at 3 TB/s.  Rounds are those of the
+  // longest queue: without the work queues an XCD runs its own items only (124
+  // tiles in two parts and 8 text chunks, 33 on an XCD of 32 CUs: 151 us).
+  const double block_us = (0.75 + 0.3 * route.rows * a->D / 32768.0) *
+                          (a->dtype == LVSA_FP32 ? 2.5 : route.pairs ? 0.6 : 1.0);
+  const int64_t text_fill = ceil_div(ceil_div(a->n_tq, route.rows) * text_chunks_of(a) * a->H * a->B, kXcds);
   const int64_t blocks = guessed_tile_blocks(a);
   const double whole = 8.0 + blocks * block_us + 5.0;
   double best = whole - (5.0 > 0.07 * whole ? 5.0 : 0.07 * whole);
   for (int k = 2; k <= kMaxParts && blocks >= 6 * k; ++k) {
     const VideoSplit w{(int)ceil_div(rest, kXcds), k, route.rows};
     const int64_t bytes = video_ws_bytes(a, w);
-    const double t = 8.0 + ceil_div(rest * k, groups) * (blocks * block_us / k + 5.0) + 3.0 + bytes / 3e6;
+    const int64_t rounds = ceil_div((w.tiles * k + text_fill) * kXcds, groups);
+    const double t = 8.0 + rounds * (blocks * block_us / k + 5.0) + 3.0 + bytes / 3e6;
     if (t < best && bytes <= kMaxVideoSplitBytes) {
       best = t;
       v = w;
@@ -549,7 +575,7 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
   }
   p.use_stream = route.stream || a->block_q == kStream12BM;
   p.dual = route.dual;
-  p.half = route.half;
+  p.half = route.pairs ? 2 : route.half ? 1 : 0;
   p.plan_shift = route.shift;
   // With a workspace, the single-stream kernel runs one persistent
   // work-group per CU (two with the dual and the half map) over the work

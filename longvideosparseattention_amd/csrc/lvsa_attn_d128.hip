@@ -6,6 +6,17 @@
 namespace lvsa {
 
 int launch_d128(const AttnParams& prm, int block_q, bool bf16, hipStream_t stream) {
+  if (prm.half == 2) {
+    // two key groups of 4 waves
+    if (bf16) {
+      hipLaunchKernelGGL((attn_fwd_stream_kernel<128, 4, __bf16, false, true, 2>), dim3(prm.grid), dim3(64 * 8), 0,
+                         stream, prm);
+    } else {
+      hipLaunchKernelGGL((attn_fwd_stream_kernel<128, 4, _Float16, false, true, 2>), dim3(prm.grid), dim3(64 * 8), 0,
+                         stream, prm);
+    }
+    return launch_status("lvsa_attn_fwd");
+  }
   if (prm.half) {
     // 4 waves of 32 rows, two work-groups per CU
     if (bf16) {

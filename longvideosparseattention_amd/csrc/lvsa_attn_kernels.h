@@ -84,8 +84,8 @@ struct AttnParams {
   // D = 64, 256-row tiles on the single-stream kernel: the dual map (4 waves
   // of 64 rows, two work-groups per CU) rather than 8 waves of 32 rows
   int dual;
-  // D = 64 and 128 on the single-stream kernel: the half map, tiles of 128
-  // rows; with plan_shift 1 the plan's tiles have 256 and two tiles share one
+  // D = 64 and 128 on the single-stream kernel: the half map (2: with two key
+  // groups), tiles of 128 rows; with plan_shift 1 the plan's tiles have 256 and two tiles share one
   // entry list
   int half, plan_shift;
   // Key-range split of each queue's last video tiles: the last min(vsplit,

@@ -102,8 +102,10 @@ __device__ __forceinline__ void vset(U32Split<LO, HI>& v, int i, uint32_t x) {
 // address lds0, the normalised O (or the text partial) and the LSE to memory.
 // DW selects the dual-wide map of D = 192 (4 waves of 64 rows on the wide
 // map's rings, 256-row tiles), HALF the half map of D = 64 and 128 (4 waves of
-// 32 rows, 128-row tiles, two work-groups per CU).
-template <int D, int NW, typename E, bool DW = false, bool HALF = false>
+// 32 rows, 128-row tiles, two work-groups per CU).  KG = 2 (half map): two
+// groups of 4 waves take the first and the second half of the entries, each
+// with a ring of its own, and are merged by log-sum-exp through LDS.
+template <int D, int NW, typename E, bool DW = false, bool HALF = false, int KG = 1>
 __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem& it, uint32_t lds0) {
   static_assert(((D == 128 || D == 96) && NW == 8) || (D == 64 && (NW == 8 || NW == 12 || NW == 4)) ||
                     ((D == 192 || D == 256) && NW == 4) || (D == 128 && NW == 4 && HALF),
@@ -127,7 +129,9 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
   constexpr int NQK = D / 16;
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = KG == 1 ? wave_id : wave_id % NW;   // row wave
+  const int kg = KG == 1 ? 0 : wave_id / NW;           // key group
   const int h = lane >> 5;
   const int i32 = lane & 31;
 
@@ -163,6 +167,15 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
   const bool partial = (text && p.text_chunks > 1) || it.vhalf >= 0;
   int e0, e1;
   item_entries(p, it, e0, e1);
+  const uint32_t lds_item = lds0;
+  int ahead = 0;                       // blocks that group 0 takes more than this one
+  if constexpr (KG == 2) {
+    const int n0 = (e1 - e0 + 1) / 2;
+    ahead = kg == 0 ? 0 : n0 - (e1 - e0 - n0);
+    if (kg == 0) e1 = e0 + n0;
+    else e0 += n0;
+    lds0 += (uint32_t)(kg * 2 * (kRing2 ? 2 : kPPStages) * TILE);
+  }
   const int n = e1 - e0;
 
   // Q fragments (B operand of S^T = K Q^T): row i32 of each 32-row half of
@@ -404,6 +417,42 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
     }
 #pragma clang diagnostic pop
   }
+  if constexpr (KG == 2) {
+    // The key loop passes a barrier per block, and one more before the drain
+    // of a two-stage ring; a group of fewer blocks (one fewer at most) makes
+    // up for the rest here.
+    const int rest = ahead == 0 ? 0 : ahead + ((kRing2 && n == 0) ? 1 : 0);
+    for (int b = 0; b < rest; ++b) wg_barrier();
+    constexpr int W = 16 * NT + 2;     // registers a lane hands over
+    auto* x = (__attribute__((address_space(3))) float*)lds_item + wave * W * 64 + lane;
+    const float l_own = sum_halves(ml[1]);
+    floatx16 own[4] = {o0, o1, o2, o3};
+    __syncthreads();                   // both groups have left their rings
+    if (kg == 1) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[(16 * t + i) * 64] = own[t][i];
+      x[16 * NT * 64] = ml[0];
+      x[(16 * NT + 1) * 64] = l_own;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = x[16 * NT * 64], l1 = x[(16 * NT + 1) * 64];
+    const float m = vmax(ml[0], m1);
+    const float a0 = __builtin_amdgcn_exp2f(ml[0] - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) own[t][i] = a0 * own[t][i] + a1 * x[(16 * t + i) * 64];
+    o0 = own[0];
+    o1 = own[1];
+    o2 = own[2];
+    o3 = own[3];
+    ml[0] = m;
+    // the epilogue adds both lane halves
+    ml[1] = h == 0 ? a0 * l_own + a1 * l1 : 0.f;
+  }
 
   // Epilogue, per 32-row half: combine the row sum of both lane halves,
   // normalise, store.
@@ -445,14 +494,14 @@ __device__ __forceinline__ void stream_item(const AttnParams& p, const WorkItem&
 // out of the LDS ring until every wave has left the key loop.  The dual map
 // (D = 64, 4 waves) runs two work-groups per CU: 256 VGPRs per wave and a
 // 64 KiB ring each; so does the half map.  DW: the dual-wide map of D = 192,
-// HALF: the half map (stream_item).
-template <int D, int NW, typename E, bool DW = false, bool HALF = false>
-__global__ __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) void attn_fwd_stream_kernel(AttnParams p) {
+// HALF: the half map, KG: its key groups (stream_item).
+template <int D, int NW, typename E, bool DW = false, bool HALF = false, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128) ? 2 : 1) void attn_fwd_stream_kernel(AttnParams p) {
   // one K or V block (D = 96 on the D = 128 pitch, D = 192 on the D = 256 pitch)
   constexpr int TILE = kBN * 2 * (D == 96 ? 128 : D == 192 ? 256 : D);
   // K and V stages: four each, two each in the wide map (4 waves, D = 192 and
   // 256) and the half map of D = 128
-  __shared__ __attribute__((aligned(1024))) char smem_raw[2 * ((NW == 4 && D >= 128) ? 2 : kPPStages) * TILE];
+  __shared__ __attribute__((aligned(1024))) char smem_raw[KG * 2 * ((NW == 4 && D >= 128) ? 2 : kPPStages) * TILE];
   __shared__ int next_item;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char*)smem_raw;
   int qx = 0, dry = 0;                    // thread 0: queue being drained, queues found empty
@@ -470,7 +519,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) void attn_f
       it = map_work(p);
       if (it.tile < 0) break;
     }
-    stream_item<D, NW, E, DW, HALF>(p, it, lds0);   // one call site: one copy of the key loop
+    stream_item<D, NW, E, DW, HALF, KG>(p, it, lds0);   // one call site: one copy of the key loop
     __syncthreads();
   }
 }

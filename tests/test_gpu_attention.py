@@ -899,9 +899,9 @@ def test_work_queues_match_static_grid(cfg, gpu, monkeypatch):
 
 PARTS = [
     # T, P, H, Hkv, D, n_txt, dtype: fewer rounds than kSplitRounds with a part-filled last one
-    (9, 512, 4, 2, 128, 0, torch.bfloat16),     # the half map on a 256-row plan, no queues
+    (9, 512, 2, 1, 128, 0, torch.bfloat16),     # the half map on a 256-row plan, no queues
     (33, 400, 6, 6, 128, 40, torch.float16),    # 312 tiles: the work queues, text chunks
-    (9, 600, 3, 1, 64, 0, torch.bfloat16),      # the half map of D = 64
+    (9, 600, 2, 1, 64, 0, torch.bfloat16),      # the half map of D = 64
     (9, 600, 3, 3, 96, 5, torch.bfloat16),
     (9, 500, 4, 2, 192, 0, torch.bfloat16),     # dual-wide map
     (9, 500, 2, 2, 256, 9, torch.float16),      # wide map, 128-row tiles
