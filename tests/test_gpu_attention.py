@@ -973,6 +973,22 @@ def test_half_map(cfg, D, gpu):
         torch.testing.assert_close(res[3], rtl.to(gpu), atol=2e-2, rtol=0)
 
 
+@pytest.mark.parametrize("D", [64, 96, 128, 192, 256])
+@pytest.mark.parametrize("rest", [1, 15, 16, 17, 31, 32])
+def test_output_stores_end_at_the_last_row(rest, D, gpu):
+    """Lanes of a stream-kernel wave store parts of each other's rows: every remainder of a wave's 32 rows
+    against the oracle, in a strided output whose rows past the end and heads beside it stay untouched."""
+    P, H = 384 + rest, 2
+    m = _meta(1, P, 1, 1, 4)
+    q, k, v = (x.to(gpu) for x in _draw([(1, P, H, D)] * 3, seed=rest))
+    buf = torch.full((1, P + 40, H + 1, D), 7.0, dtype=q.dtype, device=gpu)
+    out = buf[:, :P, :H]
+    hip_ops.attn_fwd(q, k, v, m.full_plan(q.device, P, P, 0, 0, D, q.dtype), out=out)
+    ro, _ = oa.per_frame_sdpa(q.float(), k.float(), v.float(), [{0}], P)
+    _close(out, ro, f"{P} rows, D {D}")
+    assert (buf[:, P:] == 7).all() and (buf[:, :, H:] == 7).all()
+
+
 TALL = [
     # T, P, W, kfi, off, H, Hkv, D, n_txt, dtype, B  (head size 64, frames >= 383 rows: 384-row tiles possible)
     (13, 1350, 1, 4, 0, 6, 6, 64, 226, torch.bfloat16, 1),     # CogVideoX frame and text sizes
