@@ -19,12 +19,15 @@
 //   split_f32_kernel splits K and V once per call into the scratch, in the
 //   order in which the MFMAs read their operands, so the attention kernel
 //   only copies them to LDS.  Q is split when a tile is loaded, P in the
-//   softmax.  Tiles whose numbers leave the split's range (a non-finite or
-//   overflowing result, V blocks of a tile more than 2^15 apart) are computed
-//   again by the fp32 loop, so such inputs give what they gave there.
+//   softmax.  One power of two serves a block of K or V (a row of Q), so
+//   numbers below 2^-16 of its largest lose bits one by one.  Tiles that meet
+//   a block with more than a few of them (kSmallExp), infinity, a
+//   non-finite result, an overflowing score or V blocks too far apart are
+//   computed again by the fp32 loop, so such inputs give what they gave there.
 //
-// Measured against float64 (relative 2-norm), 9 x 256 tokens, 12 heads,
-// D = 128: see the dispatch in launch_f32.
+// Error against float64 (relative 2-norm) on N(0, 1) inputs, split and fp32
+// MFMAs: 3.9e-7 and 8.9e-7 at 9 x 256 tokens, 12 heads, D = 128; 1.2e-6 and
+// 2.0e-6 at 13 x 1350 + 226 text tokens, 6 heads, D = 64.
 #include "lvsa_attn_kernels.h"
 
 namespace lvsa {
@@ -265,10 +268,17 @@ __global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void attn_fwd_f32_kerne
 //      16 st + 8 (j / 4) + 4 h + j % 4, j = 0 .. 7 (the keys whose P the lane
 //      of row i already holds).
 // After the slots, one int per slot: the block's exponent e, x = (hi + lo) 2^e
-// with the largest |hi| in [2^14, 2^15] (kZeroBlock: all zero).  Rows past the
-// source's end are zeros.
+// with the largest |hi| in [2^14, 2^15] (kZeroBlock: all zero, kWideBlock: not
+// for the split).  Rows past the source's end are zeros.
 constexpr int kZeroBlock = INT32_MIN;
+constexpr int kWideBlock = INT32_MIN + 1;
 constexpr int kSplitExp = 14;     // exponent of the largest scaled number
+// Scaled numbers from 2^-2 on keep 22 bits: lo's last bit is 2^-24 there.
+// Smaller ones are off by up to 2^-25 whatever their size, which shows where a
+// row or channel holds little else: an outlier in another row of the block
+// (one that the tile's rows may not even attend) or in another channel.  Of
+// N(0, 1) numbers 5 in 10^5 are that small.
+constexpr int kSmallExp = -2;
 
 __host__ __device__ constexpr int64_t split_slot_bytes(int D) { return 4LL * kBN * D; }
 
@@ -309,11 +319,61 @@ __device__ __forceinline__ void split8(const float* x, float sc, halfx8& hi, hal
 }
 
 // Exponent to scale a group of numbers by, from the largest of their |x| (0
-// and non-finite ones included: the latter stay non-finite).  Bounded so that
-// the scale and its inverse are normal numbers.
+// and infinity included: the latter stays infinite).  Bounded so that the
+// scale and its inverse are normal numbers.
 __device__ __forceinline__ int split_exponent(float amax) {
   const int e = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFF) - 127;
   return (e < -112 ? -112 : e) - kSplitExp;
+}
+
+// |x| as an integer in its order, zero as the largest: one v_lshl_add.
+__device__ __forceinline__ uint32_t size_key(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 1u; }
+// Nonzero numbers to be scaled by 2^-e are small if their size_key is below this.
+__device__ __forceinline__ uint32_t small_key(int e) { return size_key(ldexpf(1.f, e + kSmallExp)); }
+
+// Too many small numbers in a share of a row or channel: more than two and
+// more than a quarter of its `n` nonzero ones.
+__device__ __forceinline__ bool mostly_small(int small, int n) { return small > 2 && 4 * small > n; }
+
+// Whether a wave's part x of a block (lane (i, h): NF fragments of 8 numbers)
+// holds rows or channels of mostly small numbers, or is mostly small as a
+// whole.  The numbers j of a fragment over the 32 lanes i are one channel of a
+// K block and one row of a V block; a lane's own numbers are one row of K
+// (over all fragments, by_lane) and one channel of V in each fragment.  Run
+// after the stores and only by waves with a small number (a tenth of them on
+// N(0, 1) inputs), it adds 0.7 us to the 12.0 of 9 x 256 tokens, 12 heads, D =
+// 128, and 0.8 to the 18.6 of 13 x 1350 + 226 tokens, 6 heads, D = 64.
+template <int NF>
+__device__ __forceinline__ bool wide_part(const float (&x)[NF][8], uint32_t below, float own_max, bool by_lane) {
+  // two small numbers in all cannot be too many (the usual case)
+  int few = 0;
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) few += size_key(x[i][j]) < below;
+  if (__popcll(__ballot(few > 0)) <= 2 && !__ballot(few > 1) && __popcll(__ballot(own_max > 0.f)) > 8) return false;
+  bool wide = false;
+  int own = 0, own_small = 0, all = 0, all_small = 0;
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bool nz = x[i][j] != 0.f, sm = size_key(x[i][j]) < below;
+      const uint64_t n = __ballot(nz), m = __ballot(sm);
+      const int n0 = __popc((uint32_t)n), n1 = __popc((uint32_t)(n >> 32));
+      const int m0 = __popc((uint32_t)m), m1 = __popc((uint32_t)(m >> 32));
+      wide |= mostly_small(m0, n0) || mostly_small(m1, n1);
+      all += n0 + n1;
+      all_small += m0 + m1;
+      own += nz;
+      own_small += sm;
+    }
+    if (!by_lane || i == NF - 1) {
+      wide |= mostly_small(own_small, own);
+      own = own_small = 0;
+    }
+  }
+  return wide || 4 * all_small > all;
 }
 
 // One slot per work-group.  HBM bound: reads the block once and writes as many
@@ -342,6 +402,7 @@ __global__ __launch_bounds__(kThreads) void split_f32_kernel(AttnParams p) {
 
   float x[NF][8];
   float amax = 0.f;
+  uint32_t least = ~0u;           // size_key of the smallest nonzero number
 #pragma unroll
   for (int i = 0; i < NF; ++i) {
     const int f = wave * NF + i;
@@ -367,8 +428,13 @@ __global__ __launch_bounds__(kThreads) void split_f32_kernel(AttnParams p) {
       }
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[i][j]));
+    for (int j = 0; j < 8; ++j) {
+      amax = fmaxf(amax, fabsf(x[i][j]));
+      const uint32_t key = size_key(x[i][j]);
+      least = least < key ? least : key;
+    }
   }
+  const float own_max = amax;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
   if (lane == 0) wmax[wave] = amax;
@@ -388,7 +454,12 @@ __global__ __launch_bounds__(kThreads) void split_f32_kernel(AttnParams p) {
     *reinterpret_cast<halfx8*>(d) = hi;
     *reinterpret_cast<halfx8*>(d + (D / 8) * 1024) = lo;
   }
-  if (threadIdx.x == 0) p.split_exp[slot] = amax == 0.f ? kZeroBlock : e;
+  // while the stores are under way
+  const uint32_t below = small_key(e);
+  bool wide = amax == INFINITY;   // the block's other numbers would be scaled to 0; a NaN spoils only its own
+  if (__ballot(least < below)) wide |= wide_part<NF>(x, below, own_max, !is_v);
+  wide = __syncthreads_or(wide);
+  if (threadIdx.x == 0) p.split_exp[slot] = amax == 0.f ? kZeroBlock : wide ? kWideBlock : e;
 }
 
 // KG groups of four waves take the tile's key blocks in turn (group g blocks
@@ -454,6 +525,7 @@ void attn_fwd_split_kernel(AttnParams p) {
   // Q of row i32, scaled by the row's power of two: d = 16c + 8h .. + 7.
   halfx8 qh[ND], ql[ND];
   int eq;                       // Q = (hi + lo) 2^eq
+  bool redo = false;            // the tile leaves the split's range
   {
     const int64_t qr = my_row < t.nrows ? my_row : (int64_t)t.nrows - 1;
     const char* qp = t.qbase + qr * t.qrs + 32 * h;
@@ -467,8 +539,9 @@ void attn_fwd_split_kernel(AttnParams p) {
       for (int j = 0; j < 4; ++j) {
         q[c][j] = a[j];
         q[c][4 + j] = b[j];
-        amax = fmaxf(amax, fmaxf(fabsf(a[j]), fabsf(b[j])));
       }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(q[c][j]));
     }
     amax = fmaxf(amax, __shfl_xor(amax, 32));
     eq = split_exponent(amax);
@@ -487,13 +560,17 @@ void attn_fwd_split_kernel(AttnParams p) {
   float m_run = -1e30f;         // running max of s * scale * log2(e)
   float l_run = 0.f;            // this lane's share of the row sum
   int vexp = -200;              // exponent of oacc (uniform): the largest of the V blocks so far
-  bool redo = false;            // the tile leaves the split's range
   // P is split times 2^12: the running max moves once a block's max exceeds
   // it by more than 3, so that stays within 2^15, and fp16 holds P's lo part
   // down to 2^-37 of the largest P.  (Scaled after the exponential: 12 added
   // to its argument would round the argument to 4 bits less.)
   constexpr int kPExp = 12;
   constexpr float kMaxLag = 3.f;
+  // P of a V block 2^lag below the largest is split times 2^(12 - lag), so that
+  // it adds to oacc at its scale.  A lag of 15 still leaves rows that attend
+  // only such blocks closer to float64 than the fp32 loop does (20 x 192
+  // tokens, D = 128: 3.8e-7 and 8.0e-7).
+  constexpr int kMaxVLag = 15;
 
   const int rounds = (t.e1 - t.e0 + KG - 1) / KG;
   // Two groups run half a round apart (one barrier), so that on each SIMD one
@@ -572,23 +649,28 @@ void attn_fwd_split_kernel(AttnParams p) {
       }
       float mx = vmax(vmax(vmax(mc[0], mc[1]), mc[2]), mc[3]);
       mx = fmaxf(mx, __shfl_xor(mx, 32));
+      // the fp32 loop takes the tile: no further blocks here
+      if (kexp == kWideBlock || ve == kWideBlock) {
+        redo = true;
+        e = t.e1;
+      }
       // An all-zero K block's scores are zero whatever the exponent.
-      const int es = eq + (kexp == kZeroBlock ? 0 : kexp);
+      const int es = eq + (kexp <= kWideBlock ? 0 : kexp);
       const float cs = ldexpf(p.scale_log2, es);
       const float top = ldexpf(mx, es);       // the fp32 score
       redo |= top == INFINITY;                // overflows there, not here
       const float mxs = top * p.scale_log2;
       int lag = 0;              // V of this block is 2^-lag of oacc's scale
       float down = 1.f;         // what oacc is scaled by for this block's V
-      if (ve != kZeroBlock) {
+      if (ve > kWideBlock) {
         if (ve > vexp) {
           down = vexp - ve < -126 ? 0.f : pow2i(vexp - ve);
           vexp = ve;
         }
         lag = vexp - ve;
-        if (lag > 15) {
+        if (lag > kMaxVLag) {
           redo = true;
-          lag = 15;
+          lag = kMaxVLag;
         }
       }
       if (__builtin_amdgcn_ballot_w64(mxs > m_run + kMaxLag) || down != 1.f) {

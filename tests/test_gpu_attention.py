@@ -499,6 +499,90 @@ def test_fp32_split_range(kind, D, gpu):
     torch.testing.assert_close(la, lb, atol=2e-5, rtol=1e-6, equal_nan=True)
 
 
+OUTLIERS = ["k_inf", "k_ninf", "k_nan", "k_1e6", "k_1e8", "k_1e20", "k_rows_1e8", "k_frame_1e10", "k_small_rows",
+            "v_inf", "v_1e6", "v_1e8", "v_1e20", "v_rows_1e8", "v_frame_2^8", "v_frame_2^11", "v_frame_2^13",
+            "v_frame_2^16", "v_channel", "kq_channel"]
+
+
+def _plant(kind, q, k, v, P):
+    """Outliers at the first and the last key of frame 5, in the whole frame or in one channel."""
+    first, last, frame = 5 * P, 6 * P - 1, slice(5 * P, 6 * P)
+    name, _, what = kind.partition("_")
+    t = {"k": k, "v": v}.get(name)
+    if what == "channel":
+        {"v": lambda: v[..., 3].mul_(1e9),
+         "qk": lambda: (q[..., 3].mul_(1e9), k[..., 3].mul_(1e-9)),
+         "kq": lambda: (k[..., 3].mul_(1e9), q[..., 3].mul_(1e-9)),
+         "q": lambda: (q[..., 3].mul_(1e9), k[..., 3].zero_())}[name]()
+    elif what == "small_rows":
+        k[0, ::3] *= 1e-6
+        q *= 1e5
+    elif what == "rows_1e8":
+        t[0, first] *= 1e8
+        t[0, last] *= 1e8
+    elif what == "frame_1e10":
+        t[0, frame] *= 1e10
+    elif what.startswith("frame_2^"):
+        n = int(what[8:])
+        t[0, frame] *= 2.0 ** (n - n // 2)
+        t *= 2.0 ** -(n // 2)
+        t[0, frame] *= 2.0 ** (n // 2)
+    else:
+        t[0, first, 0, 9] = t[0, last, 1, 9] = float(what.replace("ninf", "-inf"))
+
+
+@pytest.mark.parametrize("D", [64, 96, 128, 192, 256])
+@pytest.mark.parametrize("kind", OUTLIERS)
+def test_fp32_split_outliers(kind, D, gpu):
+    """fp32 inputs of a wide range: rows that do not attend the outlier but
+    share a key block with it are no further from float64 than the fp32-MFMA
+    kernel (``scratch=False``), and rows that attend it give what that kernel
+    gives.  Frames of 130 tokens, so frame 5 shares its first and last key
+    block with frames 4 and 6; only frames 4 to 6 attend it, so a tile holds
+    rows of both kinds."""
+    T, P, H = 20, 130, 2
+    N = T * P
+    m = _meta(T, P, 1, 1, 8, 3)
+    rows = om.build_frame_mask(T, P, 1, 1, 8, offset=3).rows
+    assert [f for f in range(T) if 5 in rows[f]] == [4, 5, 6]
+    q, k, v = (x.to(gpu) for x in _draw([(1, N, H, D)] * 3, seed=D, dtype=torch.float32))
+    _plant(kind, q, k, v, P)
+    plan = m.full_plan(gpu, N, N, 0, 0, D, torch.float32)
+    split, _, lse_s, _ = hip_ops.attn_fwd(q, k, v, plan, return_lse=True)
+    plain, _, lse_p, _ = hip_ops.attn_fwd(q, k, v, plan, return_lse=True, scratch=False)
+    frame = torch.arange(N, device=gpu) // P
+    ok = torch.zeros(T, T, dtype=torch.bool, device=gpu)
+    for f, r in enumerate(rows):
+        ok[f, sorted(r)] = True
+    away = torch.ones(N, dtype=torch.bool, device=gpu) if kind.endswith("channel") or "small" in kind else \
+        (frame < 4) | (frame > 6)
+    for h in range(H):
+        s = q[0, :, h].double() @ k[0, :, h].double().T / D ** 0.5
+        s.masked_fill_(~ok[frame][:, frame], float("-inf"))
+        p = torch.softmax(s, -1)
+        vh = v[0, :, h].double()
+        want, size, want_lse = p @ vh, p @ vh.abs(), torch.logsumexp(s, -1)
+        a, b, la, lb = split[0, :, h], plain[0, :, h], lse_s[0, h], lse_p[0, h]
+
+        def errors(o, lse):
+            # relative to the sum of |P V|; all, the worst row and the worst channel
+            e = ((o.double() - want) / size)[away] ** 2
+            return [x.item() for x in (e.mean().sqrt(), e.mean(1).max().sqrt(), e.mean(0).max().sqrt(),
+                                       ((lse.double() - want_lse) / want_lse)[away].abs().max())]
+
+        if kind != "v_inf":                   # 0 * inf is NaN on both kernels
+            got, ref = errors(a, la), errors(b, lb)
+            # the extremes may be half as much again, all rows 1%: tiles in parts round at other points
+            assert all(x <= f * y for x, y, f in zip(got, ref, [1.01, 1.5, 1.5, 1.5])), (kind, h, got, ref)
+        for x, y in ((a, b), (la, lb)):
+            # the rows of k_frame_1e10 that attend it: scores of 1e10 round by hundreds, so exp2 may overflow on either
+            assert kind == "k_frame_1e10" or (torch.equal(torch.isnan(x), torch.isnan(y)) and
+                                              torch.equal(torch.isinf(x), torch.isinf(y))), kind
+        if kind in ("k_inf", "k_ninf") or (kind.startswith("v") and kind != "v_inf"):
+            sel = torch.isfinite(b) & torch.isfinite(size)
+            assert ((a - b).abs()[sel] <= 2e-5 * size[sel]).all(), kind
+
+
 def test_fp32_smaller_workspace_runs_the_fp32_kernel(gpu):
     """A workspace too small for the split operands (1 KiB was enough for any
     fp32 call) still runs, on the fp32 MFMAs: bit for bit the call without."""
