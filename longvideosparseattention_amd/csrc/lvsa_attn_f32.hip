@@ -21,7 +21,7 @@
 //   only copies them to LDS.  Q is split when a tile is loaded, P in the
 //   softmax.  One power of two serves a block of K or V (a row of Q), so
 //   numbers below 2^-16 of its largest lose bits one by one.  Tiles that meet
-//   a block with more than a few of them (kSmallExp), infinity, a
+//   a block or row with more than a few of them (kSmallExp), infinity, a
 //   non-finite result, an overflowing score or V blocks too far apart are
 //   computed again by the fp32 loop, so such inputs give what they gave there.
 //
@@ -531,6 +531,7 @@ void attn_fwd_split_kernel(AttnParams p) {
     const char* qp = t.qbase + qr * t.qrs + 32 * h;
     float q[ND][8];
     float amax = 0.f;
+    uint32_t least = ~0u;
 #pragma unroll
     for (int c = 0; c < ND; ++c) {
       const floatx4 a = *reinterpret_cast<const floatx4*>(qp + 64 * c);
@@ -541,11 +542,30 @@ void attn_fwd_split_kernel(AttnParams p) {
         q[c][4 + j] = b[j];
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(q[c][j]));
+      for (int j = 0; j < 8; ++j) {
+        amax = fmaxf(amax, fabsf(q[c][j]));
+        const uint32_t key = size_key(q[c][j]);
+        least = least < key ? least : key;
+      }
     }
     amax = fmaxf(amax, __shfl_xor(amax, 32));
     eq = split_exponent(amax);
     const float sc = pow2i(-eq);
+    const uint32_t below = small_key(eq);
+    if (__ballot(least < below)) {
+      int n = 0, small = 0;
+#pragma unroll
+      for (int c = 0; c < ND; ++c) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          n += q[c][j] != 0.f;
+          small += size_key(q[c][j]) < below;
+        }
+      }
+      n += __shfl_xor(n, 32);
+      small += __shfl_xor(small, 32);
+      redo = 4 * small > n;
+    }
 #pragma unroll
     for (int c = 0; c < ND; ++c) {
 #pragma unroll
