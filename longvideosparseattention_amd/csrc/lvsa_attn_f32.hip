@@ -579,7 +579,8 @@ void attn_fwd_split_kernel(AttnParams p) {
   for (int dt = 0; dt < NT; ++dt) oacc[dt] = floatx16{0};
   float m_run = -1e30f;         // running max of s * scale * log2(e)
   float l_run = 0.f;            // this lane's share of the row sum
-  int vexp = -200;              // exponent of oacc (uniform): the largest of the V blocks so far
+  constexpr int kNoV = -200;
+  int vexp = kNoV;              // exponent of oacc (uniform): the largest of the V blocks so far
   // P is split times 2^12: the running max moves once a block's max exceeds
   // it by more than 3, so that stays within 2^15, and fp16 holds P's lo part
   // down to 2^-37 of the largest P.  (Scaled after the exponential: 12 added
@@ -590,7 +591,7 @@ void attn_fwd_split_kernel(AttnParams p) {
   // it adds to oacc at its scale.  A lag of 15 still leaves rows that attend
   // only such blocks closer to float64 than the fp32 loop does (20 x 192
   // tokens, D = 128: 3.8e-7 and 8.0e-7).
-  constexpr int kMaxVLag = 15;
+  constexpr int kMaxVLag = 15, kMaxRise = 64;
 
   const int rounds = (t.e1 - t.e0 + KG - 1) / KG;
   // Two groups run half a round apart (one barrier), so that on each SIMD one
@@ -684,6 +685,8 @@ void attn_fwd_split_kernel(AttnParams p) {
       float down = 1.f;         // what oacc is scaled by for this block's V
       if (ve > kWideBlock) {
         if (ve > vexp) {
+          // further down, oacc would leave fp32's range itself
+          redo |= vexp != kNoV && ve - vexp > kMaxRise;
           down = vexp - ve < -126 ? 0.f : pow2i(vexp - ve);
           vexp = ve;
         }
