@@ -612,7 +612,7 @@ void attn_fwd_split_kernel(AttnParams p) {
       // S^T of both key halves: the small products (hi lo, lo hi) first, so
       // only the D / 16 hi hi MFMAs round at the size of S
       floatx16 s[2] = {floatx16{0}, floatx16{0}};
-      if constexpr (true) __builtin_amdgcn_s_setprio(1);
+      __builtin_amdgcn_s_setprio(1);
       {
         halfx8 a[4 * ND];
         // operands 0 .. 4 ND - 1: (lo, hi) of both halves per k-step, then hi again (b)
@@ -651,7 +651,7 @@ void attn_fwd_split_kernel(AttnParams p) {
           }
         }
       }
-      if constexpr (true) __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_setprio(0);
       if ((now.y & 3u) != kKindNone) {
         const uint32_t keep = block_keep_bits(p, now.x, now.y, my_tile_row, my_row, t.nrows, h, relw);
 #pragma unroll
