@@ -583,6 +583,33 @@ def test_fp32_split_outliers(kind, D, gpu):
             assert ((a - b).abs()[sel] <= 2e-5 * size[sel]).all(), kind
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_fp32_split_v_rise(D, gpu, monkeypatch):
+    """The last V blocks 2^130 above the others, attended by some rows of a
+    tile only: the other rows keep their result.  Frames of 192 tokens lie on
+    the key blocks; a tile holds rows of frames 6 and 7, frame 7 attends the
+    last frame and frame 6 does not."""
+    T, P, H = 9, 192, 2
+    N = T * P
+    m = _meta(T, P, 1, 1, None)
+    rows = om.build_frame_mask(T, P, 1, 1, None).rows
+    assert 8 in rows[7] and 8 not in rows[6] and 7 * P % 128 == 64
+    q, k, v = (x.to(gpu) for x in _draw([(1, N, H, D)] * 3, seed=D, dtype=torch.float32))
+    monkeypatch.setenv("LVSA_VIDEO_SPLIT", "0")   # no part that holds the last frame alone
+    v *= 2.0 ** -65
+    v[:, 8 * P:] *= 2.0 ** 65
+    v[:, 8 * P:] *= 2.0 ** 65
+    plan = m.full_plan(gpu, N, N, 0, 0, D, torch.float32)
+    split = hip_ops.attn_fwd(q, k, v, plan)[0][0, 7 * P - 64:7 * P].double()
+    plain = hip_ops.attn_fwd(q, k, v, plan, scratch=False)[0][0, 7 * P - 64:7 * P].double()
+    seen = torch.cat([torch.arange(f * P, (f + 1) * P) for f in sorted(rows[6])]).to(gpu)
+    for h in range(H):
+        s = q[0, 7 * P - 64:7 * P, h].double() @ k[0, seen, h].double().T / D ** 0.5
+        want = torch.softmax(s, -1) @ v[0, seen, h].double()
+        err = [((x[:, h] - want).norm() / want.norm()).item() for x in (split, plain)]
+        assert err[0] <= 1.01 * err[1], err
+
+
 def test_fp32_smaller_workspace_runs_the_fp32_kernel(gpu):
     """A workspace too small for the split operands (1 KiB was enough for any
     fp32 call) still runs, on the fp32 MFMAs: bit for bit the call without."""
