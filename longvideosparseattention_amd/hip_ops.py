@@ -512,8 +512,12 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan,
             capi.check("lvsa_attn_workspace_query", rc)
         if ws_bytes.value > 0:
             # work-queue counters (zeroed by the call), partials, fp32 pairs
-            ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=device)
-            a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes.value
+            # (as large as K and V); short of memory, the call runs without
+            try:
+                ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=device)
+                a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes.value
+            except torch.cuda.OutOfMemoryError:
+                pass
     _call(device, "lvsa_attn_fwd", C.byref(a))
     return call.out, call.out_t, call.lse, call.lse_t
 

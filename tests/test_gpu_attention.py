@@ -625,6 +625,28 @@ def test_fp32_smaller_workspace_runs_the_fp32_kernel(gpu):
     assert torch.equal(call.out, want)
 
 
+def test_fp32_without_memory_for_the_scratch(gpu):
+    """Where memory for the fp16 pairs of K and V is short, an fp32 call runs
+    without them (on the fp32 MFMAs) instead of failing."""
+    T, P, H, D = 16, 1024, 8, 128
+    m = _meta(T, P, 1, 1, 4, 1)
+    q, k, v = (x.to(gpu) for x in _draw([(1, T * P, H, D)] * 3, dtype=torch.float32))   # 64 MiB each
+    plan = m.full_plan(gpu, T * P, T * P, 0, 0, D, torch.float32)
+    want = hip_ops.attn_fwd(q, k, v, plan, scratch=False)[0]
+    out = torch.empty_like(q)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    limit = torch.cuda.memory_reserved(gpu) + (64 << 20)
+    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(gpu).total_memory, gpu)
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            torch.empty(128 << 20, dtype=torch.uint8, device=gpu)
+        hip_ops.attn_fwd(q, k, v, plan, out=out)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    assert torch.equal(out, want)
+
+
 def test_fp32_wrapper_and_prefill(gpu):
     """fp32 through the block-sparse wrapper (planned for fp16, run in fp32:
     the wrapper re-plans for 128-row tiles) and the dense prefill."""
