@@ -241,6 +241,7 @@ class _DeviceState:
     """
 
     mask: hip_ops.DeviceMask
+    pattern: Tuple = ()                                    # LVSAMetadata._pattern() of the mask
     plans: Dict[Tuple, hip_ops.BlockPlan] = field(default_factory=dict)
     ready: Optional[torch.cuda.Event] = None
     version: int = 0
@@ -356,6 +357,12 @@ class LVSAMetadata:
     _attended_rows: List[List[int]] = field(default_factory=list, repr=False)
     _device_state: Dict[str, _DeviceState] = field(default_factory=dict, repr=False)
     _home_device: Optional[torch.device] = field(default=None, repr=False)
+    _built_pattern: Tuple = field(default=(), repr=False)   # the pattern that build derived the fields of
+
+    def _pattern(self) -> Tuple:
+        return (self.total_latent_frames, self.num_patches, self.window_size, self.n_first_frames,
+                self.key_frame_interval, self.keyframe_offset, self.expand_window, self.rank, self.world,
+                tuple(self.boundary_guards), self.max_row_frames)
 
     @classmethod
     @torch.compiler.disable
@@ -459,7 +466,7 @@ class LVSAMetadata:
                 lcop.append((fr * P - gts, ci * P))
 
         gmask = torch.tensor(list(is_global), dtype=torch.int8)
-        return cls(
+        m = cls(
             total_latent_frames=T, num_patches=P, window_size=W, n_first_frames=n_first_frames,
             key_frame_interval=kfi, expand_window=expand_window, rank=rank, world=world,
             local_seq=local_seq, global_token_start=gts, global_indices=G, global_set=Gs,
@@ -471,6 +478,8 @@ class LVSAMetadata:
             keyframe_offset=keyframe_offset, boundary_guards=guards, fi_nnz=nnz,
             max_row_frames=row_max, _attended_rows=attended_rows,
         )
+        m._built_pattern = m._pattern()
+        return m
 
     # ── Lazily materialised tables of the reference API ──
 
@@ -534,7 +543,7 @@ class LVSAMetadata:
         key = str(device)
         st = self._device_state.get(key)
         if st is None:
-            st = _DeviceState(hip_ops.mask_build(self._mask_params(), device))
+            st = _DeviceState(hip_ops.mask_build(self._mask_params(), device), self._pattern())
             st.built(device)
             self._device_state[key] = st
         st.join(device)
@@ -584,7 +593,7 @@ class LVSAMetadata:
                 q_frame0=gts // P, max_row_frames=max(1, 2 * self.window_size + 1), block_q=block_q)
             # rel_window holds at most 2W + 1 frames per row and every other tile list is
             # bounded by its blocks, so the capacity is exact: nothing to read back
-            plan._verified = True
+            plan._verified |= st.pattern == self._pattern()
             st.plans[key] = plan
             st.built(st.mask.info.device)
         return plan
@@ -604,8 +613,9 @@ class LVSAMetadata:
             plan = hip_ops.plan_build(
                 st.mask.rel_full, n_q=n_q, n_k=n_k, n_x=n_text_k, n_tq=n_text_q, R=P, Cf=P,
                 max_row_frames=max(1, self.max_row_frames), block_q=block_q)
-            # max_row_frames is the longest row of this pattern: the capacity is exact
-            plan._verified = True
+            # max_row_frames is the longest row of the pattern that build derived it for: the capacity is
+            # exact there (not on an instance whose fields were replaced)
+            plan._verified |= st.pattern == self._pattern() == self._built_pattern
             st.plans[key] = plan
             st.built(st.mask.info.device)
         return plan

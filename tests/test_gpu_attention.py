@@ -8,6 +8,7 @@ k, v, shapes [B, N, H, D], rounded to the compute dtype.
 """
 
 import ctypes as C
+import dataclasses
 import math
 
 import pytest
@@ -1211,6 +1212,17 @@ def test_plan_overflow_and_block_k_are_rejected(gpu):
     good = hip_ops.plan_build(st.mask.rel_full, n_q=T * P, n_k=T * P, R=P, Cf=P, max_row_frames=m.max_row_frames)
     out, _, _, _ = hip_ops.attn_fwd(q, k, v, good)
     assert torch.equal(out, lv.lvsa_attention(q, k, v, m))
+
+
+@pytest.mark.parametrize("change", [dict(window_size=9), dict(max_row_frames=1), dict(n_first_frames=20)], ids=str)
+def test_replaced_metadata_fields_cannot_truncate_a_plan(change, gpu):
+    """Fields replaced on a built instance leave max_row_frames behind: the
+    plan's capacity is checked, as for any other caller of plan_build."""
+    T, P, H, D = 24, 300, 2, 128
+    m = dataclasses.replace(_meta(T, P, 1, 1, 8, 1), _device_state={}, **change)
+    q, k, v = (x.to(gpu) for x in _draw([(1, T * P, H, D)] * 3))
+    with pytest.raises(RuntimeError, match="exceed the capacity"):
+        lv.lvsa_attention(q, k, v, m)
 
 
 def test_wrapper_rejects_out_of_range_columns(gpu):
