@@ -435,9 +435,7 @@ __device__ int tile_count(const PlanCtx& c, int t) {
 // tile walking its ~400 entries took 146 us for 13 frames of 1350 tokens (35
 // us for 33 of 256), which every new pattern waits for.
 template <bool kFill>
-__global__ __launch_bounds__(kPlanThreads) void plan_tiles_kernel(PlanCtx c, int32_t* indptr, uint32_t* entries,
-                                                                  int64_t cap) {
-  const int t = blockIdx.x;
+__device__ __forceinline__ void plan_tile(const PlanCtx& c, int t, int32_t* indptr, uint32_t* entries, int64_t cap) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int64_t begin = kFill ? (int64_t)indptr[t] : 0;
   const int64_t end = kFill ? (int64_t)indptr[t + 1] : 0;
@@ -494,6 +492,16 @@ __global__ __launch_bounds__(kPlanThreads) void plan_tiles_kernel(PlanCtx c, int
   if (kFill)
     for (int j = tid; j < c.nxc; j += kPlanThreads) emit(count + j, kSrcExtra | (uint32_t)j, dense_desc(c, c.p.n_x, j));
   if (!kFill && tid == 0) indptr[t + 1] = (int32_t)(count + c.nxc);
+}
+
+// A launch holds at most 2^32 threads, so plans of more than kPlanGrid tiles
+// (tiles of a few rows) take several per work-group.
+constexpr uint32_t kPlanGrid = 1u << 22;
+template <bool kFill>
+__global__ __launch_bounds__(kPlanThreads) void plan_tiles_kernel(PlanCtx c, int32_t* indptr, uint32_t* entries,
+                                                                  int64_t cap) {
+  for (uint32_t t = blockIdx.x; t < (uint32_t)(c.n_vt + c.n_tt); t += gridDim.x)
+    plan_tile<kFill>(c, (int)t, indptr, entries, cap);
 }
 
 // Row pointers from per-tile counts, clamped to the entry capacity
@@ -735,17 +743,18 @@ int lvsa_plan_build(const lvsa_plan_params* p, int32_t* tile_indptr, uint32_t* e
     return launch_status("lvsa_plan_build");
   }
   int32_t* status = (int32_t*)workspace;
+  const dim3 grid((uint32_t)n < kPlanGrid ? (uint32_t)n : kPlanGrid);
   if (n <= kCountTiles && (c.n_vt == 0 || (p->block_q - 1) / p->R + 2 <= kCountFrames)) {
     hipLaunchKernelGGL(plan_scan_kernel<true>, dim3(1), dim3(kScanThreads), 0, stream, c, tile_indptr, n, max_entries,
                        status);
   } else {
-    hipLaunchKernelGGL(plan_tiles_kernel<false>, dim3((unsigned)n), dim3(kPlanThreads), 0, stream, c, tile_indptr,
-                       entries, max_entries);
+    hipLaunchKernelGGL(plan_tiles_kernel<false>, grid, dim3(kPlanThreads), 0, stream, c, tile_indptr, entries,
+                       max_entries);
     hipLaunchKernelGGL(plan_scan_kernel<false>, dim3(1), dim3(kScanThreads), 0, stream, c, tile_indptr, n, max_entries,
                        status);
   }
-  hipLaunchKernelGGL(plan_tiles_kernel<true>, dim3((unsigned)n), dim3(kPlanThreads), 0, stream, c, tile_indptr,
-                     entries, max_entries);
+  hipLaunchKernelGGL(plan_tiles_kernel<true>, grid, dim3(kPlanThreads), 0, stream, c, tile_indptr, entries,
+                     max_entries);
   return launch_status("lvsa_plan_build");
 }
 

@@ -200,6 +200,17 @@ def test_plan_block_lists(T, P, W, kfi, bq, bk, gpu):
     assert (plan.entries[: indptr[-1], 0].cpu().numpy().astype(np.int64) & 0x7FFFFFFF).tolist() == cols
 
 
+def test_plan_of_more_tiles_than_a_launch_holds(gpu):
+    """2^24 + 3 tiles of one row over one key block: 2^32 threads and more at
+    a work-group of 256 per tile, so work-groups take several tiles."""
+    n = (1 << 24) + 3
+    rel = torch.ones(1, 1, dtype=torch.int32, device=gpu)
+    plan = hip_ops.plan_build(rel, n_q=n, n_k=64, R=n, Cf=64, max_row_frames=1, block_q=1, block_k=64)
+    assert plan.n_tiles == n and plan.status[:2].tolist() == [0, n]
+    assert torch.equal(plan.tile_indptr, torch.arange(n + 1, dtype=torch.int32, device=gpu))
+    assert not plan.entries[:n].any()
+
+
 def test_window_golden_arbitrary_global_sets(golden, gpu):
     """The reference's window bounds for 600 arbitrary global sets: each set
     goes in as boundary guards (no anchors, no keyframe grid), so the device's
