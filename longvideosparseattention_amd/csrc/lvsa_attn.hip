@@ -28,12 +28,14 @@ int cu_count() {
   return cached[dev];
 }
 
-// Key blocks of a video tile, guessed (the plan's counts are on the device):
-// about six frames of anchors and window and a keyframe in eight, and the
-// extra rows.  Only balance depends on it.
-int64_t guessed_tile_blocks(const lvsa_attn_args* a) {
-  const int64_t C = a->C > 0 ? a->C : 1, frames = ceil_div(a->n_k, C);
-  const int64_t attended = 6 + ceil_div(frames, 8);
+// Key blocks of a video tile of `rows` rows, guessed (the plan's counts are on
+// the device): about six frames of anchors and window and a keyframe in eight,
+// one more for each further query frame of the tile, and the extra rows.  Only
+// balance depends on it.
+int64_t guessed_tile_blocks(const lvsa_attn_args* a, int rows) {
+  const int64_t C = a->C > 0 ? a->C : 1, R = a->R > 0 ? a->R : 1, frames = ceil_div(a->n_k, C);
+  const int64_t more = rows % R == 0 || R % rows == 0 ? ceil_div(rows, R) - 1 : ceil_div(rows - 1, R);
+  const int64_t attended = 6 + ceil_div(frames, 8) + more;
   const int64_t all = ceil_div(a->n_k, kBN);
   const int64_t b = attended < frames ? ceil_div(attended * C, kBN) : all;
   return (b < all ? b : all) + ceil_div(a->n_x, kBN);
@@ -43,11 +45,10 @@ int64_t guessed_tile_blocks(const lvsa_attn_args* a) {
 // third of a Wan / HunyuanVideo video tile and below a CogVideoX one, so the
 // chunks fill the launch's last round at a granularity finer than a tile
 // (64 measured the same at CogVideoX and 0.3% slower at HunyuanVideo).
-// Text tiles of one such chunk beside shorter video tiles run in chunks as
-// long as those (at least kMinTextChunkBlocks), unless that takes more than
-// kMaxSmallText of scratch or than the caller's: 24 frames of 130 tokens, 12
-// heads, 37 text tokens ran its one 50-block text tile per head whole, three
-// times as long as its video tiles (69.6 us per call, 59.1 in chunks).
+// Text tiles of one such chunk beside shorter video tiles may run in chunks as
+// long as those (at least kMinTextChunkBlocks, wanted_text_chunks), where
+// split_of finds that to end the launch sooner and they take at most
+// kMaxSmallText of scratch and the caller's.
 constexpr int kTextChunkBlocks = 128, kMinTextChunkBlocks = 16;
 constexpr int kMaxTextChunks = 64;
 constexpr int64_t kMaxSmallText = 16LL << 20;
@@ -57,13 +58,13 @@ int64_t text_ws_bytes(const lvsa_attn_args* a, int chunks) {
   return 4 * (text_ws_o_elems(chunks, a->B, a->H, a->n_tq, a->D) + 2LL * chunks * a->B * a->H * a->n_tq);
 }
 
-// Text chunks per text tile (1 = no split).
-int text_chunks_of(const lvsa_attn_args* a) {
+// Most text chunks per text tile (1 = no split).
+int wanted_text_chunks(const lvsa_attn_args* a) {
   if (a->n_tq == 0) return 1;
   const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
   const int64_t c = ceil_div(blocks, kTextChunkBlocks);
   if (c <= 1 && a->n_q > 0) {
-    const int64_t tile = guessed_tile_blocks(a);
+    const int64_t tile = guessed_tile_blocks(a, 1);
     const int f = (int)ceil_div(blocks, tile > kMinTextChunkBlocks ? tile : kMinTextChunkBlocks);
     if (text_ws_bytes(a, f) <= kMaxSmallText) return f < 1 ? 1 : f;
   }
@@ -74,7 +75,7 @@ int text_chunks_of(const lvsa_attn_args* a) {
 // tiles in 16 bit.
 int text_chunks_least(const lvsa_attn_args* a) {
   const int64_t blocks = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN);
-  return a->dtype == LVSA_FP32 || blocks <= kTextChunkBlocks ? 1 : text_chunks_of(a);
+  return a->dtype == LVSA_FP32 || blocks <= kTextChunkBlocks ? 1 : wanted_text_chunks(a);
 }
 
 // The video split of a call: `tiles` tiles of `rows` rows per queue in `parts`
@@ -119,15 +120,8 @@ Scratch scratch_of(const lvsa_attn_args* a, int chunks, VideoSplit v, int64_t sl
   if (slots) s.bytes = s.split + f32_split_bytes(slots, a->D);
   return s;
 }
-VideoSplit video_split_of(const lvsa_attn_args* a);
-// What lvsa_attn_workspace_query asks for, and the least that a workspace must
-// be (whole tiles, fp32 on the fp32 MFMAs).
 Scratch scratch_least(const lvsa_attn_args* a) { return scratch_of(a, text_chunks_least(a), VideoSplit{}, 0); }
-Scratch scratch_full(const lvsa_attn_args* a, bool video_split = true) {
-  const int64_t slots = f32_split_slots(a);
-  if (a->dtype == LVSA_FP32 && slots == 0) return scratch_least(a);
-  return scratch_of(a, text_chunks_of(a), video_split ? video_split_of(a) : VideoSplit{}, slots);
-}
+Scratch scratch_full(const lvsa_attn_args* a, bool video_split = true);
 
 // Zero the work-queue counters (a kernel, not a memset, so the call can be
 // captured in a HIP graph and replayed).
@@ -158,7 +152,7 @@ bool no_key_split() {
 // tiles whole.
 int64_t queue_fill(const lvsa_attn_args* a, int rows) {
   return ceil_div(ceil_div(a->n_q, rows) * a->H * a->B, kXcds) +
-         ceil_div(ceil_div(a->n_tq, rows) * text_chunks_of(a) * a->H * a->B, kXcds);
+         ceil_div(ceil_div(a->n_tq, rows) * wanted_text_chunks(a) * a->H * a->B, kXcds);
 }
 
 // Which kernel a call runs, and on tiles of how many rows.
@@ -236,73 +230,164 @@ Route route_of(const lvsa_attn_args* a) {
   return r;
 }
 
-// Work-groups of the call's kernel that run at once.  fp32: one per CU with
-// two key groups for at most that many items (launch_f32).
-int64_t concurrent_groups(const lvsa_attn_args* a, const Route& r, int64_t cus, int64_t vwork) {
-  if (a->dtype == LVSA_FP32) {
-    const int64_t work = vwork + ceil_div(a->n_tq, r.rows) * text_chunks_of(a) * a->H * a->B;
-    return cus * (work <= cus ? 1 : a->D == 64 ? 3 : a->D <= 128 ? 2 : 1);
-  }
-  return cus * (!r.stream && r.rows == kBM && a->D <= 128 ? 2 : r.per_cu);
+// Launches of this many rounds of work-groups gain nothing from a finer last
+// round, nor from short text tiles in chunks.
+constexpr int kSplitRounds = 5;
+constexpr int kMaxParts = 8;
+constexpr int64_t kMaxVideoSplitBytes = 48LL << 20;
+
+// What a call splits.
+struct Split {
+  int chunks;
+  VideoSplit v;
+};
+
+// Work-groups per CU of the call's kernel for that many items.  fp32: one
+// with two key groups for at most an item per CU (launch_f32).
+int groups_per_cu(const lvsa_attn_args* a, const Route& r, int64_t items, int64_t cus) {
+  if (items <= cus) return 1;
+  if (a->dtype == LVSA_FP32) return a->D == 64 ? 3 : a->D <= 128 ? 2 : 1;
+  return !r.stream && r.rows == kBM && a->D <= 128 ? 2 : r.per_cu;
 }
 
-// Video tiles that run as parts of their key ranges at the end of the launch,
-// so that its last round is finer than whole tiles.  None with
-// LVSA_VIDEO_SPLIT=0.
+// Microseconds per key block of an item with per_cu items on its CU, as
+// measured on launches of one round, tiles of 128 and 256 rows (with x = 1 for
+// 256 rows of D = 128): the single-stream kernel 0.53 to 2.24 (two key groups:
+// 0.54 at D = 128), the 4-wave kernel with masks in every block 1.35 to 2.49,
+// fp32 1.6 to 5.8.
+double block_us(const lvsa_attn_args* a, const Route& r, int per_cu) {
+  const double x = r.rows * a->D / 32768.0;
+  if (a->dtype == LVSA_FP32) return (0.15 + 5.3 * x) * per_cu;
+  if (!r.stream && r.rows == kBM) return per_cu == 1 ? 0.55 + 2.0 * x : 0.73 + 2.5 * x;
+  return (0.2 + 1.4 * x) * per_cu * (r.pairs ? 0.62 : 1.0);
+}
+
+// Estimated microseconds of a launch with the split s: the longest queue's
+// items in their order, each taken by the first CU that is free (without the
+// work queues an XCD runs its own items too: 124 tiles in two parts and 8 text
+// chunks, 33 on an XCD of 32 CUs: 151 us).  Work-groups that share a CU count
+// as one after the other (alone on it each runs nearly as much faster), but
+// the longest item takes its time beside another.  8 us to start and end a
+// launch and 5 per item; a merge 3, and its partials once each way at 4.6
+// TB/s.
+double launch_us(const lvsa_attn_args* a, const Route& r, int64_t cus, const Split& s) {
+  const int64_t all = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN), tile = guessed_tile_blocks(a, r.rows);
+  const int64_t videos = ceil_div(ceil_div(a->n_q, r.rows) * a->H * a->B, kXcds);
+  const int64_t texts = ceil_div(ceil_div(a->n_tq, r.rows) * s.chunks * a->H * a->B, kXcds);
+  const int64_t split = s.v.tiles < videos ? s.v.tiles : videos;
+  struct Items {
+    int64_t n, blocks;
+  } items[4] = {{s.chunks == 1 ? texts : 0, all},
+                {videos - split, tile},
+                {split * s.v.parts, s.v.parts ? ceil_div(tile, s.v.parts) : 0},
+                {s.chunks == 1 ? 0 : texts, ceil_div(all, s.chunks)}};
+  const int per_cu = groups_per_cu(a, r, kXcds * (texts + videos + split * (s.v.parts - 1)), cus);
+  const double per_item = 5.0 / per_cu, per_block = block_us(a, r, per_cu) / per_cu;
+  // CUs by the time at which they are free, ascending: a class of
+  // equal items adds one time at most
+  struct Free {
+    double t;
+    int64_t n;
+  } free[6] = {{0.0, cus / kXcds > 0 ? cus / kXcds : 1}};
+  int nf = 1;
+  double end = 0.0;
+  for (const Items& it : items) {
+    const double us = per_item + it.blocks * per_block;
+    if (it.n > 0 && us * per_cu > end) end = us * per_cu;
+    for (int64_t left = it.n; left > 0;) {
+      const int64_t x = left < free[0].n ? left : free[0].n;
+      const double t = free[0].t + us;
+      left -= x;
+      end = t > end ? t : end;
+      if (x == free[0].n) {
+        for (int i = 1; i < nf; ++i) free[i - 1] = free[i];
+        --nf;
+      } else {
+        free[0].n -= x;
+      }
+      int at = nf;
+      while (at > 0 && free[at - 1].t > t) --at;
+      if (at > 0 && free[at - 1].t == t) {
+        free[at - 1].n += x;
+        continue;
+      }
+      for (int i = nf; i > at; --i) free[i] = free[i - 1];
+      free[at] = {t, x};
+      ++nf;
+    }
+  }
+  return 8.0 + end + (s.v.tiles > 0 ? 3.0 + video_ws_bytes(a, s.v) / 2.3e6 : 0.0) +
+         (s.chunks > 1 ? 3.0 + text_ws_bytes(a, s.chunks) / 2.3e6 : 0.0);
+}
+
+// The split of a call: text chunks, and video tiles that run as parts of their
+// key ranges at the end of the launch (none with LVSA_VIDEO_SPLIT=0), so that
+// its last round is finer than whole tiles.
+// - Long text tiles always run in chunks.
 // - The dual map over the work queues: its two work-groups per CU take whole
 //   tiles at half the CU's rate, so a last round of whole tiles leaves CUs
 //   idle for longer.  As many tiles per queue as the queue has work-groups on
 //   its XCD, halved (32), in two parts (CogVideoX 0.9% faster).
-// - Otherwise launches of fewer than kSplitRounds rounds, whose last round is
-//   not full: its tiles in the number of parts that ends soonest by a model of
-//   the last round (below), where that saves 7% and 5 us of it.  33 frames of 390
-//   tokens, 12 heads, D = 128 (612 tiles, 2.4 rounds): 383 -> 338 us and 10
-//   for the merge; 9 frames of 256 (108 tiles, one round): 46 -> 36 + 10, so
-//   whole.  Longer launches gain little from their last round and pay the same
-//   merge (Wan 4x and HunyuanVideo, 24 and 20 rounds, within +-0.5%).
-constexpr int kSplitRounds = 5, kMaxParts = 8;
-constexpr int64_t kMaxVideoSplitBytes = 48LL << 20;
-VideoSplit video_split_of(const lvsa_attn_args* a) {
-  VideoSplit v;
+// - Otherwise launches of fewer than kSplitRounds rounds: the tiles of a last
+//   round that is not full in the number of parts, and short text tiles in
+//   chunks, that end the launch soonest (launch_us), where parts save 6 us and
+//   6% of it (chunks alone 3 us and 4%).  33 frames of 390 tokens, 12 heads,
+//   D = 128 (612 tiles, 2.4 rounds): 383 -> 338 us and 10 for the merge; 9
+//   frames of 256 (108 tiles, one round): 46 -> 36 + 10, so whole; 33 frames
+//   of 400, 6 heads, 40 text tokens: 247 us whole and 272 in parts, beside
+//   which the text chunks are the longest items.  24 frames of 130, 12 heads,
+//   D = 128, 37 text tokens ran its one 50-block text tile per head whole,
+//   three times as long as its video tiles (69.6 us, 59.1 in chunks); 13
+//   frames of 600, 24 heads, D = 64, 226 text tokens take 261 us with whole
+//   text tiles, first in the launch, and 295 with chunks at its end.  Longer
+//   launches gain little from their last round and pay the same merge (Wan 4x
+//   and HunyuanVideo, 24 and 20 rounds, within +-0.5%).
+Split split_of(const lvsa_attn_args* a, const Route& r, bool video) {
+  const int want = wanted_text_chunks(a);
+  const bool long_text = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN) > kTextChunkBlocks || a->n_q == 0;
+  Split best{long_text ? want : 1, VideoSplit{}};
   const int64_t cus = cu_count();
-  if (no_key_split() || a->n_q == 0 || a->block_q <= 0 || a->block_q == kStream12BM || cus <= 0) return v;
-  const Route route = route_of(a);
-  const int64_t vwork = ceil_div(a->n_q, route.rows) * a->H * a->B;
-  const int64_t groups = concurrent_groups(a, route, cus, vwork);
-  if (route.dual) {
-    const int64_t work = vwork + ceil_div(a->n_tq, route.rows) * text_chunks_of(a) * a->H * a->B;
-    if (work > groups) {
-      const int64_t s = groups / (2 * kXcds), per_queue = ceil_div(vwork, kXcds);
-      v.tiles = (int)(s < per_queue ? s : per_queue);
-      v.parts = 2;
-      v.rows = route.rows;
-      return v;
+  if (a->n_q == 0 || cus <= 0) return best;
+  const int64_t vwork = ceil_div(a->n_q, r.rows) * a->H * a->B;
+  const int64_t twork = ceil_div(a->n_tq, r.rows) * a->H * a->B;
+  const int64_t groups = cus * groups_per_cu(a, r, vwork + twork * want, cus);
+  video = video && !no_key_split() && a->block_q != kStream12BM;
+  const bool dual = video && r.dual && vwork + twork > groups;
+  if (dual) {
+    const int64_t s = groups / (2 * kXcds), per_queue = ceil_div(vwork, kXcds);
+    best.v = VideoSplit{(int)(s < per_queue ? s : per_queue), 2, r.rows};
+  }
+  const int64_t blocks = guessed_tile_blocks(a, r.rows);
+  const int64_t rest = vwork % cus;
+  const int most = dual || !video || rest == 0 ? 1 : (int)(blocks / 6 < kMaxParts ? blocks / 6 : kMaxParts);
+  if (vwork >= kSplitRounds * groups || (most < 2 && (long_text || want == 1))) return best;
+  const double whole = launch_us(a, r, cus, best);
+  auto margin = [whole](double us, double share) { return us > share * whole ? us : share * whole; };
+  double least = whole;
+  for (int chunks = best.chunks, more = 1; more; chunks = want) {
+    more = !long_text && chunks < want;
+    for (int k = 1; k <= most || k == 1; ++k) {
+      Split s{chunks, dual ? best.v : VideoSplit{}};
+      if (k > 1) s.v = VideoSplit{(int)ceil_div(rest, kXcds), k, r.rows};
+      if (k > 1 && video_ws_bytes(a, s.v) > kMaxVideoSplitBytes) break;
+      double t = launch_us(a, r, cus, s);
+      if (k > 1) t += margin(6.0, 0.06);
+      else if (chunks > 1 && !long_text) t += margin(3.0, 0.04);
+      if (t < least) {
+        least = t;
+        best = s;
+      }
     }
   }
-  const int64_t rest = vwork % groups;
-  if (vwork >= kSplitRounds * groups || rest == 0) return v;
-  // Microseconds, as measured on launches of one round: about 1 per key block
-  // (fp32: 2.5 times that, key groups: 0.6), 8 to start and end a launch and 5
-  // per item; the merge 3 and its partials at 3 TB/s.  Rounds are those of the
-  // longest queue: without the work queues an XCD runs its own items only (124
-  // tiles in two parts and 8 text chunks, 33 on an XCD of 32 CUs: 151 us).
-  const double block_us = (0.75 + 0.3 * route.rows * a->D / 32768.0) *
-                          (a->dtype == LVSA_FP32 ? 2.5 : route.pairs ? 0.6 : 1.0);
-  const int64_t text_fill = ceil_div(ceil_div(a->n_tq, route.rows) * text_chunks_of(a) * a->H * a->B, kXcds);
-  const int64_t blocks = guessed_tile_blocks(a);
-  const double whole = 8.0 + blocks * block_us + 5.0;
-  double best = whole - (5.0 > 0.07 * whole ? 5.0 : 0.07 * whole);
-  for (int k = 2; k <= kMaxParts && blocks >= 6 * k; ++k) {
-    const VideoSplit w{(int)ceil_div(rest, kXcds), k, route.rows};
-    const int64_t bytes = video_ws_bytes(a, w);
-    const int64_t rounds = ceil_div((w.tiles * k + text_fill) * kXcds, groups);
-    const double t = 8.0 + rounds * (blocks * block_us / k + 5.0) + 3.0 + bytes / 3e6;
-    if (t < best && bytes <= kMaxVideoSplitBytes) {
-      best = t;
-      v = w;
-    }
-  }
-  return v;
+  return best;
+}
+
+Scratch scratch_full(const lvsa_attn_args* a, bool video_split) {
+  const int64_t slots = f32_split_slots(a);
+  if (a->dtype == LVSA_FP32 && slots == 0) return scratch_least(a);
+  if (a->block_q <= 0) return scratch_of(a, text_chunks_least(a), VideoSplit{}, slots);
+  const Split s = split_of(a, route_of(a), video_split);
+  return scratch_of(a, s.chunks, s.v, slots);
 }
 
 // Exact log-sum-exp merge of the text chunks (lvsa-vllm-omni/lvsa_vllm_omni/

@@ -1031,10 +1031,46 @@ def test_work_queues_match_static_grid(cfg, gpu, monkeypatch):
         _close(ot1[:1], rto, "queued text rows")
 
 
+def _scratch_bytes(q, k, v, m, kt=None, vt=None, qt=None):
+    """What lvsa_attn_workspace_query asks for the fused call."""
+    n_t = 0 if kt is None else kt.shape[1]
+    plan = m.full_plan(q.device, q.shape[1], k.shape[1], n_t, 0 if qt is None else n_t, q.shape[3], q.dtype)
+    call = hip_ops.attn_args(q, k, v, plan, kx=kt, vx=vt, qt=qt)
+    n = C.c_int64()
+    capi.check("lvsa_attn_workspace_query", capi.lib().lvsa_attn_workspace_query(C.byref(call.args), C.byref(n)))
+    return n.value
+
+
+def _partials(tiles, parts, rows, D):
+    """Bytes of the video split's partials."""
+    return 8 * tiles * parts * rows * (D + 2) * 4
+
+
+@pytest.mark.parametrize("cfg,want", [
+    # T, P, W, kfi, H, Hkv, D, n_txt: partials in bytes (256 compute units)
+    ((13, 600, 1, 4, 24, 24, 64, 226), _partials(32, 2, 256, 64)),       # the dual map's halves, text tiles whole
+    ((6, 300, 1, 4, 12, 6, 96, 11), 0),                             # the text tile is as long as the video tiles
+    ((24, 445, 1, 8, 8, 8, 128, 123), 2 * 8 * 123 * (128 + 2) * 4),  # long text in two chunks, no parts beside them
+    ((6, 390, 2, 4, 12, 12, 128, 200), 0),
+    ((24, 130, 2, 8, 12, 12, 128, 37), 3 * 12 * 37 * (128 + 2) * 4),  # a text tile three times as long: chunks
+    ((33, 390, 2, 8, 12, 12, 128, 0), _partials(13, 2, 256, 128)),       # 100 tiles in the last round: halves
+], ids=str)
+def test_splits_only_where_the_launch_ends_sooner(cfg, want, gpu):
+    """Text chunks and key-range parts by the scratch that a call asks for.
+    The calls without were 6% to 40% slower with them."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("counts of a GPU of 256 compute units")
+    T, P, W, kfi, H, Hkv, D, n_txt = cfg
+    m = _meta(T, P, W, 1, kfi, 1)
+    q, k, v = (torch.empty(1, T * P, h, D, dtype=torch.bfloat16, device=gpu) for h in (H, Hkv, Hkv))
+    text = [torch.empty(1, n_txt, h, D, dtype=torch.bfloat16, device=gpu) for h in (Hkv, Hkv, H)] if n_txt else []
+    assert _scratch_bytes(q, k, v, m, *text) == -(-want // 256) * 256 + 1024
+
+
 PARTS = [
     # T, P, H, Hkv, D, n_txt, dtype: fewer rounds than kSplitRounds with a part-filled last one
     (9, 512, 2, 1, 128, 0, torch.bfloat16),     # the half map on a 256-row plan, no queues
-    (33, 400, 6, 6, 128, 40, torch.float16),    # 312 tiles: the work queues, text chunks
+    (25, 300, 12, 12, 128, 40, torch.float16),  # 360 tiles: the work queues, text chunks
     (9, 600, 2, 1, 64, 0, torch.bfloat16),      # the half map of D = 64
     (9, 600, 3, 3, 96, 5, torch.bfloat16),
     (9, 500, 4, 2, 192, 0, torch.bfloat16),     # dual-wide map
@@ -1059,7 +1095,11 @@ def test_video_tiles_in_parts(cfg, gpu, monkeypatch):
         seed=33, dtype=dt))
     kw = dict(k_text=kt, v_text=vt, q_text=qt) if n_txt else {}
     parts = lv.lvsa_attention(q, k, v, m, return_lse=True, **kw)
+    text = (kt, vt, qt) if n_txt else ()
+    split = _scratch_bytes(q, k, v, m, *text)
     monkeypatch.setenv("LVSA_VIDEO_SPLIT", "0")
+    # (the outputs can differ without parts: LVSA_VIDEO_SPLIT=0 also turns the two key groups off)
+    assert split >= _scratch_bytes(q, k, v, m, *text) + _partials(1, 2, 128, D), "no tile is split"
     whole = lv.lvsa_attention(q, k, v, m, return_lse=True, **kw)
     assert not torch.equal(parts[0], whole[0]), "no tile was split"
     # one rounding of the output type (|O| < 1) each; fp32: a few of the merge
