@@ -250,6 +250,14 @@ int groups_per_cu(const lvsa_attn_args* a, const Route& r, int64_t items, int64_
   return !r.stream && r.rows == kBM && a->D <= 128 ? 2 : r.per_cu;
 }
 
+// Work-groups of a CU that launch_us lets run side by side.  The single-stream
+// kernel's, alone on a CU, are nearly as much faster (D = 128, 128 rows: 0.9
+// and 1.7 us per block), so they count as one after the other; the 4-wave and
+// the fp32 kernel's are not (1.6 and 2.0; 4 and 5.2).
+int side_by_side(const lvsa_attn_args* a, const Route& r, int per_cu) {
+  return a->dtype == LVSA_FP32 || (!r.stream && r.rows == kBM) ? per_cu : 1;
+}
+
 // Microseconds per key block of an item with per_cu items on its CU, as
 // measured on launches of one round, tiles of 128 and 256 rows (with x = 1 for
 // 256 rows of D = 128): the single-stream kernel 0.53 to 2.24 (two key groups:
@@ -263,13 +271,11 @@ double block_us(const lvsa_attn_args* a, const Route& r, int per_cu) {
 }
 
 // Estimated microseconds of a launch with the split s: the longest queue's
-// items in their order, each taken by the first CU that is free (without the
-// work queues an XCD runs its own items too: 124 tiles in two parts and 8 text
-// chunks, 33 on an XCD of 32 CUs: 151 us).  Work-groups that share a CU count
-// as one after the other (alone on it each runs nearly as much faster), but
-// the longest item takes its time beside another.  8 us to start and end a
-// launch and 5 per item; a merge 3, and its partials once each way at 4.6
-// TB/s.
+// items in their order, each taken by the first work-group that is free
+// (without the work queues an XCD runs its own items too: 124 tiles in two
+// parts and 8 text chunks, 33 on an XCD of 32 CUs: 151 us); the longest item
+// takes its time beside another one.  8 us to start and end a launch and 5 per
+// item; a merge 3, and its partials once each way at 4.6 TB/s.
 double launch_us(const lvsa_attn_args* a, const Route& r, int64_t cus, const Split& s) {
   const int64_t all = ceil_div(a->n_k, kBN) + ceil_div(a->n_x, kBN), tile = guessed_tile_blocks(a, r.rows);
   const int64_t videos = ceil_div(ceil_div(a->n_q, r.rows) * a->H * a->B, kXcds);
@@ -282,18 +288,19 @@ double launch_us(const lvsa_attn_args* a, const Route& r, int64_t cus, const Spl
                 {split * s.v.parts, s.v.parts ? ceil_div(tile, s.v.parts) : 0},
                 {s.chunks == 1 ? 0 : texts, ceil_div(all, s.chunks)}};
   const int per_cu = groups_per_cu(a, r, kXcds * (texts + videos + split * (s.v.parts - 1)), cus);
-  const double per_item = 5.0 / per_cu, per_block = block_us(a, r, per_cu) / per_cu;
-  // CUs by the time at which they are free, ascending: a class of
+  const int side = side_by_side(a, r, per_cu);
+  const double share = (double)side / per_cu, per_item = 5.0 * share, per_block = block_us(a, r, per_cu) * share;
+  // work-groups by the time at which they are free, ascending: a class of
   // equal items adds one time at most
   struct Free {
     double t;
     int64_t n;
-  } free[6] = {{0.0, cus / kXcds > 0 ? cus / kXcds : 1}};
+  } free[6] = {{0.0, cus * side / kXcds > 0 ? cus * side / kXcds : 1}};
   int nf = 1;
   double end = 0.0;
   for (const Items& it : items) {
     const double us = per_item + it.blocks * per_block;
-    if (it.n > 0 && us * per_cu > end) end = us * per_cu;
+    if (it.n > 0 && us > end * share) end = us / share;
     for (int64_t left = it.n; left > 0;) {
       const int64_t x = left < free[0].n ? left : free[0].n;
       const double t = free[0].t + us;
@@ -350,7 +357,8 @@ Split split_of(const lvsa_attn_args* a, const Route& r, bool video) {
   if (a->n_q == 0 || cus <= 0) return best;
   const int64_t vwork = ceil_div(a->n_q, r.rows) * a->H * a->B;
   const int64_t twork = ceil_div(a->n_tq, r.rows) * a->H * a->B;
-  const int64_t groups = cus * groups_per_cu(a, r, vwork + twork * want, cus);
+  const int per_cu = groups_per_cu(a, r, vwork + twork * want, cus);
+  const int64_t groups = cus * per_cu;
   video = video && !no_key_split() && a->block_q != kStream12BM;
   const bool dual = video && r.dual && vwork + twork > groups;
   if (dual) {
@@ -358,7 +366,7 @@ Split split_of(const lvsa_attn_args* a, const Route& r, bool video) {
     best.v = VideoSplit{(int)(s < per_queue ? s : per_queue), 2, r.rows};
   }
   const int64_t blocks = guessed_tile_blocks(a, r.rows);
-  const int64_t rest = vwork % cus;
+  const int64_t rest = vwork % (cus * side_by_side(a, r, per_cu));
   const int most = dual || !video || rest == 0 ? 1 : (int)(blocks / 6 < kMaxParts ? blocks / 6 : kMaxParts);
   if (vwork >= kSplitRounds * groups || (most < 2 && (long_text || want == 1))) return best;
   const double whole = launch_us(a, r, cus, best);
