@@ -643,6 +643,12 @@ extern "C" int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream) {
     p.split = (char*)a->workspace + ws.split;
     p.split_exp = (int32_t*)(p.split + ws.slots * 4LL * kBN * a->D);
   }
+  // Calls without text rows and of fewer query rows than keys (per K/V head)
+  // may leave most of K and V unattended.  Each work-group of the split then
+  // reads the relation rows first (at most 16 KiB of them).
+  const int64_t rel_words = a->n_q > 0 ? ((a->q_tok0 % p.R + a->n_q - 1) / p.R + 1) * (int64_t)a->words : 0;
+  p.split_seen = ws.slots && a->n_tq == 0 && a->n_q > 0 && (int64_t)a->n_q * p.group < a->n_k &&
+                 a->words <= kSeenWords && rel_words <= 4096;
   p.vsplit = ws.v.tiles;
   p.vparts = ws.v.parts;
   p.vws = ws.v.tiles > 0 ? (float*)((char*)a->workspace + ws.video) : nullptr;

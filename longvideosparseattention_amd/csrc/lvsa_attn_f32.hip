@@ -376,16 +376,14 @@ __device__ __forceinline__ bool wide_part(const float (&x)[NF][8], uint32_t belo
   return wide || 4 * all_small > all;
 }
 
-// One slot per work-group.  HBM bound: reads the block once and writes as many
-// bytes; the conversions are a few instructions per number.
+// One slot.  HBM bound: reads the block once and writes as many bytes; the
+// conversions are a few instructions per number.
 template <int D>
-__global__ __launch_bounds__(kThreads) void split_f32_kernel(AttnParams p) {
+__device__ __forceinline__ void split_slot(const AttnParams& p, int slot, float* wmax) {
   constexpr int NF = D / 32;      // fragments per wave
   constexpr int ND = D / 16, NT = D / 32;
-  __shared__ float wmax[kWaves];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h = lane >> 5, i32 = lane & 31;
-  const int slot = blockIdx.x;
   const int nkc = (p.n_k + kBN - 1) / kBN, nbt = nkc + (p.n_x + kBN - 1) / kBN;
   const bool is_v = slot & 1;
   int r = slot >> 1;
@@ -460,6 +458,58 @@ __global__ __launch_bounds__(kThreads) void split_f32_kernel(AttnParams p) {
   if (__ballot(least < below)) wide |= wide_part<NF>(x, below, own_max, !is_v);
   wide = __syncthreads_or(wide);
   if (threadIdx.x == 0) p.split_exp[slot] = amax == 0.f ? kZeroBlock : wide ? kWideBlock : e;
+}
+
+template <int D>
+__global__ __launch_bounds__(kThreads) void split_f32_kernel(AttnParams p) {
+  __shared__ float wmax[kWaves];
+  split_slot<D>(p, blockIdx.x, wmax);
+}
+
+// Whether a tile can list the block of a slot: it holds rows of a key frame in
+// `seen` (a relation row), or extra rows, which every tile lists.
+__device__ __forceinline__ bool slot_seen(const AttnParams& p, int slot, const uint32_t* seen) {
+  const int nkc = (p.n_k + kBN - 1) / kBN, nbt = nkc + (p.n_x + kBN - 1) / kBN;
+  const int blk = (slot >> 1) % nbt;
+  if (blk >= nkc) return true;
+  const uint32_t k0 = (uint32_t)blk * kBN, k1 = k0 + kBN < (uint32_t)p.n_k ? k0 + kBN : (uint32_t)p.n_k;
+  const uint32_t f0 = p.kf0 + (p.ko + k0) / (uint32_t)p.C, f1 = p.kf0 + (p.ko + k1 - 1) / (uint32_t)p.C;
+  bool any = false;
+  for (uint32_t f = f0; f <= f1 && (f >> 5) < (uint32_t)p.words; ++f) any |= (seen[f >> 5] >> (f & 31)) & 1u;
+  return any;
+}
+
+// The same for calls of fewer query rows than keys, which may attend few of
+// them: only the blocks that a tile can list.  A work-group takes every
+// gridDim-th slot and tests 256 of them at a time, a thread each.  One tile
+// that attends 2 of 8,000 blocks (12 heads, D = 128) takes 25 us on the fp32
+// MFMAs, 2,643 with every block split and 34 so; 6 of 800 blocks 62, 293 and
+// 35; 16 tiles of 10 of 800 121, 307 and 95.
+template <int D>
+__global__ __launch_bounds__(kThreads) void split_seen_f32_kernel(AttnParams p) {
+  __shared__ float wmax[kWaves];
+  __shared__ uint32_t seen[kSeenWords];
+  __shared__ uint64_t todo[kWaves];
+  const int tid = threadIdx.x;
+  for (int w = tid; w < p.words; w += kThreads) seen[w] = 0;
+  __syncthreads();
+  const int rows = (int)((p.qo + (uint32_t)(p.n_q - 1)) / (uint32_t)p.R) + 1;
+  for (int i = tid; i < rows * p.words; i += kThreads) {
+    const uint32_t x = p.rel[(int64_t)p.qf0 * p.words + i];
+    if (x) atomicOr(&seen[i % p.words], x);
+  }
+  __syncthreads();
+  for (int64_t s0 = blockIdx.x; s0 < p.split_slots; s0 += (int64_t)gridDim.x * kThreads) {
+    const int64_t mine = s0 + (int64_t)gridDim.x * tid;
+    const uint64_t on = __ballot(mine < p.split_slots && slot_seen(p, (int)mine, seen));
+    if ((tid & 63) == 0) todo[tid >> 6] = on;
+    __syncthreads();
+    for (int w = 0; w < kWaves; ++w) {
+      for (uint64_t m = todo[w]; m; m &= m - 1)
+        split_slot<D>(p, (int)(s0 + (int64_t)gridDim.x * (64 * w + __builtin_ctzll(m))), wmax);
+    }
+    __syncthreads();   // `todo` has been read
+  }
 }
 
 // KG groups of four waves take the tile's key blocks in turn (group g blocks
@@ -813,7 +863,13 @@ int launch_f32_d(const AttnParams& p, int cus, hipStream_t stream) {
     hipLaunchKernelGGL(attn_fwd_f32_kernel<D>, grid, dim3(kThreads), 0, stream, p);
     return launch_status("lvsa_attn_fwd (fp32)");
   }
-  hipLaunchKernelGGL(split_f32_kernel<D>, dim3(p.split_slots), dim3(kThreads), 0, stream, p);
+  if (p.split_seen) {
+    const int groups = 8 * (cus > 0 ? cus : 1);
+    hipLaunchKernelGGL(split_seen_f32_kernel<D>, dim3(p.split_slots < groups ? p.split_slots : groups), dim3(kThreads),
+                       0, stream, p);
+  } else {
+    hipLaunchKernelGGL(split_f32_kernel<D>, dim3(p.split_slots), dim3(kThreads), 0, stream, p);
+  }
   const int rc = launch_status("lvsa_attn_fwd (fp32 split)");
   if (rc != LVSA_OK) return rc;
   if constexpr (D <= 128) {

@@ -103,10 +103,11 @@ struct AttnParams {
   uint32_t* queues;
   int grid;
   // fp32 inputs: K and V split into fp16 pairs (lvsa_attn_f32.hip), split_slots
-  // blocks at `split` with their exponents at split_exp; null: the fp32 kernel
+  // blocks at `split` with their exponents at split_exp; null: the fp32
+  // kernel.  split_seen: only blocks of key frames that some row attends
   char* split;
   int32_t* split_exp;
-  int split_slots;
+  int split_slots, split_seen;
 };
 
 // Bytes of the work-queue counters at the end of the attention workspace.
@@ -132,6 +133,7 @@ int launch_d256(const AttnParams& prm, int block_q, bool bf16, hipStream_t strea
 // compute units; scratch of `slots` split key blocks (their exponents last).
 int launch_f32(const AttnParams& prm, int D, int cus, hipStream_t stream);
 int64_t f32_split_bytes(int64_t slots, int D);
+constexpr int kSeenWords = 1024;   // relation words of the split_seen kernel
 
 namespace {
 

@@ -626,6 +626,33 @@ def test_fp32_smaller_workspace_runs_the_fp32_kernel(gpu):
     assert torch.equal(call.out, want)
 
 
+@pytest.mark.parametrize("R,Cf,MB,NB", [(128, 128, 1, 40), (70, 100, 3, 60), (200, 1, 2, 1100), (64, 64, 5, 33)], ids=str)
+def test_fp32_split_leaves_unattended_blocks_out(R, Cf, MB, NB, gpu):
+    """Fewer query rows than keys: only key blocks that some row attends are
+    split (the exponents of the others stay as the scratch held them)."""
+    H, Hkv, D = 2, 1, 64
+    N = NB * Cf
+    g = torch.Generator().manual_seed(NB)
+    rows = [sorted({0 if r else NB - 1} | set(torch.randperm(NB, generator=g)[:3].tolist())) for r in range(MB)]
+    indptr = torch.tensor([0] + [len(r) for r in rows]).cumsum(0).int().to(gpu)
+    indices = torch.tensor(sum(rows, []), dtype=torch.int32, device=gpu)
+    w = lv.BlockSparseAttentionWrapper()
+    w.plan(indptr, indices, MB * R, N, R, Cf, H, Hkv, D, q_data_type=torch.float32)
+    q, k, v = (x.to(gpu) for x in _draw([(1, MB * R, H, D), (1, N, Hkv, D), (1, N, Hkv, D)], dtype=torch.float32))
+    plain = hip_ops.attn_fwd(q, k, v, w._plan, scratch=False)[0]
+    call = hip_ops.attn_args(q, k, v, w._plan)
+    n = C.c_int64()
+    capi.check("lvsa_attn_workspace_query", capi.lib().lvsa_attn_workspace_query(C.byref(call.args), C.byref(n)))
+    blocks = -(-N // 64)
+    ws = torch.full((n.value // 4,), 77, dtype=torch.int32, device=gpu)
+    call.args.workspace, call.args.workspace_bytes = ws.data_ptr(), n.value
+    capi.check("lvsa_attn_fwd", capi.lib().lvsa_attn_fwd(C.byref(call.args), hip_ops._stream(call.out.device)))
+    _close(call.out, plain, "split", max_abs=FP32_MAX_ABS, mean_abs=FP32_MEAN_ABS)
+    listed = {key // 64 for r in rows for b in r for key in range(b * Cf, (b + 1) * Cf)}
+    split = (ws[-2 * blocks:].reshape(blocks, 2) != 77).cpu()
+    assert [b for b in range(blocks) if split[b].any()] == sorted(listed) and len(listed) < blocks
+
+
 def test_fp32_without_memory_for_the_scratch(gpu):
     """Where memory for the fp16 pairs of K and V is short, an fp32 call runs
     without them (on the fp32 MFMAs) instead of failing."""
