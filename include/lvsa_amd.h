@@ -50,9 +50,11 @@ typedef enum lvsa_status {
   LVSA_ERR_HIP = -4            /* a HIP runtime call failed (launch error)        */
 } lvsa_status;
 
-/* LVSA_FP32: fp32 in and out, fp32 products and accumulation (the reference
- * computes in the caller's dtype, lvsa/sparse_attention.py:670, 689-704);
- * 128-row tiles, text tiles unsplit.                                        */
+/* LVSA_FP32: fp32 in and out with fp32 accumulation and softmax (the
+ * reference computes in the caller's dtype, lvsa/sparse_attention.py:670,
+ * 689-704); 128-row tiles.  With the scratch of lvsa_attn_workspace_query the
+ * products run on operands split into two fp16 numbers, where the numbers
+ * allow it; otherwise, and without it, on the fp32 matrix instructions.      */
 typedef enum lvsa_dtype { LVSA_BF16 = 0, LVSA_FP16 = 1, LVSA_FP32 = 2 } lvsa_dtype;
 
 /* ───────────────────────── frame mask builder ─────────────────────────── */
@@ -220,21 +222,27 @@ typedef struct lvsa_attn_args {
   int32_t rel_rows;
   /* optional scratch (device memory, lvsa_attn_workspace_query bytes, 16-byte
    * aligned; its contents on entry do not matter).  With it:
-   * - each text-query tile's key range is split into chunks that run as
-   *   separate work items after the video tiles and are merged by a second
-   *   launch (exact log-sum-exp merge, as flashinfer_runner.py:184-197), so
-   *   the long text tiles fill the launch's last round instead of
-   *   lengthening it;
+   * - text-query tiles longer than 128 key blocks, and shorter ones where an
+   *   estimate of the launch favours it, run as chunks of their key range
+   *   after the video tiles and are merged by a second launch (exact
+   *   log-sum-exp merge, as flashinfer_runner.py:184-197), so that they fill
+   *   the launch's last round instead of lengthening it;
    * - the single-stream kernel (every 16-bit head size) runs one persistent
-   *   work-group per CU (two for head size 64) that takes work items from
-   *   eight per-XCD queues (counters in the last 1 KiB, zeroed by the call)
-   *   and steals from the other XCDs' queues once its own is empty, so XCDs
-   *   that run faster take over items of slower ones;
-   * - at head size 64 (two work-groups per CU) each queue's last video
-   *   tiles run as two key-range halves each, merged by a third launch as
-   *   the text chunks are, when the scratch holds their partials (the size
-   *   lvsa_attn_workspace_query returns; a smaller scratch of at least the
-   *   text split and the counters runs the tiles whole).
+   *   work-group per CU (two with the maps of head sizes 64 and 128 that run
+   *   two) that takes work items from eight per-XCD queues (1 KiB of
+   *   counters, zeroed by the call) and steals from the other XCDs' queues
+   *   once its own is empty, so XCDs that run faster take over items of
+   *   slower ones;
+   * - the last video tiles of a launch run as 2 to 8 parts of their key
+   *   ranges, merged by a third launch as the text chunks are, where the
+   *   estimate favours it (every kernel, launches of fewer than five rounds;
+   *   at head size 64 every launch over the queues, in two parts);
+   * - fp32: K and V as pairs of fp16 numbers, written by a launch before the
+   *   attention, as many bytes as K and V.
+   * A smaller scratch is used as far as it goes: without the parts; then the
+   * least that is accepted, the chunks of long text tiles in 16 bit and the
+   * counters (1 KiB for fp32), with all other tiles whole and fp32 on the
+   * fp32 matrix instructions.
    * Null: one work-group per work item, text tiles whole and first.          */
   void* workspace;
   int64_t workspace_bytes;
@@ -246,11 +254,11 @@ typedef struct lvsa_attn_args {
  * encoder-query attention (lvsa/lvsa_processor.py:710-735) with one launch.   */
 LVSA_API int lvsa_attn_fwd(const lvsa_attn_args* a, hipStream_t stream);
 
-/* Bytes of scratch lvsa_attn_fwd uses for `a`: the text-tile split
- * partials (none without text queries), the video-tile split partials (head
- * size 64, when the call has enough tiles for the work queues; their number
- * follows the current device's compute units) and 1 KiB of work-queue
- * counters; host only, nothing is launched.
+/* Bytes of scratch lvsa_attn_fwd uses for `a`: the partials of the text chunks
+ * and of the video tiles in parts (at most 48 MiB but at head size 64; their
+ * number follows the current device's compute units), 1 KiB of work-queue
+ * counters and, for fp32, the fp16 pairs of K and V (as many bytes as both;
+ * none where they would pass 16 GiB); host only, nothing is launched.
  * Replaces the float workspace the FlashInfer wrapper is planned with
  * (flashinfer_runner.py:75-79, lvsa/lvsa_processor.py:798-804: 128 MB).      */
 LVSA_API int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes);
@@ -258,13 +266,13 @@ LVSA_API int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes);
 /* lvsa_attn_fwd without any allocation, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  It has no counterpart in the reference.  The
- * scratch (work-queue counters and the text-tile split) comes from a static
+ * scratch comes from a static
  * device array of LVSA_NOALLOC_SCRATCH_BYTES per GPU (a->workspace is
  * ignored), which each GPU the library runs on holds until the process
- * ends; a call whose text split and counters need more returns
- * LVSA_ERR_CAPACITY (the video split runs only when it fits as well).  All calls on one GPU share that array: calls
- * that overlap on one GPU (other streams, other threads) race, so serialise
- * them.  The caller still passes inputs and outputs; nothing else differs
+ * ends.  A call whose least scratch is more returns LVSA_ERR_CAPACITY; the
+ * rest (parts, short text tiles in chunks, fp32 pairs) is used when all of it
+ * fits.  All calls on one GPU share that array: calls that overlap on one GPU
+ * (other streams, other threads) race, so serialise them.  The caller still passes inputs and outputs; nothing else differs
  * from lvsa_attn_fwd.                                                         */
 #define LVSA_NOALLOC_SCRATCH_BYTES (64LL << 20)
 LVSA_API int lvsa_attn_fwd_noalloc(const lvsa_attn_args* a, hipStream_t stream);

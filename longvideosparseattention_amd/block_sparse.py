@@ -40,8 +40,9 @@ class BlockSparseAttentionWrapper:
     """HIP block-sparse attention over a block CSR (FlashInfer-compatible subset).
 
     ``float_workspace_buffer`` is accepted for signature compatibility; the
-    plan lives on the device, and the only scratch (for split text tiles) is
-    taken per call from torch's caching allocator.
+    plan lives on the device, and a call's scratch (queue counters, partials of
+    tiles in parts, for fp32 as many bytes as K and V) is taken per call from
+    torch's caching allocator.
     """
 
     def __init__(self, float_workspace_buffer: Optional[torch.Tensor] = None, backend: str = "auto"):

@@ -2,7 +2,8 @@
 // (lvsa_attn_kernels.h, lvsa_attn_stream.h), in a translation unit of their
 // own so that adding them leaves the compiler's code for the other head sizes
 // unchanged.  Tiles of 384 rows run the 12-wave single-stream kernel (three
-// waves per SIMD); tiles of 256 rows the 8-wave one or the ping-pong kernel.
+// waves per SIMD); tiles of 256 rows the dual map, the 8-wave one or the
+// ping-pong kernel; tiles of 128 rows the half map or the 4-wave kernel.
 #include "lvsa_attn_stream.h"
 
 namespace lvsa {

@@ -10,11 +10,13 @@
 // single-stream kernel does not take (frames too short for it) and the
 // LVSA_ATTN_KERNEL=pp comparison:
 //   attn_fwd_pp_kernel   256-row tiles, 8 waves x 32 rows in two groups that
-//                        alternate an MFMA phase with a softmax phase (D = 64,
-//                        96 and 128);
+//                        alternate an MFMA phase with a softmax phase (D = 96
+//                        on frames below 255 rows; D = 64, 96 and 128 on
+//                        sources that the single-stream loop cannot address
+//                        or whose tail crosses a frame);
 //   attn_fwd_kernel      128-row tiles, 4 waves x 32 rows, one barrier per
-//                        block (D = 192 and 256, whose Q and O need 320
-//                        registers; any head size with LVSA_ATTN_BLOCK_Q=128).
+//                        block (every head size but 96 on frames below 127
+//                        rows).
 // Both compute, per wave and key block:
 //   S^T = K · Q^T      v_mfma_f32_32x32x16_{bf16,f16}: A = K rows from LDS
 //                      (ds_read_b128), B = Q held in registers for the tile
@@ -77,16 +79,16 @@ struct AttnParams {
   // unnormalised partials to ws for attn_text_merge_kernel.
   int n_vwork, n_twork, text_chunks, text_first;
   float* ws;
-  // D = 128, 256-row tiles: run the single-stream kernel (its loop handles
-  // descriptors "none" and "two-part", which is all such a plan holds when
-  // query frames span at least 255 rows and key frames at least 64)
+  // Run the single-stream kernel (its loop handles descriptors "none" and
+  // "two-part", which is all a plan holds when query frames span at least a
+  // tile less one row and key frames at least 64)
   int use_stream;
   // D = 64, 256-row tiles on the single-stream kernel: the dual map (4 waves
   // of 64 rows, two work-groups per CU) rather than 8 waves of 32 rows
   int dual;
   // D = 64 and 128 on the single-stream kernel: the half map (2: with two key
-  // groups), tiles of 128 rows; with plan_shift 1 the plan's tiles have 256 and two tiles share one
-  // entry list
+  // groups), tiles of 128 rows; with plan_shift 1 the plan's tiles have 256
+  // and two tiles share one entry list
   int half, plan_shift;
   // Key-range split of each queue's last video tiles: the last min(vsplit,
   // videos of the queue) video items of queue x run as vparts (0: two) equal
@@ -97,8 +99,8 @@ struct AttnParams {
   int vsplit, vparts;
   float* vws;
   // Work queues (single-stream kernel with a workspace): `grid` persistent
-  // work-groups, one per CU (two with the dual map), take work items from 8 queues, one per XCD,
-  // whose counters (kQueueStride bytes apart, zeroed before the launch) are
+  // work-groups, one per CU (two with the dual and the half map), take work
+  // items from 8 queues, one per XCD, whose counters (kQueueStride bytes apart, zeroed before the launch) are
   // at `queues`; null: one work-group per item, mapped by map_work.
   uint32_t* queues;
   int grid;
@@ -272,8 +274,8 @@ struct WorkItem {
 // the K/V blocks they share stay in that XCD's L2), the last n_split of them
 // as vparts key ranges each, and the split text chunks t = x, x + 8, ... (the
 // shortest, last).  The parts and the chunks make the launch's last round
-// finer than whole tiles.  A work-group takes items from the queue of its own XCD and, once that is empty, from the next ones in turn:
-// XCDs that run faster take over the items of the slower ones at the end, so
+// finer than whole tiles.  A work-group takes items from the queue of its own
+// XCD and, once that is empty, from the next ones in turn: XCDs that run faster take over the items of the slower ones at the end, so
 // the launch does not wait for the slowest XCD's fixed share.
 struct QueueShape {
   int n_first, v0, n_video, n_split, n_last;   // n_split of the n_video video items run as `parts` parts

@@ -66,7 +66,7 @@ def attn_block_q(head_dim: int = 128, dtype: Optional[torch.dtype] = None, frame
     for 256: the single-stream kernel's wide map (4 waves, one
     per SIMD, when query frames span at least 127 rows and key frames at
     least 64) or else the 4-wave kernel; and 128 for fp32 inputs at every
-    head size (the fp32 kernel).
+    head size (the fp32 kernels).
 
     ``LVSA_ATTN_BLOCK_Q`` (128, 256 or 384) overrides the choice for 64 and
     128 in 16-bit, and 128 that for 192, for comparisons; so does
@@ -492,9 +492,11 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan,
     ``lse`` is the natural-log log-sum-exp ``[B, H, S]`` (fp32) when requested.
     ``scratch`` (the default) passes the call's device scratch: the counters of
     the work queues that balance the single-stream kernel's work-groups over
-    the XCDs, and the partials that let long text-query tiles run as key-range
-    chunks merged by log-sum-exp.  ``False`` launches one work-group per work
-    item and runs each text tile whole.
+    the XCDs, the partials that let text-query tiles and a launch's last video
+    tiles run as key ranges merged by log-sum-exp, and for fp32 K and V as
+    pairs of fp16 numbers (as many bytes as K and V).  ``False``, or memory too
+    short for it, launches one work-group per work item, runs every tile whole
+    and fp32 on the fp32 MFMAs.
     """
     call = attn_args(q, k, v, plan, kx=kx, vx=vx, qt=qt, scale=scale, return_lse=return_lse, out=out,
                      out_t=out_t)
@@ -512,7 +514,7 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: BlockPlan,
             capi.check("lvsa_attn_workspace_query", rc)
         if ws_bytes.value > 0:
             # work-queue counters (zeroed by the call), partials, fp32 pairs
-            # (as large as K and V); short of memory, the call runs without
+            # (as large as K and V)
             try:
                 ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=device)
                 a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes.value

@@ -631,7 +631,7 @@ _COMPUTE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 def _compute_dtype(t: torch.Tensor) -> torch.dtype:
     """The caller's dtype, as the reference computes (``lvsa/sparse_attention.py:670,
     689-704``): bf16 and fp16 on the 16-bit MFMA kernels, fp32 on the fp32
-    kernel; other types (fp64) run in fp32 and are cast back."""
+    kernels; other types (fp64) run in fp32 and are cast back."""
     return t.dtype if t.dtype in _COMPUTE_DTYPES else torch.float32
 
 
