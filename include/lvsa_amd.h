@@ -266,13 +266,13 @@ LVSA_API int lvsa_attn_workspace_query(const lvsa_attn_args* a, int64_t* bytes);
 /* lvsa_attn_fwd without any allocation, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  It has no counterpart in the reference.  The
- * scratch comes from a static
- * device array of LVSA_NOALLOC_SCRATCH_BYTES per GPU (a->workspace is
- * ignored), which each GPU the library runs on holds until the process
- * ends.  A call whose least scratch is more returns LVSA_ERR_CAPACITY; the
- * rest (parts, short text tiles in chunks, fp32 pairs) is used when all of it
- * fits.  All calls on one GPU share that array: calls that overlap on one GPU
- * (other streams, other threads) race, so serialise them.  The caller still passes inputs and outputs; nothing else differs
+ * scratch comes from a static device array of LVSA_NOALLOC_SCRATCH_BYTES per
+ * GPU (a->workspace is ignored), which each GPU the library runs on holds
+ * until the process ends.  A call whose least scratch is more returns
+ * LVSA_ERR_CAPACITY; the rest (parts, short text tiles in chunks, fp32 pairs)
+ * is used when all of it fits.  All calls on one GPU share that array: calls
+ * that overlap on one GPU (other streams, other threads) race, so serialise
+ * them.  The caller still passes inputs and outputs; nothing else differs
  * from lvsa_attn_fwd.                                                         */
 #define LVSA_NOALLOC_SCRATCH_BYTES (64LL << 20)
 LVSA_API int lvsa_attn_fwd_noalloc(const lvsa_attn_args* a, hipStream_t stream);

@@ -100,8 +100,9 @@ struct AttnParams {
   float* vws;
   // Work queues (single-stream kernel with a workspace): `grid` persistent
   // work-groups, one per CU (two with the dual and the half map), take work
-  // items from 8 queues, one per XCD, whose counters (kQueueStride bytes apart, zeroed before the launch) are
-  // at `queues`; null: one work-group per item, mapped by map_work.
+  // items from 8 queues, one per XCD, whose counters (kQueueStride bytes apart,
+  // zeroed before the launch) are at `queues`; null: one work-group per item,
+  // mapped by map_work.
   uint32_t* queues;
   int grid;
   // fp32 inputs: K and V split into fp16 pairs (lvsa_attn_f32.hip), split_slots
@@ -112,7 +113,7 @@ struct AttnParams {
   int split_slots, split_seen;
 };
 
-// Bytes of the work-queue counters at the end of the attention workspace.
+// Bytes of the work-queue counters in the attention workspace.
 constexpr int kQueueStride = 128;                  // one counter per 128-byte line
 constexpr int64_t kQueueBytes = 8 * kQueueStride;
 
@@ -275,8 +276,9 @@ struct WorkItem {
 // as vparts key ranges each, and the split text chunks t = x, x + 8, ... (the
 // shortest, last).  The parts and the chunks make the launch's last round
 // finer than whole tiles.  A work-group takes items from the queue of its own
-// XCD and, once that is empty, from the next ones in turn: XCDs that run faster take over the items of the slower ones at the end, so
-// the launch does not wait for the slowest XCD's fixed share.
+// XCD and, once that is empty, from the next ones in turn: XCDs that run faster
+// take over the items of the slower ones at the end, so the launch does not
+// wait for the slowest XCD's fixed share.
 struct QueueShape {
   int n_first, v0, n_video, n_split, n_last;   // n_split of the n_video video items run as `parts` parts
   int parts;
