@@ -39,7 +39,7 @@ from longvideosparseattention_amd import flops as lvflops  # noqa: E402
 
 MFMA_BF16_PEAK_TFLOPS = 2500.0
 # MI355X dense MFMA; an fp32 product runs as three fp16 ones
-MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "f16": 2500.0, "f32": 2500.0 / 3}
+MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "f16": 2500.0, "f32": 833.3}
 HBM_PEAK_GBS = 8000.0
 
 CONFIGS = {
@@ -283,7 +283,7 @@ def main(argv=None) -> int:
     per_call_tf = sorted(flops[offsets[i % len(offsets)]][0] / (call_ms[i] * 1e-3) / 1e12 for i in range(args.steps))
     achieved_median = per_call_tf[args.steps // 2] if args.steps % 2 else \
         0.5 * (per_call_tf[args.steps // 2 - 1] + per_call_tf[args.steps // 2])
-    bytes_per_call = 4 * (N + n_text) * H * D * 2
+    bytes_per_call = 4 * (N + n_text) * H * D * q.element_size()
     tag = args.config + ("" if args.window is None else f"_w{W}") + (
         "" if args.head_dim is None or args.head_dim == CONFIGS[args.config][3] else f"_d{D}")
     traffic, traffic_src, traffic_note = profiled_traffic(tag)
@@ -297,7 +297,7 @@ def main(argv=None) -> int:
         kernel = "attn_fwd_split_kernel"
 
     line = {
-        "metric": f"block-sparse attn ms/call + effective TFLOP/s (% {'a third of the fp16' if dname == 'f32' else 'bf16'} "
+        "metric": f"block-sparse attn ms/call + effective TFLOP/s (% {'split-fp16' if dname == 'f32' else 'bf16'} "
                   "MFMA peak), " + {"wan4x": "Wan 4x shape"}.get(args.config, args.config + " shape"),
         "value": round(value, 2),
         "unit": "TFLOP/s",
